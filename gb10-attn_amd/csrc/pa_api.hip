@@ -408,6 +408,55 @@ int hip_status(hipError_t e, const char* what) {
   return fail(PA_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
+// Prefill kernel parameters of checked arguments (cu, T: variable-length layout).
+PrefillParams prefill_params(const DecodeArgs& a, const int32_t* cu, int64_t T, double scale) {
+  PrefillParams pp;
+  memset(&pp, 0, sizeof(pp));
+  const DecodeParams& p = a.p;
+  pp.q = p.q; pp.out = p.out; pp.k = p.k; pp.v = p.v;
+  pp.block_tables = p.block_tables; pp.context_lens = p.context_lens;
+  pp.k_sb = p.k_sb; pp.k_st = p.k_st; pp.k_sh = p.k_sh;
+  pp.v_sb = p.v_sb; pp.v_st = p.v_st; pp.v_sh = p.v_sh;
+  pp.bt_stride = p.bt_stride; pp.num_blocks = p.num_blocks;
+  pp.B = p.B; pp.S = p.Sq; pp.H = p.H; pp.HKV = p.HKV; pp.G = p.G; pp.D = p.D; pp.BS = p.BS; pp.MB = p.MB;
+  pp.q_dtype = p.q_dtype; pp.out_dtype = p.out_dtype;
+  // FP8 K tiles take q's type when q is fp16 or bf16 (the codes convert exactly to both).
+  pp.q_split = a.kv_dtype == kFP8 ? p.q_dtype == kF32 : p.q_dtype != a.kv_dtype;
+  pp.bs_div = p.bs_div;
+  pp.cu_q = cu;
+  pp.q_total = T;
+  pp.vscale = 1.0f;
+  // The kernel applies the sign of the scale to q (exactly) and keeps the
+  // softmax scale positive, so the running max of raw scores orders as the scaled ones.
+  const double log2e = 1.4426950408889634;
+  pp.q_and = 0xffffffffu;
+  pp.q_xor = 0u;
+  pp.q_sign = 1.0f;
+  pp.qscale = (float)(scale * log2e);
+  if (scale < 0) {
+    pp.q_xor = 0x80008000u;
+    pp.q_sign = -1.0f;
+    pp.qscale = (float)(-scale * log2e);
+  } else if (scale == 0) {
+    pp.q_and = 0u;
+    pp.q_sign = 0.0f;
+    pp.qscale = 1.0f;
+  }
+  return pp;
+}
+
+// The matrix-core kernel serves paged_attention_prefill over 16-bit and FP8
+// caches for chunks of at least kPrefill32Rows rows; fp32 and fp64 caches,
+// shorter chunks and a q that is not 16-byte aligned run as a decode problem
+// per query row.  Contexts 64-4096, matrix kernel against decode kernel: at 64
+// rows 14.3 vs 15.0 us (one sequence of 12 heads, context 512), 15.2 vs 75.9
+// (eight sequences); at 16 rows 13.4 vs 11.1 and 14.4 vs 24.9.
+constexpr int kPrefill32Rows = 64;
+bool prefill32_eligible(const DecodeArgs& a, const pa_tensor_t* q) {
+  return (a.kv_dtype == kF16 || a.kv_dtype == kBF16 || a.kv_dtype == kFP8) && a.p.Sq >= kPrefill32Rows &&
+         (reinterpret_cast<uintptr_t>(q->data) & 15) == 0;
+}
+
 // One direct decode launch (one partition per sequence): v1, v2 and the
 // fp32 prefill path.
 int run_direct(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const pa_tensor_t* v,
@@ -418,6 +467,10 @@ int run_direct(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, con
   int rc = check_args(out, q, k, v, bt, ctx, scale, prefill, &a);
   if (rc) return rc;
   if ((int64_t)a.p.B * a.p.Sq * a.p.H == 0) return PA_OK;
+  if (prefill && prefill32_eligible(a, q))
+    return hip_status(launch_prefill32(prefill_params(a, nullptr, 0, scale), a.kv_dtype,
+                                       static_cast<hipStream_t>(stream)),
+                      "prefill kernel launch");
   a.p.parts = 1;
   a.p.part_tokens = 0;
   a.p.direct = 1;
@@ -537,39 +590,9 @@ int run_prefill_mfma(DecodeArgs& a, const pa_tensor_t* q, const int32_t* cu, int
   if ((int64_t)a.p.B * a.p.Sq * a.p.H == 0) return PA_OK;
   if ((reinterpret_cast<uintptr_t>(q->data) & 15) != 0)
     return fail(PA_ERR_UNSUPPORTED, "the MFMA path needs a 16-byte aligned q");
-  PrefillParams pp;
-  memset(&pp, 0, sizeof(pp));
-  const DecodeParams& p = a.p;
-  pp.q = p.q; pp.out = p.out; pp.k = p.k; pp.v = p.v;
-  pp.block_tables = p.block_tables; pp.context_lens = p.context_lens;
-  pp.k_sb = p.k_sb; pp.k_st = p.k_st; pp.k_sh = p.k_sh;
-  pp.v_sb = p.v_sb; pp.v_st = p.v_st; pp.v_sh = p.v_sh;
-  pp.bt_stride = p.bt_stride; pp.num_blocks = p.num_blocks;
-  pp.B = p.B; pp.S = p.Sq; pp.H = p.H; pp.HKV = p.HKV; pp.G = p.G; pp.D = p.D; pp.BS = p.BS; pp.MB = p.MB;
-  pp.q_dtype = p.q_dtype; pp.out_dtype = p.out_dtype;
-  // FP8 K tiles take q's type when q is fp16 or bf16 (the codes convert exactly to both).
-  pp.q_split = a.kv_dtype == kFP8 ? p.q_dtype == kF32 : p.q_dtype != a.kv_dtype;
-  pp.bs_div = p.bs_div;
-  pp.cu_q = cu;
-  pp.q_total = T;
+  PrefillParams pp = prefill_params(a, cu, T, scale);
   pp.skip_single = route_single ? 1 : 0;
   pp.vscale = (float)v_scale;
-  // The kernel applies the sign of the scale to q (exactly) and keeps the
-  // softmax scale positive, so the running max of raw scores orders as the scaled ones.
-  const double log2e = 1.4426950408889634;
-  pp.q_and = 0xffffffffu;
-  pp.q_xor = 0u;
-  pp.q_sign = 1.0f;
-  pp.qscale = (float)(scale * log2e);
-  if (scale < 0) {
-    pp.q_xor = 0x80008000u;
-    pp.q_sign = -1.0f;
-    pp.qscale = (float)(-scale * log2e);
-  } else if (scale == 0) {
-    pp.q_and = 0u;
-    pp.q_sign = 0.0f;
-    pp.qscale = 1.0f;
-  }
   return hip_status(launch_prefill_mfma(pp, a.kv_dtype, static_cast<hipStream_t>(stream)),
                     "prefill kernel launch");
 }

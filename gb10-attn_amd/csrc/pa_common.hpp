@@ -184,6 +184,7 @@ hipError_t launch_decode(const DecodeParams& p, int kv_dtype, int gc, hipStream_
 extern thread_local int t_decode_fused;
 hipError_t launch_reduce(const ReduceParams& p, hipStream_t stream);
 hipError_t launch_prefill_mfma(const PrefillParams& p, int kv_dtype, hipStream_t stream);
+hipError_t launch_prefill32(const PrefillParams& p, int kv_dtype, hipStream_t stream);
 hipError_t launch_write_kv(const WriteParams& p, hipStream_t stream);
 
 // Head packing (heads contiguous in the pool; MHA, or GQA groups of four over

@@ -1,0 +1,61 @@
+// pa_prefill32.hip -- launches of the fp32-precision matrix-core prefill
+// (prefill32_kernel of pa_prefill.hpp): paged_attention_prefill over 16-bit
+// and FP8 caches.
+#include "pa_prefill.hpp"
+
+namespace pa {
+
+template <typename KV, int D, int kQP, bool kSplit>
+static hipError_t launch_p32_q(const PrefillParams& p, hipStream_t stream) {
+  static std::atomic<int64_t> cache[64];
+  const auto kernel = prefill32_kernel<KV, D, kQP, kSplit>;
+  PrefillParams q = p;
+  constexpr int QB = kSplit ? 2 * PfShape<D>::QW : PfShape<D>::QB;
+  q.q_tiles = (p.S + QB - 1) / QB;
+  const int64_t units = (int64_t)q.B * q.H * q.q_tiles;
+  int64_t cus = 0, per_cu = 0;
+  residency(kernel, cache, &cus, &per_cu);
+  q.wg_cus = units > cus && units <= cus * per_cu ? (int32_t)cus : 0;  // one resident wave
+  note_launch("pa::prefill32_kernel<%s, %d, %d, %s>", KV::kName, D, kQP, kSplit ? "true" : "false");
+  hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(kPfThreads), 0, stream, q);
+  return hipGetLastError();
+}
+
+template <typename KV, int D, int kQP>
+static hipError_t launch_p32(const PrefillParams& p, hipStream_t stream) {
+  if constexpr (PfShape<D>::MT == 2) {
+    // Key-split mode (64 query rows per work-group) for grids of few
+    // work-groups, and for up to 64 rows (half of the plain mode's waves would
+    // have none).
+    static std::atomic<int64_t> cache[64];
+    int64_t cus = 0, per_cu = 0;
+    residency(prefill32_kernel<KV, D, kQP, false>, cache, &cus, &per_cu);
+    const int64_t plain = (int64_t)p.B * p.H * ((p.S + PfShape<D>::QB - 1) / PfShape<D>::QB);
+    if (p.S <= 64 || (cus > 0 && plain < cus)) return launch_p32_q<KV, D, kQP, true>(p, stream);
+  }
+  return launch_p32_q<KV, D, kQP, false>(p, stream);
+}
+
+template <typename KV, int kQP>
+static hipError_t launch_p32_kv(const PrefillParams& p, hipStream_t stream) {
+  switch (p.D) {
+    case 32: return launch_p32<KV, 32, kQP>(p, stream);
+    case 64: return launch_p32<KV, 64, kQP>(p, stream);
+    case 128: return launch_p32<KV, 128, kQP>(p, stream);
+    case 256: return launch_p32<KV, 256, kQP>(p, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// q in the cache's 16-bit type is one exact piece; else two fp16 pieces (fp16
+// and FP8 caches) or three bf16 ones.
+hipError_t launch_prefill32(const PrefillParams& p, int kv_dtype, hipStream_t stream) {
+  if (kv_dtype == kF16)
+    return p.q_dtype == kF16 ? launch_p32_kv<KvF16, 1>(p, stream) : launch_p32_kv<KvF16, 2>(p, stream);
+  if (kv_dtype == kBF16)
+    return p.q_dtype == kBF16 ? launch_p32_kv<KvBF16, 1>(p, stream) : launch_p32_kv<KvBF16, 3>(p, stream);
+  if (kv_dtype == kFP8) return launch_p32_kv<KvFP8, 2>(p, stream);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace pa

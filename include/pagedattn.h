@@ -172,7 +172,8 @@ int pa_plan_partitions(int64_t num_seqs, int64_t num_heads, int64_t num_kv_heads
                        int64_t head_dim, int64_t max_context, int64_t num_compute_units,
                        int64_t* partition_tokens, int64_t* num_partitions);
 
-/* Causal (chunked) prefill, fp32 arithmetic.  Replaces paged_attention_prefill(),
+/* Causal (chunked) prefill at fp32 precision (over 16-bit and FP8 caches on
+ * the matrix cores, fp32 operands carried as sums of 16-bit pieces).  Replaces paged_attention_prefill(),
  * kernels/paged_attn_prefill.h:13-15 (kernels/paged_attn_prefill.cu:122-175).
  * Query s of sequence b sits at q_pos = ctx_b - S + s and attends keys
  * [0, q_pos]; q_pos < 0 gives a zero row (kernels/paged_attn_prefill.cu:62-74). */

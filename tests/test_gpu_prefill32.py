@@ -1,0 +1,141 @@
+"""GPU parity of paged_attention_prefill's matrix-core kernel (16-bit and FP8
+caches; fp32 precision through 16-bit pieces) against attention in 64 bits on
+the same values, each row over its own keys only.
+
+Tolerance: fp32 arithmetic.  A score s carries an absolute rounding of about
+|s| 2^-24, which is the relative error of its weight, and the other steps a
+few roundings of 2^-24; with |s| up to 8 (N(0, 1) data and the scales used
+here) the 2-norm of an output's error stays below 16 * 2^-24 (1e-6) of the
+result's.  FP8 caches hold N(0, 1) itself: times 8 the scores reach 80 and
+that bound 5e-6 (1.1e-6 was measured).
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from _helpers import to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+F8 = torch.float8_e4m3fn
+
+
+def case(B, S, H, HKV, D, BS, ctx, kv, qt, seed):
+    inp = oracle.paged_inputs(B, 1, HKV, D, BS, ctx, seed=seed, kv_dtype="f32" if kv == "fp8" else kv, extra_blocks=2)
+    q = oracle.quantize(np.random.default_rng(seed).standard_normal((B, S, H, D), dtype=np.float32), qt)
+    if kv == "fp8":
+        k, v = (torch.from_numpy(inp[n]).to(F8) for n in "kv")
+        k32, v32 = k.float(), v.float()
+    else:
+        k, v = to_dev(inp["k"], kv, "cpu"), to_dev(inp["v"], kv, "cpu")
+        k32, v32 = k.float(), v.float()
+    return to_dev(q, qt, "cpu"), k, v, inp["bt"], np.asarray(ctx, np.int32), k32, v32
+
+
+def attention64(q, k32, v32, bt, ctx, scale):
+    """Every row's attention over its own keys in 64 bits; rows before the context are zeros."""
+    B, S, H, D = q.shape
+    BS, HKV = k32.shape[1], k32.shape[2]
+    out = torch.zeros(q.shape, dtype=torch.float64)
+    for b in range(B):
+        n = int(ctx[b])
+        pg = torch.from_numpy(bt[b, :-(-n // BS)].astype(np.int64))
+        k = k32[pg].reshape(-1, HKV, D)[:n].double()
+        v = v32[pg].reshape(-1, HKV, D)[:n].double()
+        for s in range(S):
+            t = n - S + s + 1
+            if t <= 0:
+                continue
+            for h in range(H):
+                g = h // (H // HKV)
+                w = torch.softmax((k[:t, g] @ q[b, s, h].double()) * scale, 0)
+                out[b, s, h] = w @ v[:t, g]
+    return out
+
+
+def run(pa, dev, q, k, v, bt, ctx, scale, **kw):
+    return to_host(pa.paged_attention_prefill(q.to(dev), k.to(dev), v.to(dev), torch.from_numpy(bt).to(dev),
+                                              torch.from_numpy(ctx).to(dev), scale, **kw))
+
+
+def close64(got, want):
+    got, want = torch.from_numpy(got).double(), want
+    fine = torch.isfinite(want)
+    assert torch.equal(fine, torch.isfinite(got))
+    assert torch.equal(torch.isnan(want), torch.isnan(got))
+    assert torch.equal(want[~fine & ~torch.isnan(want)], got[~fine & ~torch.isnan(want)])
+    err = float((got - want)[fine].norm() / want[fine].norm())
+    assert err < 1e-6, err
+
+
+@pytest.mark.parametrize("kv,qt", [("f16", "f32"), ("f16", "f16"), ("bf16", "f32"), ("bf16", "bf16"),
+                                   ("fp8", "f32"), ("fp8", "bf16")])
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+def test_prefill32(pa, dev, kv, qt, D):
+    """Edges of the 32/64/128-row blocks and 32/64-key tiles; chunked, padded
+    and empty sequences; both grid modes; page sizes that do not divide a tile."""
+    for i, (B, S, H, HKV, BS, ctx, scale) in enumerate([
+            (3, 64, 4, 2, 16, [64, 160, 20], 1 / np.sqrt(D)), (2, 65, 2, 1, 5, [129, 64], -0.2),
+            (1, 129, 2, 2, 32, [129], 0.3), (2, 97, 2, 1, 16, [127, 0], 0.0)]):
+        print(f"prefill32 {kv} {qt} D={D} case {i}", flush=True)
+        q, k, v, bt, c, k32, v32 = case(B, S, H, HKV, D, BS, ctx, kv, qt, D + i)
+        got = run(pa, dev, q, k, v, bt, c, scale)
+        assert "prefill32_kernel" in pa.last_launch(), pa.last_launch()
+        close64(got, attention64(q, k32, v32, bt, c, scale))
+
+
+@pytest.mark.parametrize("kv", ["f16", "bf16"])
+def test_prefill32_plain_mode(pa, dev, kv):
+    """A grid of at least a work-group per CU (128 rows per work-group)."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    H = -(-cus // 4)
+    q, k, v, bt, c, k32, v32 = case(2, 130, H, 1, 64, 16, [130, 200], kv, "f32", 5)
+    print("plain mode", kv, flush=True)
+    got = run(pa, dev, q, k, v, bt, c, 0.125)
+    assert pa.last_launch().endswith("false>"), pa.last_launch()
+    close64(got[:, :, :2], attention64(q[:, :, :2].contiguous(), k32, v32, bt, c, 0.125))
+
+
+def test_prefill32_q_range(pa, dev):
+    """Rows of very large and very small q (the fp16 pieces are scaled by row)
+    and rows that mix both; output types."""
+    q, k, v, bt, c, k32, v32 = case(1, 72, 2, 2, 64, 16, [100], "f16", "f32", 9)
+    q[0, :10] *= 1e-30
+    q[0, 10:20] *= 300.0
+    q[0, 20:30, :, ::2] *= 1e-5
+    q[0, 30] = 0.0
+    print("q range", flush=True)
+    want = attention64(q, k32, v32, bt, c, 0.01)
+    close64(run(pa, dev, q, k, v, bt, c, 0.01), want)
+    for ot, tol in ((torch.float16, 2 ** -11), (torch.bfloat16, 2 ** -8)):
+        got = run(pa, dev, q, k, v, bt, c, 0.01, out_dtype=ot)
+        assert float((torch.from_numpy(got).double() - want).norm() / want.norm()) < tol
+
+
+@pytest.mark.parametrize("kv", ["f16", "bf16", "fp8"])
+def test_prefill32_non_finite(pa, dev, kv):
+    """Inf and NaN reach exactly the rows that attend them (a masked key's V is
+    not multiplied into earlier rows), with the value a chain of fp32 products
+    gives; an invalid block id poisons the rows that read its page."""
+    B, S, H, D, BS, ctx = 1, 100, 2, 64, 16, [150]
+    q, k, v, bt, c, k32, v32 = case(B, S, H, H, D, BS, ctx, kv, "f32", 21)
+
+    def put(x, x32, key, head, dim, val):
+        page, row = int(bt[0, key // BS]), key % BS
+        if kv == "fp8":
+            x.view(torch.uint8)[page, row, head, dim] = 0x7f  # NaN
+            x32[page, row, head, dim] = float("nan")
+        else:
+            x[page, row, head, dim] = val
+            x32[page, row, head, dim] = val
+
+    put(v, v32, 120, 0, 3, float("inf"))
+    put(v, v32, 97, 1, 7, float("nan"))
+    put(k, k32, 140, 1, 9, float("-inf"))
+    print("non-finite", kv, flush=True)
+    close64(run(pa, dev, q, k, v, bt, c, 0.125), attention64(q, k32, v32, bt, c, 0.125))
+    bad = bt.copy()
+    bad[0, 5] = 10 ** 6  # keys 80..95: rows whose own keys include one of them
+    got = run(pa, dev, q, k, v, bad, c, 0.125)
+    assert np.isnan(got[0, 30:]).all() and np.isfinite(got[0, :30, :]).all()
