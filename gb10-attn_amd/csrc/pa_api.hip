@@ -420,6 +420,10 @@ PrefillParams prefill_params(const DecodeArgs& a, const int32_t* cu, int64_t T, 
   pp.bt_stride = p.bt_stride; pp.num_blocks = p.num_blocks;
   pp.B = p.B; pp.S = p.Sq; pp.H = p.H; pp.HKV = p.HKV; pp.G = p.G; pp.D = p.D; pp.BS = p.BS; pp.MB = p.MB;
   pp.q_dtype = p.q_dtype; pp.out_dtype = p.out_dtype;
+  // The heads of a group packed into the rows while the packed row count fits 32 bits.
+  pp.gp = (int64_t)p.Sq * p.G <= INT32_MAX - 512 ? p.G : 1;
+  pp.HG = p.H / pp.gp;
+  pp.gp_div = make_fastdiv((uint32_t)pp.gp);
   // FP8 K tiles take q's type when q is fp16 or bf16 (the codes convert exactly to both).
   pp.q_split = a.kv_dtype == kFP8 ? p.q_dtype == kF32 : p.q_dtype != a.kv_dtype;
   pp.bs_div = p.bs_div;
@@ -809,6 +813,7 @@ int paged_attention_prefill_varlen_scaled(pa_tensor_t* out, const pa_tensor_t* q
   rc = check_args(&o4, &q4, k_cache, v_cache, block_tables, context_lens, scale * k_scale, true, &a);
   if (rc) return rc;
   if (max_q_len == 0 || T == 0) return PA_OK;
+  a.p.Sq = (int)std::min<int64_t>(mq, T);  // no sequence has more than T rows
   g_launches.clear();
   const int32_t* cu = static_cast<const int32_t*>(cu_seqlens_q->data);
   // Sequences that bring one query row (decode steps of the batch) go to the

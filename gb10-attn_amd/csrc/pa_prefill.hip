@@ -10,8 +10,8 @@ static hipError_t launch_pf_q(const PrefillParams& p, hipStream_t stream) {
   const auto kernel = prefill_mfma_kernel<KV, D, kSplitQ, kSplit>;
   PrefillParams q = p;
   constexpr int QB = kSplit ? 2 * PfShape<D>::QW : PfShape<D>::QB;
-  q.q_tiles = (p.S + QB - 1) / QB;
-  int64_t units = (int64_t)q.B * q.H * q.q_tiles;
+  q.q_tiles = (int32_t)(((int64_t)p.S * p.gp + QB - 1) / QB);
+  int64_t units = (int64_t)q.B * q.HG * q.q_tiles;
   int64_t cus = 0, per_cu = 0;
   residency(kernel, cache, &cus, &per_cu);
   q.wg_cus = units > cus && units <= cus * per_cu ? (int32_t)cus : 0;  // one resident wave
@@ -20,8 +20,8 @@ static hipError_t launch_pf_q(const PrefillParams& p, hipStream_t stream) {
   // T / QB + sequences).
   q.vl_compact = 0;
   if (p.cu_q && p.B <= kVlMaxSeqs) {
-    const int64_t ub = (p.q_total + QB - 1) / QB + std::min<int64_t>(p.B, p.q_total);
-    units = (int64_t)q.H * std::min<int64_t>((int64_t)q.B * q.q_tiles, ub);
+    const int64_t ub = (p.q_total * p.gp + QB - 1) / QB + std::min<int64_t>(p.B, p.q_total);
+    units = (int64_t)q.HG * std::min<int64_t>((int64_t)q.B * q.q_tiles, ub);
     q.vl_compact = 1;
     q.wg_cus = 0;
   }
@@ -36,8 +36,8 @@ static hipError_t launch_pp(const PrefillParams& p, hipStream_t stream) {
   static std::atomic<int64_t> cache[64];
   const auto kernel = prefill_pp_kernel<KV, D>;
   PrefillParams q = p;
-  q.q_tiles = (p.S + kPpRows - 1) / kPpRows;
-  const int64_t units = (int64_t)q.B * q.H * q.q_tiles;
+  q.q_tiles = (int32_t)(((int64_t)p.S * p.gp + kPpRows - 1) / kPpRows);
+  const int64_t units = (int64_t)q.B * q.HG * q.q_tiles;
   int64_t cus = 0, per_cu = 0;
   residency(kernel, cache, &cus, &per_cu, kPpThreads);
   q.wg_cus = units > cus && units <= cus * per_cu ? (int32_t)cus : 0;  // one resident wave

@@ -11,8 +11,8 @@ static hipError_t launch_p32_q(const PrefillParams& p, hipStream_t stream) {
   const auto kernel = prefill32_kernel<KV, D, kQP, kSplit>;
   PrefillParams q = p;
   constexpr int QB = kSplit ? 2 * PfShape<D>::QW : PfShape<D>::QB;
-  q.q_tiles = (p.S + QB - 1) / QB;
-  const int64_t units = (int64_t)q.B * q.H * q.q_tiles;
+  q.q_tiles = (int32_t)(((int64_t)p.S * p.gp + QB - 1) / QB);
+  const int64_t units = (int64_t)q.B * q.HG * q.q_tiles;
   int64_t cus = 0, per_cu = 0;
   residency(kernel, cache, &cus, &per_cu);
   q.wg_cus = units > cus && units <= cus * per_cu ? (int32_t)cus : 0;  // one resident wave
