@@ -28,6 +28,7 @@ EXPORTS = (
     "choose_num_splits", "choose_num_splits_for", "pa_plan_partitions",
     "paged_attention_prefill", "paged_attention_prefill_wmma", "paged_attention_prefill_wmma_scaled",
     "paged_attention_prefill_varlen", "paged_attention_prefill_varlen_scaled",
+    "paged_attention_prefill_split", "paged_attention_prefill_workspace_size",
     "pa_write_kv", "pa_write_kv_scaled",
 )
 
@@ -104,6 +105,10 @@ def lib() -> C.CDLL:
     L.paged_attention_prefill_varlen.argtypes = six + [T, i64, C.c_double, P]
     L.paged_attention_prefill_varlen_scaled.restype = C.c_int
     L.paged_attention_prefill_varlen_scaled.argtypes = six + [T, i64, C.c_double, C.c_double, C.c_double, P]
+    L.paged_attention_prefill_split.restype = C.c_int
+    L.paged_attention_prefill_split.argtypes = six + [T, i64, C.c_double, C.c_double, C.c_double, C.c_int, P, sz, P]
+    L.paged_attention_prefill_workspace_size.restype = sz
+    L.paged_attention_prefill_workspace_size.argtypes = [T, T, T, i64]
     L.pa_write_kv.restype = C.c_int
     L.pa_write_kv.argtypes = [T, T, T, T, T, P]
     L.pa_write_kv_scaled.restype = C.c_int

@@ -387,6 +387,26 @@ int make_plan(const DecodeParams& p, int gc, int kv_bytes, int64_t num_splits, P
   return PA_OK;
 }
 
+// The decode rows' plan of a variable-length batch of B sequences:
+// paged_attention_v3's, where its split gains eight times what pays there (the
+// grid also holds the work-groups of sequences that bring more rows, and the
+// merge is one more launch among four).  32/8 heads of 128, bf16: one decode
+// row and one 64-row chunk at context 8000 292 -> 55 us (decode and prefill
+// split), eight rows and three chunks of ragged contexts to 4000 98 -> 68;
+// sixteen rows and two 512-row chunks at 2048, below the bound, 102 -> 106.
+int plan_varlen_decode(const DecodeParams& p, int gc, int kv_bytes, Plan* plan) {
+  int cus = 0, rc;
+  if ((rc = make_plan(p, gc, kv_bytes, 0, plan)) || plan->direct) return rc;
+  if ((rc = device_cu_count(&cus))) return rc;
+  const double rows = (double)p.MB * p.BS * p.D / 64.0, units = (double)p.B * p.HKV * ((p.G + gc - 1) / gc);
+  if (rows * rows * cus < 8.0 * (double)knobs().split_pay * units) {
+    plan->parts = 1;
+    plan->part_tokens = 0;
+    plan->direct = true;
+  }
+  return PA_OK;
+}
+
 size_t workspace_bytes_for(int64_t B, int64_t H, int64_t D, const Plan& plan) {
   if (plan.direct) return 0;
   const size_t rows = (size_t)B * H * plan.parts;
@@ -408,6 +428,39 @@ int hip_status(hipError_t e, const char* what) {
   return fail(PA_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
+// The heads of a group packed into the rows while the packed row count fits 32 bits.
+void pack_heads(PrefillParams& pp) {
+  pp.gp = (int64_t)pp.S * pp.G <= INT32_MAX - 512 ? pp.G : 1;
+  pp.HG = pp.H / pp.gp;
+  pp.gp_div = make_fastdiv((uint32_t)pp.gp);
+}
+
+bool prefill_kv(int kv_dtype) { return kv_dtype == kF16 || kv_dtype == kBF16 || kv_dtype == kFP8; }
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// Caller's workspace of a prefill call (none: the call runs unsplit).
+struct PrefillWorkspace {
+  void* ptr = nullptr;
+  size_t bytes = 0;
+  bool given = false;
+};
+
+// Plans the context split of a call with a workspace and binds it (after
+// `before` bytes of it that the call's decode rows take).
+int bind_split(PrefillParams& pp, bool varlen, const PrefillWorkspace& ws, size_t before = 0) {
+  if (!ws.given) return PA_OK;
+  int cus = 0, rc;
+  if ((rc = device_cu_count(&cus))) return rc;
+  const size_t bytes = plan_prefill_split(pp, varlen, cus), need = bytes + before;
+  if (need > 0 && (!ws.ptr || ws.bytes < need))
+    return fail(PA_ERR_WORKSPACE, "workspace too small: need %zu bytes, got %zu", need, ws.ptr ? ws.bytes : 0);
+  if (need > 0 && (reinterpret_cast<uintptr_t>(ws.ptr) & 255) != 0)
+    return fail(PA_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+  if (bytes > 0) bind_prefill_split(pp, static_cast<char*>(ws.ptr) + before, bytes);
+  return PA_OK;
+}
+
 // Prefill kernel parameters of checked arguments (cu, T: variable-length layout).
 PrefillParams prefill_params(const DecodeArgs& a, const int32_t* cu, int64_t T, double scale) {
   PrefillParams pp;
@@ -420,10 +473,7 @@ PrefillParams prefill_params(const DecodeArgs& a, const int32_t* cu, int64_t T, 
   pp.bt_stride = p.bt_stride; pp.num_blocks = p.num_blocks;
   pp.B = p.B; pp.S = p.Sq; pp.H = p.H; pp.HKV = p.HKV; pp.G = p.G; pp.D = p.D; pp.BS = p.BS; pp.MB = p.MB;
   pp.q_dtype = p.q_dtype; pp.out_dtype = p.out_dtype;
-  // The heads of a group packed into the rows while the packed row count fits 32 bits.
-  pp.gp = (int64_t)p.Sq * p.G <= INT32_MAX - 512 ? p.G : 1;
-  pp.HG = p.H / pp.gp;
-  pp.gp_div = make_fastdiv((uint32_t)pp.gp);
+  pack_heads(pp);
   // FP8 K tiles take q's type when q is fp16 or bf16 (the codes convert exactly to both).
   pp.q_split = a.kv_dtype == kFP8 ? p.q_dtype == kF32 : p.q_dtype != a.kv_dtype;
   pp.bs_div = p.bs_div;
@@ -457,24 +507,24 @@ PrefillParams prefill_params(const DecodeArgs& a, const int32_t* cu, int64_t T, 
 // (eight sequences); at 16 rows 13.4 vs 11.1 and 14.4 vs 24.9.
 constexpr int kPrefill32Rows = 64;
 bool prefill32_eligible(const DecodeArgs& a, const pa_tensor_t* q) {
-  return (a.kv_dtype == kF16 || a.kv_dtype == kBF16 || a.kv_dtype == kFP8) && a.p.Sq >= kPrefill32Rows &&
-         (reinterpret_cast<uintptr_t>(q->data) & 15) == 0;
+  return prefill_kv(a.kv_dtype) && a.p.Sq >= kPrefill32Rows && aligned16(q->data);
 }
 
 // One direct decode launch (one partition per sequence): v1, v2 and the
 // fp32 prefill path.
 int run_direct(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const pa_tensor_t* v,
                const pa_tensor_t* bt, const pa_tensor_t* ctx, double scale, bool prefill,
-               void* stream) {
+               void* stream, const PrefillWorkspace& ws = {}) {
   g_launches.clear();
   DecodeArgs a;
   int rc = check_args(out, q, k, v, bt, ctx, scale, prefill, &a);
   if (rc) return rc;
   if ((int64_t)a.p.B * a.p.Sq * a.p.H == 0) return PA_OK;
-  if (prefill && prefill32_eligible(a, q))
-    return hip_status(launch_prefill32(prefill_params(a, nullptr, 0, scale), a.kv_dtype,
-                                       static_cast<hipStream_t>(stream)),
-                      "prefill kernel launch");
+  if (prefill && prefill32_eligible(a, q)) {
+    PrefillParams pp = prefill_params(a, nullptr, 0, scale);
+    if ((rc = bind_split(pp, false, ws))) return rc;
+    return hip_status(launch_prefill32(pp, a.kv_dtype, static_cast<hipStream_t>(stream)), "prefill kernel launch");
+  }
   a.p.parts = 1;
   a.p.part_tokens = 0;
   a.p.direct = 1;
@@ -483,6 +533,23 @@ int run_direct(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, con
   a.p.hp = pack_for(a.p, dtype_bytes(a.kv_dtype), 1, cus);
   return hip_status(launch_decode(a.p, a.kv_dtype, a.gc, static_cast<hipStream_t>(stream)),
                     "decode kernel launch");
+}
+
+// The reduce launch of a planned and bound split.
+ReduceParams reduce_params(const DecodeParams& p) {
+  ReduceParams r;
+  r.out = p.out;
+  r.ws_acc = p.ws_acc;
+  r.ws_m = p.ws_m;
+  r.ws_l = p.ws_l;
+  r.context_lens = p.context_lens;
+  r.B = p.B; r.H = p.H; r.D = p.D; r.MB = p.MB; r.BS = p.BS;
+  r.out_dtype = p.out_dtype;
+  r.parts = p.parts;
+  r.part_tokens = p.part_tokens;
+  r.cu_q = p.cu_q;
+  r.q_total = p.q_total;
+  return r;
 }
 
 enum V3Phase { kBoth = 3, kPartition = 1, kReduce = 2 };
@@ -566,16 +633,7 @@ int run_v3(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const p
     if ((rc = hip_status(launch_decode(a.p, a.kv_dtype, a.gc, s), "partition kernel launch"))) return rc;
   }
   if ((phases & kReduce) && !plan.direct && !t_decode_fused) {
-    ReduceParams r;
-    r.out = a.p.out;
-    r.ws_acc = a.p.ws_acc;
-    r.ws_m = a.p.ws_m;
-    r.ws_l = a.p.ws_l;
-    r.context_lens = a.p.context_lens;
-    r.B = a.p.B; r.H = a.p.H; r.D = a.p.D; r.MB = a.p.MB; r.BS = a.p.BS;
-    r.out_dtype = a.p.out_dtype;
-    r.parts = a.p.parts;
-    r.part_tokens = a.p.part_tokens;
+    const ReduceParams r = reduce_params(a.p);
     if ((rc = hip_status(launch_reduce(r, s), "reduce kernel launch"))) return rc;
   }
   return PA_OK;
@@ -584,21 +642,119 @@ int run_v3(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const p
 // MFMA prefill launch for checked arguments; cu != null selects the
 // variable-length layout (rows cu[b] .. cu[b+1] of a packed [T, H, D] q/out).
 int run_prefill_mfma(DecodeArgs& a, const pa_tensor_t* q, const int32_t* cu, int64_t T, double scale,
-                     void* stream, bool route_single = false, double v_scale = 1.0) {
+                     void* stream, bool route_single = false, double v_scale = 1.0, const PrefillWorkspace& ws = {},
+                     size_t before = 0) {
   if (!route_single) g_launches.clear();
   // kernels/paged_attn_wmma.cu:220-223 requires fp16; bf16 and FP8 (E4M3, read
   // as fp16) are served as well.
-  if (a.kv_dtype != kF16 && a.kv_dtype != kBF16 && a.kv_dtype != kFP8)
+  if (!prefill_kv(a.kv_dtype))
     return fail(PA_ERR_INVALID_ARGUMENT, "the MFMA path needs an fp16, bf16 or float8_e4m3fn KV cache");
   if (a.p.D > 256) return fail(PA_ERR_UNSUPPORTED, "unsupported head_dim for the MFMA path: %d", a.p.D);
   if ((int64_t)a.p.B * a.p.Sq * a.p.H == 0) return PA_OK;
-  if ((reinterpret_cast<uintptr_t>(q->data) & 15) != 0)
+  if (!aligned16(q->data))
     return fail(PA_ERR_UNSUPPORTED, "the MFMA path needs a 16-byte aligned q");
   PrefillParams pp = prefill_params(a, cu, T, scale);
   pp.skip_single = route_single ? 1 : 0;
   pp.vscale = (float)v_scale;
+  int rc;
+  if ((rc = bind_split(pp, cu != nullptr, ws, before))) return rc;
   return hip_status(launch_prefill_mfma(pp, a.kv_dtype, static_cast<hipStream_t>(stream)),
                     "prefill kernel launch");
+}
+
+int run_wmma_scaled(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const pa_tensor_t* v,
+                    const pa_tensor_t* bt, const pa_tensor_t* ctx, double scale, double k_scale, double v_scale,
+                    void* stream, const PrefillWorkspace& ws) {
+  if (!finite_f32(k_scale) || !finite_f32(v_scale))
+    return fail(PA_ERR_INVALID_ARGUMENT, "k_scale and v_scale must be finite");
+  // k_scale joins the softmax scale (q . (k_scale k) = (scale k_scale) q . k),
+  // v_scale multiplies the output rows.
+  DecodeArgs a;
+  int rc = check_args(out, q, k, v, bt, ctx, scale * k_scale, true, &a);
+  if (rc) return rc;
+  return run_prefill_mfma(a, q, nullptr, 0, scale * k_scale, stream, false, v_scale, ws);
+}
+
+int run_varlen(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k_cache, const pa_tensor_t* v_cache,
+               const pa_tensor_t* block_tables, const pa_tensor_t* context_lens, const pa_tensor_t* cu_seqlens_q,
+               int64_t max_q_len, double scale, double k_scale, double v_scale, void* stream,
+               const PrefillWorkspace& ws) {
+  int rc;
+  if (!finite_f32(k_scale) || !finite_f32(v_scale))
+    return fail(PA_ERR_INVALID_ARGUMENT, "k_scale and v_scale must be finite");
+  if ((rc = check_tensor(q, "q", 3, "[T, H, D]"))) return rc;
+  if ((rc = check_tensor(out, "out", 3, "[T, H, D]"))) return rc;
+  if ((rc = check_tensor(block_tables, "block_tables", 2, "[B, MB]"))) return rc;
+  if ((rc = check_tensor(cu_seqlens_q, "cu_seqlens_q", 1, "[B + 1]"))) return rc;
+  for (int i = 0; i < 3; ++i)
+    if (out->shape[i] != q->shape[i]) return fail(PA_ERR_INVALID_ARGUMENT, "out must have the shape of q");
+  if (!is_contiguous(q)) return fail(PA_ERR_INVALID_ARGUMENT, "q must be contiguous");
+  if (!is_contiguous(out)) return fail(PA_ERR_INVALID_ARGUMENT, "out must be contiguous");
+  const int64_t B = block_tables->shape[0], T = q->shape[0];
+  if (cu_seqlens_q->dtype != kI32) return fail(PA_ERR_INVALID_ARGUMENT, "cu_seqlens_q must be int32");
+  if (cu_seqlens_q->shape[0] != B + 1) return fail(PA_ERR_INVALID_ARGUMENT, "cu_seqlens_q must have B + 1 entries");
+  if (cu_seqlens_q->stride[0] != 1) return fail(PA_ERR_INVALID_ARGUMENT, "cu_seqlens_q must be contiguous");
+  if (max_q_len < 0) return fail(PA_ERR_INVALID_ARGUMENT, "max_q_len must be non-negative");
+  if (T >= (1LL << 31)) return fail(PA_ERR_UNSUPPORTED, "too many query tokens");
+  // The attention checks run on [B, max_q_len, H, D] descriptors of the packed
+  // q/out (shape and type checks only; rows are addressed through cu_seqlens_q).
+  const int64_t mq = std::max<int64_t>(max_q_len, 1);
+  pa_tensor_t q4 = {q->data, q->dtype, 4, {B, mq, q->shape[1], q->shape[2]},
+                    {mq * q->shape[1] * q->shape[2], q->shape[1] * q->shape[2], q->shape[2], 1}};
+  pa_tensor_t o4 = q4;
+  o4.data = out->data;
+  o4.dtype = out->dtype;
+  DecodeArgs a;
+  rc = check_args(&o4, &q4, k_cache, v_cache, block_tables, context_lens, scale * k_scale, true, &a);
+  if (rc) return rc;
+  if (max_q_len == 0 || T == 0) return PA_OK;
+  a.p.Sq = (int)std::min<int64_t>(mq, T);  // no sequence has more than T rows
+  g_launches.clear();
+  const int32_t* cu = static_cast<const int32_t*>(cu_seqlens_q->data);
+  // Sequences that bring one query row (decode steps of the batch) go to the
+  // decode kernel, one launch over every sequence in which the others' work-
+  // groups exit at once; the prefill kernel then skips them.  The rows are
+  // told apart on the device (cu_seqlens_q is device memory: no host sync).
+  const bool prefill_ok =
+      prefill_kv(a.kv_dtype) && a.p.D <= 256 && aligned16(q->data) && (int64_t)a.p.B * a.p.H > 0;
+  size_t decode_bytes = 0;
+  if (prefill_ok) {  // (otherwise the prefill call below reports why, before any launch)
+    DecodeArgs d = a;  // check_args folded k_scale into d.p.qscale
+    d.p.vscale = (float)v_scale;
+    d.p.Sq = 1;
+    d.p.cu_q = cu;
+    d.p.q_total = T;
+    d.p.parts = 1;
+    d.p.part_tokens = 0;
+    d.p.direct = 1;
+    // With a workspace the decode rows split too (plan_varlen_decode).
+    Plan plan;
+    plan.direct = true;
+    if (ws.given) {
+      if ((rc = plan_varlen_decode(d.p, d.gc, dtype_bytes(d.kv_dtype), &plan))) return rc;
+      decode_bytes = workspace_bytes_for(d.p.B, d.p.H, d.p.D, plan);
+      PrefillParams pp = prefill_params(a, cu, T, scale * k_scale);  // every check before the first launch
+      if ((rc = bind_split(pp, true, ws, decode_bytes))) return rc;
+    }
+    if (plan.direct) {
+      int cus = 0;
+      if ((rc = device_cu_count(&cus))) return rc;
+      d.p.hp = pack_for(d.p, dtype_bytes(d.kv_dtype), 1, cus);
+    } else {
+      d.p.parts = (int)plan.parts;
+      d.p.part_tokens = (int)plan.part_tokens;
+      d.p.direct = 0;
+      d.p.hp = plan.hp;
+      bind_workspace(&d.p, ws.ptr, plan);
+    }
+    if ((rc = hip_status(launch_decode(d.p, d.kv_dtype, d.gc, static_cast<hipStream_t>(stream)),
+                         "decode kernel launch")))
+      return rc;
+    if (!plan.direct && (rc = hip_status(launch_reduce(reduce_params(d.p), static_cast<hipStream_t>(stream)),
+                                         "reduce kernel launch")))
+      return rc;
+  }
+  return run_prefill_mfma(a, q, cu, T, scale * k_scale, stream, true, v_scale, ws, decode_bytes);
 }
 
 }  // namespace
@@ -761,14 +917,7 @@ int paged_attention_prefill_wmma_scaled(pa_tensor_t* out, const pa_tensor_t* q, 
                                         const pa_tensor_t* v_cache, const pa_tensor_t* block_tables,
                                         const pa_tensor_t* context_lens, double scale, double k_scale,
                                         double v_scale, void* stream) {
-  if (!finite_f32(k_scale) || !finite_f32(v_scale))
-    return fail(PA_ERR_INVALID_ARGUMENT, "k_scale and v_scale must be finite");
-  // k_scale joins the softmax scale (q . (k_scale k) = (scale k_scale) q . k),
-  // v_scale multiplies the output rows.
-  DecodeArgs a;
-  int rc = check_args(out, q, k_cache, v_cache, block_tables, context_lens, scale * k_scale, true, &a);
-  if (rc) return rc;
-  return run_prefill_mfma(a, q, nullptr, 0, scale * k_scale, stream, false, v_scale);
+  return run_wmma_scaled(out, q, k_cache, v_cache, block_tables, context_lens, scale, k_scale, v_scale, stream, {});
 }
 
 int paged_attention_prefill_varlen(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k_cache,
@@ -784,61 +933,66 @@ int paged_attention_prefill_varlen_scaled(pa_tensor_t* out, const pa_tensor_t* q
                                           const pa_tensor_t* context_lens, const pa_tensor_t* cu_seqlens_q,
                                           int64_t max_q_len, double scale, double k_scale, double v_scale,
                                           void* stream) {
-  int rc;
-  if (!finite_f32(k_scale) || !finite_f32(v_scale))
-    return fail(PA_ERR_INVALID_ARGUMENT, "k_scale and v_scale must be finite");
-  if ((rc = check_tensor(q, "q", 3, "[T, H, D]"))) return rc;
-  if ((rc = check_tensor(out, "out", 3, "[T, H, D]"))) return rc;
-  if ((rc = check_tensor(block_tables, "block_tables", 2, "[B, MB]"))) return rc;
-  if ((rc = check_tensor(cu_seqlens_q, "cu_seqlens_q", 1, "[B + 1]"))) return rc;
-  for (int i = 0; i < 3; ++i)
-    if (out->shape[i] != q->shape[i]) return fail(PA_ERR_INVALID_ARGUMENT, "out must have the shape of q");
-  if (!is_contiguous(q)) return fail(PA_ERR_INVALID_ARGUMENT, "q must be contiguous");
-  if (!is_contiguous(out)) return fail(PA_ERR_INVALID_ARGUMENT, "out must be contiguous");
-  const int64_t B = block_tables->shape[0], T = q->shape[0];
-  if (cu_seqlens_q->dtype != kI32) return fail(PA_ERR_INVALID_ARGUMENT, "cu_seqlens_q must be int32");
-  if (cu_seqlens_q->shape[0] != B + 1) return fail(PA_ERR_INVALID_ARGUMENT, "cu_seqlens_q must have B + 1 entries");
-  if (cu_seqlens_q->stride[0] != 1) return fail(PA_ERR_INVALID_ARGUMENT, "cu_seqlens_q must be contiguous");
-  if (max_q_len < 0) return fail(PA_ERR_INVALID_ARGUMENT, "max_q_len must be non-negative");
-  if (T >= (1LL << 31)) return fail(PA_ERR_UNSUPPORTED, "too many query tokens");
-  // The attention checks run on [B, max_q_len, H, D] descriptors of the packed
-  // q/out (shape and type checks only; rows are addressed through cu_seqlens_q).
-  const int64_t mq = std::max<int64_t>(max_q_len, 1);
-  pa_tensor_t q4 = {q->data, q->dtype, 4, {B, mq, q->shape[1], q->shape[2]},
-                    {mq * q->shape[1] * q->shape[2], q->shape[1] * q->shape[2], q->shape[2], 1}};
-  pa_tensor_t o4 = q4;
-  o4.data = out->data;
-  o4.dtype = out->dtype;
-  DecodeArgs a;
-  rc = check_args(&o4, &q4, k_cache, v_cache, block_tables, context_lens, scale * k_scale, true, &a);
-  if (rc) return rc;
-  if (max_q_len == 0 || T == 0) return PA_OK;
-  a.p.Sq = (int)std::min<int64_t>(mq, T);  // no sequence has more than T rows
-  g_launches.clear();
-  const int32_t* cu = static_cast<const int32_t*>(cu_seqlens_q->data);
-  // Sequences that bring one query row (decode steps of the batch) go to the
-  // decode kernel, one launch over every sequence in which the others' work-
-  // groups exit at once; the prefill kernel then skips them.  The rows are
-  // told apart on the device (cu_seqlens_q is device memory: no host sync).
-  const bool prefill_ok = (a.kv_dtype == kF16 || a.kv_dtype == kBF16 || a.kv_dtype == kFP8) && a.p.D <= 256 &&
-                          (reinterpret_cast<uintptr_t>(q->data) & 15) == 0 && (int64_t)a.p.B * a.p.H > 0;
-  if (prefill_ok) {  // (otherwise the prefill call below reports why, before any launch)
-    DecodeArgs d = a;  // check_args folded k_scale into d.p.qscale
-    d.p.vscale = (float)v_scale;
-    d.p.Sq = 1;
-    d.p.cu_q = cu;
-    d.p.q_total = T;
-    d.p.parts = 1;
-    d.p.part_tokens = 0;
-    d.p.direct = 1;
-    int cus = 0;
-    if ((rc = device_cu_count(&cus))) return rc;
-    d.p.hp = pack_for(d.p, dtype_bytes(d.kv_dtype), 1, cus);
-    if ((rc = hip_status(launch_decode(d.p, d.kv_dtype, d.gc, static_cast<hipStream_t>(stream)),
-                         "decode kernel launch")))
-      return rc;
+  return run_varlen(out, q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, max_q_len, scale, k_scale,
+                    v_scale, stream, {});
+}
+
+size_t paged_attention_prefill_workspace_size(const pa_tensor_t* q, const pa_tensor_t* k_cache,
+                                              const pa_tensor_t* block_tables, int64_t max_q_len) {
+  if (!q || (q->ndim != 3 && q->ndim != 4)) {
+    fail(PA_ERR_INVALID_ARGUMENT, "q must be [B, S, H, D] or [T, H, D]");
+    return (size_t)-1;
   }
-  return run_prefill_mfma(a, q, cu, T, scale * k_scale, stream, true, v_scale);
+  const bool varlen = q->ndim == 3;
+  if (check_tensor(q, "q", q->ndim, varlen ? "[T, H, D]" : "[B, S, H, D]") ||
+      check_tensor(k_cache, "k_cache", 4, "[NB, BS, H, D]") || check_tensor(block_tables, "block_tables", 2, "[B, MB]"))
+    return (size_t)-1;
+  const int64_t H = q->shape[q->ndim - 2], HKV = k_cache->shape[2];
+  if (HKV <= 0 || H <= 0 || H % HKV || k_cache->shape[1] <= 0) {
+    fail(PA_ERR_INVALID_ARGUMENT, HKV <= 0 || H <= 0 || H % HKV ? "n_head must be divisible by n_kv_head"
+                                                                : "block_size must be positive");
+    return (size_t)-1;
+  }
+  if (!prefill_kv(k_cache->dtype) || !aligned16(q->data) || numel(q) == 0) return 0;  // not split
+  PrefillParams pp;
+  memset(&pp, 0, sizeof(pp));
+  pp.B = (int)block_tables->shape[0];
+  pp.q_total = q->shape[0];
+  pp.S = (int)(varlen ? std::min<int64_t>(std::max<int64_t>(max_q_len, 1), q->shape[0]) : q->shape[1]);
+  pp.H = (int)H; pp.G = (int)(H / HKV); pp.D = (int)q->shape[q->ndim - 1];
+  pp.BS = (int)k_cache->shape[1]; pp.MB = (int)block_tables->shape[1];
+  pack_heads(pp);
+  int cus = 0;
+  if (device_cu_count(&cus)) return (size_t)-1;
+  const size_t bytes = plan_prefill_split(pp, varlen, cus);
+  if (!varlen) return bytes;
+  // The decode rows' split comes first.
+  DecodeParams d;
+  memset(&d, 0, sizeof(d));
+  d.B = pp.B; d.Sq = 1; d.H = pp.H; d.HKV = (int)HKV; d.G = pp.G; d.D = pp.D; d.BS = pp.BS; d.MB = pp.MB;
+  d.k_sh = k_cache->stride[2];
+  Plan plan;
+  if (plan_varlen_decode(d, decode_heads_per_wg(d.G), dtype_bytes(k_cache->dtype), &plan)) return (size_t)-1;
+  return bytes + workspace_bytes_for(d.B, d.H, d.D, plan);
+}
+
+int paged_attention_prefill_split(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k_cache,
+                                  const pa_tensor_t* v_cache, const pa_tensor_t* block_tables,
+                                  const pa_tensor_t* context_lens, const pa_tensor_t* cu_seqlens_q,
+                                  int64_t max_q_len, double scale, double k_scale, double v_scale,
+                                  int fp32_precision, void* workspace, size_t workspace_bytes, void* stream) {
+  PrefillWorkspace ws;
+  ws.ptr = workspace;
+  ws.bytes = workspace_bytes;
+  ws.given = true;
+  if (!fp32_precision && cu_seqlens_q)
+    return run_varlen(out, q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, max_q_len, scale, k_scale,
+                      v_scale, stream, ws);
+  if (!fp32_precision)
+    return run_wmma_scaled(out, q, k_cache, v_cache, block_tables, context_lens, scale, k_scale, v_scale, stream, ws);
+  if (cu_seqlens_q || k_scale != 1.0 || v_scale != 1.0)
+    return fail(PA_ERR_UNSUPPORTED, "the fp32-precision prefill serves uniform batches over unscaled caches");
+  return run_direct(out, q, k_cache, v_cache, block_tables, context_lens, scale, true, stream, ws);
 }
 
 int pa_write_kv(pa_tensor_t* k_cache, pa_tensor_t* v_cache, const pa_tensor_t* key,

@@ -87,6 +87,8 @@ struct ReduceParams {
   int32_t out_dtype;
   int32_t parts;
   int32_t part_tokens;
+  const int32_t* cu_q;  // variable-length batches: as DecodeParams
+  int64_t q_total;
 };
 
 struct PrefillParams {
@@ -118,7 +120,71 @@ struct PrefillParams {
   float vscale;      // v_scale of a scaled (FP8) cache: multiplies the output rows
   uint32_t q_and;    // the same on packed 16-bit q: bits & q_and ^ q_xor
   uint32_t q_xor;
+  // Context split (parts > 1).
+  int32_t units;       // units of the grid, per partition
+  int32_t parts;       // most partitions per unit
+  int32_t part_tiles;  // key tiles per partition
+  float* ws_acc;       // [units][parts][rows][D] un-normalised sums
+  float* ws_m;         // [units][parts][rows] reference points (log2 units; -inf: no key)
+  float* ws_l;         // [units][parts][rows] row sums (NaN: an unreadable key)
 };
+
+constexpr int kPfMinPartTiles = 4;  // fewest key tiles per partition of a prefill split
+constexpr int kVlMaxSeqs = 256;  // variable-length batches numbered compactly (four sequences per lane)
+
+// Rows per unit of a context-split prefill grid and keys per tile.
+inline int pf_split_rows(int D) { return D <= 128 ? 64 : 128; }
+inline int pf_tile_keys(int D) { return D <= 128 ? 64 : 32; }
+
+// Most units of a compacted variable-length grid of QB-row blocks.
+inline int64_t pf_compact_units(const PrefillParams& p, int QB) {
+  const int64_t tiles = ((int64_t)p.S * p.gp + QB - 1) / QB;
+  const int64_t by_rows = (p.q_total * p.gp + QB - 1) / QB + (p.B < p.q_total ? p.B : p.q_total);
+  return p.HG * (p.B * tiles < by_rows ? p.B * tiles : by_rows);
+}
+
+// Context split of a prefill grid on `cus` compute units: sets parts and
+// part_tiles, returns the bytes of workspace the partitions' sums take (0: no
+// split).
+// A work-group alone on its CU takes tile_us per 64-key tile (measured: D = 64
+// 0.86, D = 128 1.3), two take 1.25-1.35 times that between them, and a third
+// or fourth adds nothing: so a grid is brought to at most two work-groups per
+// CU, and only where the shorter chains save more than the second launch and
+// the partial sums cost (5-7 us; a variable-length
+// batch, whose grid holds idle work-groups, 12).  B = 1, S = 16, context 12288: 12 heads of
+// 64 150 -> 20 us, 32/8 heads of 128 242 -> 27 us; B = 1, S = 64, context
+// 1024: 17.5 -> 12.5 and 27.8 -> 15.7; B = 1, S = 512, context 8192, 32/8
+// heads (256 blocks, two partitions): 161 -> 111.  Without the two bounds
+// B = 4, S = 512, context 2048, 12 heads (384 blocks) took 37.1 instead of
+// 33.5 us, S = 1024 of 16/4 heads of 64 (256 blocks, 16 tiles) 19.9 instead
+// of 17.9.
+inline size_t plan_prefill_split(PrefillParams& p, bool varlen, int cus) {
+  p.parts = 1;
+  p.part_tiles = 0;
+  if (varlen && p.B > kVlMaxSeqs) return 0;
+  const int QB = pf_split_rows(p.D), KB = pf_tile_keys(p.D);
+  const int64_t tiles = ((int64_t)p.S * p.gp + QB - 1) / QB;
+  const int64_t units = varlen ? pf_compact_units(p, QB) : (int64_t)p.B * p.HG * tiles;
+  // Blocks with rows (a variable-length batch's: about its rows over QB).
+  const int64_t by_rows = p.HG * ((p.q_total * p.gp + QB - 1) / QB);
+  const int64_t busy = varlen && by_rows < units ? by_rows : units;
+  const int64_t key_tiles = ((int64_t)p.MB * p.BS + KB - 1) / KB;
+  if (busy <= 0) return 0;
+  int64_t n = 2 * (int64_t)cus / busy;
+  if (n > key_tiles / kPfMinPartTiles) n = key_tiles / kPfMinPartTiles;
+  const double tile_us = p.D <= 64 ? 0.86 : 1.3;
+  if (n < 2 || (double)key_tiles * tile_us * (1.0 - 1.35 / (double)n) < (varlen ? 12.0 : 7.0)) return 0;
+  p.part_tiles = (int32_t)((key_tiles + n - 1) / n);
+  p.parts = (int32_t)((key_tiles + p.part_tiles - 1) / p.part_tiles);
+  return (size_t)units * p.parts * QB * (p.D + 2) * 4;
+}
+// The workspace's sections for that plan.
+inline void bind_prefill_split(PrefillParams& p, void* ws, size_t bytes) {
+  const size_t rows = bytes / ((size_t)(p.D + 2) * 4);
+  p.ws_acc = static_cast<float*>(ws);
+  p.ws_m = p.ws_acc + rows * p.D;
+  p.ws_l = p.ws_m + rows;
+}
 
 // KV-cache write: new [T, HKV, D] rows -> paged pool slots (element strides).
 struct WriteParams {
@@ -187,6 +253,8 @@ hipError_t launch_decode(const DecodeParams& p, int kv_dtype, int gc, hipStream_
 extern thread_local int t_decode_fused;
 hipError_t launch_reduce(const ReduceParams& p, hipStream_t stream);
 hipError_t launch_prefill_mfma(const PrefillParams& p, int kv_dtype, hipStream_t stream);
+hipError_t launch_prefill_part(const PrefillParams& p, int kv_dtype, hipStream_t stream);
+hipError_t launch_prefill32_part(const PrefillParams& p, int kv_dtype, hipStream_t stream);
 hipError_t launch_prefill32(const PrefillParams& p, int kv_dtype, hipStream_t stream);
 hipError_t launch_write_kv(const WriteParams& p, hipStream_t stream);
 

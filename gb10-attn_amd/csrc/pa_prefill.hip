@@ -9,25 +9,10 @@ static hipError_t launch_pf_q(const PrefillParams& p, hipStream_t stream) {
   static std::atomic<int64_t> cache[64];
   const auto kernel = prefill_mfma_kernel<KV, D, kSplitQ, kSplit>;
   PrefillParams q = p;
-  constexpr int QB = kSplit ? 2 * PfShape<D>::QW : PfShape<D>::QB;
-  q.q_tiles = (int32_t)(((int64_t)p.S * p.gp + QB - 1) / QB);
-  int64_t units = (int64_t)q.B * q.HG * q.q_tiles;
-  int64_t cus = 0, per_cu = 0;
-  residency(kernel, cache, &cus, &per_cu);
-  q.wg_cus = units > cus && units <= cus * per_cu ? (int32_t)cus : 0;  // one resident wave
-  // Variable-length batches of up to kVlMaxSeqs sequences: a compacted grid
-  // of at most the units with rows (sum over sequences of ceil(rows / QB) <
-  // T / QB + sequences).
-  q.vl_compact = 0;
-  if (p.cu_q && p.B <= kVlMaxSeqs) {
-    const int64_t ub = (p.q_total * p.gp + QB - 1) / QB + std::min<int64_t>(p.B, p.q_total);
-    units = (int64_t)q.HG * std::min<int64_t>((int64_t)q.B * q.q_tiles, ub);
-    q.vl_compact = 1;
-    q.wg_cus = 0;
-  }
+  const int64_t blocks = pf_grid(kernel, cache, kSplit ? 2 * PfShape<D>::QW : PfShape<D>::QB, q);
   note_launch("pa::prefill_mfma_kernel<%s, %d, %s, %s>", KV::kName, D, kSplitQ ? "true" : "false",
               kSplit ? "true" : "false");
-  hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(kPfThreads), 0, stream, q);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kPfThreads), 0, stream, q);
   return hipGetLastError();
 }
 
@@ -68,7 +53,7 @@ static hipError_t launch_pf(const PrefillParams& p, hipStream_t stream) {
       return (int64_t)p.H * (p.cu_q ? std::min<int64_t>(grid, (p.q_total + rows - 1) / rows) : grid);
     };
     const int64_t plain = busy(PfShape<D>::QB);
-    if (cus > 0 && plain < cus)
+    if ((cus > 0 && plain < cus) || (!p.cu_q && (int64_t)p.S * p.gp <= 64))
       return p.q_split ? launch_pf_q<KV, D, true, true>(p, stream) : launch_pf_q<KV, D, false, true>(p, stream);
     // The 8-wave kernel (one work-group per CU) for grids of at least two
     // of its work-groups per CU; below that its 256-row blocks leave CUs
@@ -93,6 +78,7 @@ static hipError_t launch_pf_kv(const PrefillParams& p, hipStream_t stream) {
 }
 
 hipError_t launch_prefill_mfma(const PrefillParams& p, int kv_dtype, hipStream_t stream) {
+  if (p.parts > 1) return launch_prefill_part(p, kv_dtype, stream);
   if (kv_dtype == kF16) return launch_pf_kv<KvF16>(p, stream);
   if (kv_dtype == kBF16) return launch_pf_kv<KvBF16>(p, stream);
   if (kv_dtype == kFP8) return p.q_dtype == kBF16 ? launch_pf_kv<KvFP8QkBf16>(p, stream) : launch_pf_kv<KvFP8>(p, stream);

@@ -133,7 +133,6 @@ __device__ inline void load8f(const void* q, int dtype, int64_t idx, float (&x)[
 }
 
 constexpr int kPfThreads = 256;   // 4 waves
-constexpr int kVlMaxSeqs = 256;   // variable-length batches numbered compactly (four per lane)
 constexpr int kPfBtStage = 1024;  // block-table entries staged in LDS
 constexpr float kLazyRescale = 8.0f;  // raise the running max only past 2^8
 constexpr float kWeightCap = 32768.0f;  // 8-wave kernel: raise it when a lane's weights sum past 2^15
@@ -210,6 +209,124 @@ __device__ inline int swv(int row, int cc) {
   return row * D + (vpos<D>(row, cc) << 3);
 }
 
+// Work-group x -> partition (context split, the slow index) and unit (b, head
+// group, block of QB packed rows); false past the last unit of a compacted
+// grid (work-group uniform).
+template <int QB, bool kPart>
+__device__ __forceinline__ bool pf_unit(const PrefillParams& p, int64_t x, int lane, int& part, int64_t& unit, int& qt,
+                                        int& hg, int& b) {
+  part = 0;
+  // Work-group -> unit (b, h, query block).  Units are numbered with the
+  // query block as the slow index, longest first across all (sequence, head)
+  // pairs.  When the grid is more than one resident wave, work-group x takes
+  // unit x: the dispatcher hands the longest remaining unit to each CU slot
+  // that frees.  When every work-group is resident at once (p.wg_cus = C
+  // CUs), the dispatcher places work-groups x, x + C, x + 2C, ... on one CU;
+  // odd generations then take their units mirrored, so each CU's units add
+  // up to about the same number of key tiles (config 4a: 27-28 per CU instead
+  // of 20-34).  The mirror keeps x mod 8 (work-groups go to the 8 XCDs round
+  // robin), so a (sequence, head) pair's blocks, which read the same keys,
+  // stay on one XCD's L2.
+  const int nq = p.q_tiles;
+  const int64_t nbh = (int64_t)p.B * p.HG;
+  if (p.vl_compact) {
+    // Variable-length batch, compacted grid: the work-groups take only the
+    // (query block, sequence, head) units that have rows -- query blocks
+    // from the last (longest) down, then sequences, then heads -- and those
+    // past the last unit exit.  A grid sized by the longest sequence would
+    // dispatch a work-group for every block of every sequence, most of them
+    // (decode rows of a mixed batch, blocks past a short sequence's rows)
+    // exiting only after a memory round trip, and spread the working ones
+    // across the launch.  Per-sequence block counts sit in the lanes
+    // (kVlMaxSeqs / 64 per lane); each level costs one ballot per chunk.
+    int nbk[kVlMaxSeqs / 64];
+#pragma unroll
+    for (int c = 0; c < kVlMaxSeqs / 64; ++c) {
+      const int i = c * 64 + lane;
+      nbk[c] = 0;
+      if (i < p.B) {
+        const int qa = p.cu_q[i], qb = p.cu_q[i + 1];
+        int len = qa >= 0 && qb >= qa && (int64_t)qb <= p.q_total ? qb - qa : 0;
+        if (p.skip_single && len == 1) len = 0;
+        nbk[c] = (min(len, p.S) * p.gp + QB - 1) / QB;
+      }
+    }
+    if constexpr (kPart) {  // the partitions of the units there are, so that the idle work-groups come last
+      int mine = 0;
+#pragma unroll
+      for (int c = 0; c < kVlMaxSeqs / 64; ++c) mine += nbk[c];
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) mine += __shfl_xor(mine, o, 64);
+      const int64_t total = (int64_t)mine * p.HG;
+      if (x >= total * p.parts) return false;
+      part = (int)(x / total);
+      x -= part * total;
+    }
+    unit = x;
+    int64_t rem = x;
+    int fb = -1, ft = 0, fh = 0;
+    for (int t = nq - 1; t >= 0 && fb < 0; --t) {  // wave-uniform
+#pragma unroll
+      for (int c = 0; c < kVlMaxSeqs / 64; ++c) {
+        const uint64_t m = __builtin_amdgcn_ballot_w64(nbk[c] > t);
+        const int64_t cnt = (int64_t)__builtin_popcountll(m) * p.HG;
+        if (fb < 0) {
+          if (rem < cnt) {
+            const int k = (int)(rem / p.HG);
+            const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            const uint64_t sel = __builtin_amdgcn_ballot_w64(((m >> lane) & 1u) != 0 && rank == k);
+            fb = c * 64 + __builtin_ctzll(sel);
+            ft = t;
+            fh = (int)(rem - (int64_t)k * p.HG);
+          } else {
+            rem -= cnt;
+          }
+        }
+      }
+    }
+    if (fb < 0) return false;
+    qt = ft;
+    hg = fh;
+    b = fb;
+  } else {
+    if constexpr (kPart) {
+      part = (int)(x / p.units);
+      x -= (int64_t)part * p.units;
+    }
+    unit = x;
+    if (p.wg_cus > 0) {
+      const int64_t C = p.wg_cus, g = x / C, j = x - g * C;
+      if ((g & 1) && (g + 1) * C <= nbh * nq) x = g * C + (C % 8 == 0 ? C - 8 - (j & ~(int64_t)7) + (j & 7) : C - 1 - j);
+    }
+    qt = nq - 1 - (int)(x / nbh);
+    const int64_t bh = x % nbh;
+    hg = (int)(bh % p.HG);
+    b = (int)(bh / p.HG);
+  }
+  return true;
+}
+
+// A sequence's query rows: `S` of them (row r at position ctx - S + r)
+// starting at token tok0 of q/out, of which `served` are; false when the
+// decode kernel serves the sequence.
+__device__ __forceinline__ bool pf_rows(const PrefillParams& p, int b, int& S, int64_t& tok0, int& served) {
+  // Uniform batches: p.S rows each.  Variable-length batches: rows cu_q[b] ..
+  // cu_q[b+1] of the packed [T, H, D] q/out, at most p.S (the caller's
+  // max_q_len) of them served; a malformed range (negative, decreasing or
+  // past T) is treated as empty.
+  S = p.S;
+  tok0 = (int64_t)b * p.S;
+  if (p.cu_q) {
+    const int qa = p.cu_q[b], qb = p.cu_q[b + 1];
+    const bool ok = qa >= 0 && qb >= qa && (int64_t)qb <= p.q_total;
+    S = ok ? qb - qa : 0;
+    tok0 = ok ? qa : 0;
+    if (p.skip_single && S == 1) return false;
+  }
+  served = min(S, p.S);
+  return true;
+}
+
 // kSplit (key-split mode, tiles of two 32-key m-tiles): a work-group serves
 // 64 query rows; waves 0-1 own rows 0-31 / 32-63 over the first 32 keys of
 // every tile, waves 2-3 the same rows over the second 32, and the two halves
@@ -236,7 +353,11 @@ __device__ inline int swv(int row, int cc) {
 // fp16 cache, fp32 q: 1105 us as a decode problem per query row on the vector
 // ALU -> 42 us (10 -> 266 TFLOP/s; the fp32 matrix rate is 154), error against
 // 64 bits 3.2e-7 -> 2.5e-7.
-template <typename KV, int D, int kQP, bool kSplit, bool kX>
+//
+// kPart (context split, split_prefill*_kernel): the work-group computes one
+// partition of its block's key tiles and writes partial sums.  An instance of
+// its own: as a run-time choice it cost the others 1-6 %.
+template <typename KV, int D, int kQP, bool kSplit, bool kX, bool kPart>
 __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
   using Sh = PfShape<D>;
   constexpr int QW = Sh::QW, KB = Sh::KB, MT = Sh::MT, KS = Sh::KS, DT = Sh::DT;
@@ -268,97 +389,16 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
   const int n = lane & 31;   // query column of this lane (S^T, O^T) / key row (K operand)
   const int hh = lane >> 5;  // lane half: k-slot block of the operands
 
-  // Work-group -> unit (b, h, query block).  Units are numbered with the
-  // query block as the slow index, longest first across all (sequence, head)
-  // pairs.  When the grid is more than one resident wave, work-group x takes
-  // unit x: the dispatcher hands the longest remaining unit to each CU slot
-  // that frees.  When every work-group is resident at once (p.wg_cus = C
-  // CUs), the dispatcher places work-groups x, x + C, x + 2C, ... on one CU;
-  // odd generations then take their units mirrored, so each CU's units add
-  // up to about the same number of key tiles (config 4a: 27-28 per CU instead
-  // of 20-34).  The mirror keeps x mod 8 (work-groups go to the 8 XCDs round
-  // robin), so a (sequence, head) pair's blocks, which read the same keys,
-  // stay on one XCD's L2.
-  const int nq = p.q_tiles;
-  const int64_t nbh = (int64_t)p.B * p.HG;
-  int qt, hg, b;
-  if (p.vl_compact) {
-    // Variable-length batch, compacted grid: the work-groups take only the
-    // (query block, sequence, head) units that have rows -- query blocks
-    // from the last (longest) down, then sequences, then heads -- and those
-    // past the last unit exit.  A grid sized by the longest sequence would
-    // dispatch a work-group for every block of every sequence, most of them
-    // (decode rows of a mixed batch, blocks past a short sequence's rows)
-    // exiting only after a memory round trip, and spread the working ones
-    // across the launch.  Per-sequence block counts sit in the lanes
-    // (kVlMaxSeqs / 64 per lane); each level costs one ballot per chunk.
-    int nbk[kVlMaxSeqs / 64];
-#pragma unroll
-    for (int c = 0; c < kVlMaxSeqs / 64; ++c) {
-      const int i = c * 64 + lane;
-      nbk[c] = 0;
-      if (i < p.B) {
-        const int qa = p.cu_q[i], qb = p.cu_q[i + 1];
-        int len = qa >= 0 && qb >= qa && (int64_t)qb <= p.q_total ? qb - qa : 0;
-        if (p.skip_single && len == 1) len = 0;
-        nbk[c] = (min(len, p.S) * p.gp + QB - 1) / QB;
-      }
-    }
-    int64_t rem = blockIdx.x;
-    int fb = -1, ft = 0, fh = 0;
-    for (int t = nq - 1; t >= 0 && fb < 0; --t) {  // wave-uniform
-#pragma unroll
-      for (int c = 0; c < kVlMaxSeqs / 64; ++c) {
-        const uint64_t m = __builtin_amdgcn_ballot_w64(nbk[c] > t);
-        const int64_t cnt = (int64_t)__builtin_popcountll(m) * p.HG;
-        if (fb < 0) {
-          if (rem < cnt) {
-            const int k = (int)(rem / p.HG);
-            const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-            const uint64_t sel = __builtin_amdgcn_ballot_w64(((m >> lane) & 1u) != 0 && rank == k);
-            fb = c * 64 + __builtin_ctzll(sel);
-            ft = t;
-            fh = (int)(rem - (int64_t)k * p.HG);
-          } else {
-            rem -= cnt;
-          }
-        }
-      }
-    }
-    if (fb < 0) return;  // past the last unit (work-group uniform)
-    qt = ft;
-    hg = fh;
-    b = fb;
-  } else {
-    int64_t x = blockIdx.x;
-    if (p.wg_cus > 0) {
-      const int64_t C = p.wg_cus, g = x / C, j = x - g * C;
-      if ((g & 1) && (g + 1) * C <= nbh * nq) x = g * C + (C % 8 == 0 ? C - 8 - (j & ~(int64_t)7) + (j & 7) : C - 1 - j);
-    }
-    qt = nq - 1 - (int)(x / nbh);
-    const int64_t bh = x % nbh;
-    hg = (int)(bh % p.HG);
-    b = (int)(bh / p.HG);
-  }
+  int part, qt, hg, b;
+  int64_t unit;
+  if (!pf_unit<QB, kPart>(p, blockIdx.x, lane, part, unit, qt, hg, b)) return;  // past the last unit (work-group uniform)
   const int h0 = hg * p.gp;  // first query head of the unit
   const int kvh = h0 / p.G;
 
-  // This sequence's query rows: S of them (row r at position ctx - S + r)
-  // starting at token tok0 of q/out, of which the first Sr are served.
-  // Uniform batches: S = Sr = p.S.  Variable-length batches: rows cu_q[b] ..
-  // cu_q[b+1] of the packed [T, H, D] q/out, at most p.S (the caller's
-  // max_q_len) of them served; a malformed range (negative, decreasing or
-  // past T) is treated as empty.
-  int S = p.S;
-  int64_t tok0 = (int64_t)b * p.S;
-  if (p.cu_q) {
-    const int qa = p.cu_q[b], qb = p.cu_q[b + 1];
-    const bool ok = qa >= 0 && qb >= qa && (int64_t)qb <= p.q_total;
-    S = ok ? qb - qa : 0;
-    tok0 = ok ? qa : 0;
-    if (p.skip_single && S == 1) return;  // the decode kernel serves it (work-group uniform)
-  }
-  const int Sr = min(S, p.S) * p.gp;  // packed rows served
+  int S, served;
+  int64_t tok0;
+  if (!pf_rows(p, b, S, tok0, served)) return;
+  const int Sr = served * p.gp;  // packed rows served
   const int ctx = p.context_lens[b];
   const int maxctx = p.MB * p.BS;
   const int qs0 = qt * QB;
@@ -375,7 +415,7 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
   };
 
   if (ctx > maxctx) {  // context longer than the block table: poison rows that attend keys
-    if (live && hh == 0) {
+    if (live && hh == 0 && (!kPart || part == 0)) {
       const float fillv = ctx - S + srow < 0 ? 0.0f : __builtin_nanf("");
       const int64_t row_at = row_offset(qrow);
       for (int d = 0; d < D; ++d) store_elem(p.out, p.out_dtype, row_at + d, fillv);
@@ -388,13 +428,30 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
   }
 
   // Keys the work-group's rows can see: [0, kend); this wave's rows: [0, wave_kend).
-  const int kend = min(ctx, ctx - S + chunk_row(min(qs0 + QB, Sr) - 1) + 1);
-  const int ntiles = kend > 0 ? (kend + KB - 1) / KB : 0;
+  int kend = min(ctx, ctx - S + chunk_row(min(qs0 + QB, Sr) - 1) + 1);
+  int ntiles = kend > 0 ? (kend + KB - 1) / KB : 0;
   const int wave_last = min(qw0 + QW - 1, Sr - 1);
-  const int wave_kend = qw0 < Sr ? min(ctx, ctx - S + chunk_row(wave_last) + 1) : 0;
-  const int wave_kfull = ctx - S + chunk_row(qw0) + 1;  // keys below this are visible to every row of the wave
+  int wave_kend = qw0 < Sr ? min(ctx, ctx - S + chunk_row(wave_last) + 1) : 0;
+  int wave_kfull = ctx - S + chunk_row(qw0) + 1;  // keys below this are visible to every row of the wave
   const int qpos = ctx - S + srow;
-  const int qlim = min(qpos, kend - 1);        // last key this column may see
+  int qlim = min(qpos, kend - 1);        // last key this column may see
+  const int npages = kend > 0 ? (int)fastdiv((uint32_t)(kend - 1), p.bs_div) + 1 : 0;
+  // Context split: partition `part` of the unit's tiles, whose keys are
+  // numbered from its first one, key0, from here on.  A unit of one partition
+  // writes its output rows, the others their partial sums.
+  int key0 = 0;
+  bool whole = true;
+  if constexpr (kPart) {
+    const int n = (ntiles + p.part_tiles - 1) / p.part_tiles;
+    if (part >= max(n, 1)) return;  // work-group uniform
+    whole = n <= 1;
+    key0 = part * p.part_tiles * KB;
+    ntiles = min(p.part_tiles, ntiles - part * p.part_tiles);
+    kend -= key0;
+    wave_kend -= key0;
+    wave_kfull -= key0;
+    qlim -= key0;
+  }
 
   // Q^T operand (row qrow, dims ks*16 + hh*8 .. +8) in the KV type.  The sign of
   // the scale is applied here (exactly), so the softmax scale below is positive.
@@ -462,7 +519,6 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
   // kPfBtStage pages starting at page win0, so a tile's loads never wait
   // behind a dependent block-table load.  The window moves (at a tile
   // boundary, between barriers) when the next tile to load leaves it.
-  const int npages = kend > 0 ? (int)fastdiv((uint32_t)(kend - 1), p.bs_div) + 1 : 0;
   int win0 = 0;
   auto stage = [&](int first) {
     win0 = first;
@@ -470,11 +526,11 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
     for (int i = threadIdx.x; i < cnt; i += kPfThreads) s_bt[i] = bt_row[first + i];
   };
   auto ensure_window = [&](int t) {  // work-group uniform
-    const int last = min(t * KB + KB, kend) - 1;
+    const int last = key0 + min(t * KB + KB, kend) - 1;
     const int plast = (int)fastdiv((uint32_t)last, p.bs_div);
     if (plast >= win0 + kPfBtStage) {
       __syncthreads();
-      stage((int)fastdiv((uint32_t)(t * KB), p.bs_div));
+      stage((int)fastdiv((uint32_t)(key0 + t * KB), p.bs_div));
       __syncthreads();
     }
   };
@@ -510,12 +566,12 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
       const int row = wave * 64 + lane;
       const int kabs = t * KB + row;
       const bool valid = kabs < kend;
-      const int kk = valid ? kabs : 0;
+      const int kk = key0 + (valid ? kabs : 0);
       const int pg = (int)fastdiv((uint32_t)kk, p.bs_div);
       const int off = kk - pg * p.BS;
       const int blk = s_bt[valid ? pg - win0 : 0];
       const bool okb = (uint64_t)(int64_t)blk < nb;
-      if (valid && !okb) badkey = min(badkey, kabs);
+      if (valid && !okb) badkey = min(badkey, key0 + kabs);
       const bool use = valid && okb;
       const uint32_t ub = use ? (uint32_t)blk : 0u, uo = use ? (uint32_t)off : 0u;
       tb[row] = u64x2_t{(uint64_t)ub * k_sbb + uo * k_stb,
@@ -844,7 +900,7 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
     // Double-buffered tiles, unrolled by two so each LDS buffer (and offset
     // table) is a distinct object: tile t+1's loads and tile t+2's offset
     // table are produced while tile t is computed; one barrier per tile.
-    stage(0);
+    stage((int)fastdiv((uint32_t)key0, p.bs_div));
     __syncthreads();
     build(0, s_off0);
     if (ntiles > 1) {
@@ -938,6 +994,7 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
     const float a = m == -__builtin_inff() ? 0.0f : fast_exp2(m - mn);
     const float c = m2 == -__builtin_inff() ? 0.0f : fast_exp2(m2 - mn);
     l = l * a + l2 * c;
+    m = mn;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
@@ -956,6 +1013,21 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
   const int qpos_e = ctx - S + chunk_row(qrow_e);
   const int64_t row_at = row_offset(qrow_e);
   const bool bad = bad_from <= qpos_e;
+  if (kPart && !whole) {  // this partition's sums (a row with an unreadable key: NaN)
+    const int64_t e = (unit * p.parts + part) * QB + rw * QW + n;
+    if (hh == 0) {
+      p.ws_m[e] = m;
+      p.ws_l[e] = bad ? __builtin_nanf("") : lt;
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<float4_t*>(p.ws_acc + e * D + dt * 32 + 8 * j + 4 * hh) =
+            float4_t{o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]};
+    }
+    return;
+  }
   // (kX: a row whose weights are all 0, every score -Inf, is 0 / 0.)
   const float inv = lt > 0.0f || (kX && qpos_e >= 0) ? p.vscale / lt : 0.0f;
   // Slots 4j .. 4j+3 of m-tile dt are 4 consecutive dims: one 8-byte (16-bit
@@ -998,14 +1070,91 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
 template <typename KV, int D, bool kSplitQ, bool kSplit>
 __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(PfShape<D>::WAVES_PER_EU)))
 void prefill_mfma_kernel(const PrefillParams p) {
-  prefill_body<KV, D, kSplitQ ? 2 : 1, kSplit, false>(p);
+  prefill_body<KV, D, kSplitQ ? 2 : 1, kSplit, false, false>(p);
 }
 
 // The fp32-precision kernel (kX above).
 template <typename KV, int D, int kQP, bool kSplit>
 __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(PfShape<D>::WAVES_PER_EU)))
 void prefill32_kernel(const PrefillParams p) {
-  prefill_body<KV, D, kQP, kSplit, true>(p);
+  prefill_body<KV, D, kQP, kSplit, true, false>(p);
+}
+
+// One partition of a context split.
+template <typename KV, int D, bool kSplitQ, bool kSplit>
+__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(PfShape<D>::WAVES_PER_EU)))
+void split_prefill_mfma_kernel(const PrefillParams p) {
+  prefill_body<KV, D, kSplitQ ? 2 : 1, kSplit, false, true>(p);
+}
+
+template <typename KV, int D, int kQP, bool kSplit>
+__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(PfShape<D>::WAVES_PER_EU)))
+void split_prefill32_kernel(const PrefillParams p) {
+  prefill_body<KV, D, kQP, kSplit, true, true>(p);
+}
+
+// Merge of a context split's partitions (log-sum-exp rule, as the decode
+// split's): one thread per 4 dims of a row, the unit's rows in blocks along
+// grid y.  Partition states and sums are a few MB: eight partitions' rows are
+// in flight per thread, since the loads' latency is what it takes.
+template <int D>
+struct PfReduce {
+  static constexpr int QB = D <= 128 ? 64 : 128;  // rows per unit of a split grid
+  static constexpr int ROWS = kPfThreads / (D / 4);
+};
+
+template <int D, bool kX>
+__global__ __launch_bounds__(kPfThreads) void prefill_reduce_kernel(const PrefillParams p) {
+  constexpr int QB = PfReduce<D>::QB, KB = PfShape<D>::KB;
+  int part, qt, hg, b, S, served;
+  int64_t unit, tok0;
+  if (!pf_unit<QB, true>(p, blockIdx.x, threadIdx.x & 63, part, unit, qt, hg, b) || part > 0) return;
+  if (!pf_rows(p, b, S, tok0, served)) return;
+  const int Sr = served * p.gp, qs0 = qt * QB;
+  const int r = blockIdx.y * PfReduce<D>::ROWS + threadIdx.x / (D / 4), d = threadIdx.x % (D / 4) * 4;
+  const int ctx = p.context_lens[b];
+  if (qs0 + r >= Sr || ctx > p.MB * p.BS) return;
+  auto chunk_row = [&](int x) { return (int)fastdiv((uint32_t)x, p.gp_div); };
+  const int kend = min(ctx, ctx - S + chunk_row(min(qs0 + QB, Sr) - 1) + 1);
+  const int n = kend > 0 ? ((kend + KB - 1) / KB + p.part_tiles - 1) / p.part_tiles : 0;
+  if (n <= 1) return;  // the unit's one partition wrote its rows
+  const int64_t e0 = unit * p.parts * QB + r;
+  float M = -__builtin_inff(), L = 0.0f;
+  float4_t acc = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  constexpr int NL = 8;
+  for (int j0 = 0; j0 < n; j0 += NL) {
+    float mj[NL], lj[NL];
+    float4_t x[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int64_t e = e0 + (int64_t)min(j0 + i, n - 1) * QB;
+      mj[i] = p.ws_m[e];
+      lj[i] = p.ws_l[e];
+      x[i] = *reinterpret_cast<const float4_t*>(p.ws_acc + e * D + d);
+    }
+    float mn = M;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) mn = fmaxf(mn, mj[i]);
+    const float ref = mn == -__builtin_inff() ? 0.0f : mn;  // (no key so far: every weight is 0)
+    const float corr = fast_exp2(M - ref);
+    M = mn;
+    L *= corr;
+    acc *= corr;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const float w = fast_exp2(mj[i] - ref);
+      if (j0 + i < n) {
+        L += w * lj[i];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c] = fmaf(w, x[i][c], acc[c]);
+      }
+    }
+  }
+  const int row = qs0 + r, sr = chunk_row(row), qpos = ctx - S + sr;
+  const float inv = L > 0.0f || L != L || (kX && qpos >= 0) ? p.vscale / L : 0.0f;
+  const int64_t at = ((tok0 + sr) * p.H + hg * p.gp + row - sr * p.gp) * D + d;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) store_elem(p.out, p.out_dtype, at + c, acc[c] * inv);
 }
 
 // Ping-pong prefill (64-key tiles; 16-bit caches with q in the KV type, or
@@ -1630,6 +1779,27 @@ static void residency(F kernel, std::atomic<int64_t> (&cache)[64], int64_t* cus,
   if (dev < 64) cache[dev].store(((int64_t)n << 8) | k, std::memory_order_relaxed);
   *cus = n;
   *per_cu = k;
+}
+
+// Grid of a 4-wave kernel of QB-row blocks: its work-groups, and the fields of
+// q that number them.
+template <typename F>
+static int64_t pf_grid(F kernel, std::atomic<int64_t> (&cache)[64], int QB, PrefillParams& q) {
+  q.q_tiles = (int32_t)(((int64_t)q.S * q.gp + QB - 1) / QB);
+  int64_t units = (int64_t)q.B * q.HG * q.q_tiles;
+  int64_t cus = 0, per_cu = 0;
+  residency(kernel, cache, &cus, &per_cu);
+  q.wg_cus = units > cus && units <= cus * per_cu ? (int32_t)cus : 0;  // one resident wave
+  // Variable-length batches of up to kVlMaxSeqs sequences: a compacted grid
+  // of at most the units with rows (sum over sequences of ceil(rows / QB) <
+  // T / QB + sequences).
+  q.vl_compact = 0;
+  if (q.cu_q && q.B <= kVlMaxSeqs) {
+    units = pf_compact_units(q, QB);
+    q.vl_compact = 1;
+    q.wg_cus = 0;
+  }
+  return units;
 }
 
 }  // namespace pa

@@ -10,14 +10,9 @@ static hipError_t launch_p32_q(const PrefillParams& p, hipStream_t stream) {
   static std::atomic<int64_t> cache[64];
   const auto kernel = prefill32_kernel<KV, D, kQP, kSplit>;
   PrefillParams q = p;
-  constexpr int QB = kSplit ? 2 * PfShape<D>::QW : PfShape<D>::QB;
-  q.q_tiles = (int32_t)(((int64_t)p.S * p.gp + QB - 1) / QB);
-  const int64_t units = (int64_t)q.B * q.HG * q.q_tiles;
-  int64_t cus = 0, per_cu = 0;
-  residency(kernel, cache, &cus, &per_cu);
-  q.wg_cus = units > cus && units <= cus * per_cu ? (int32_t)cus : 0;  // one resident wave
+  const int64_t blocks = pf_grid(kernel, cache, kSplit ? 2 * PfShape<D>::QW : PfShape<D>::QB, q);
   note_launch("pa::prefill32_kernel<%s, %d, %d, %s>", KV::kName, D, kQP, kSplit ? "true" : "false");
-  hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(kPfThreads), 0, stream, q);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kPfThreads), 0, stream, q);
   return hipGetLastError();
 }
 
@@ -50,6 +45,7 @@ static hipError_t launch_p32_kv(const PrefillParams& p, hipStream_t stream) {
 // q in the cache's 16-bit type is one exact piece; else two fp16 pieces (fp16
 // and FP8 caches) or three bf16 ones.
 hipError_t launch_prefill32(const PrefillParams& p, int kv_dtype, hipStream_t stream) {
+  if (p.parts > 1) return launch_prefill32_part(p, kv_dtype, stream);
   if (kv_dtype == kF16)
     return p.q_dtype == kF16 ? launch_p32_kv<KvF16, 1>(p, stream) : launch_p32_kv<KvF16, 2>(p, stream);
   if (kv_dtype == kBF16)

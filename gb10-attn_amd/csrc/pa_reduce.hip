@@ -59,6 +59,15 @@ __global__ __launch_bounds__(64 * kReduceWaves) void reduce_kernel(const ReduceP
   };
   load_rows(0, P);
 
+  // Output row: b, or in a variable-length batch the packed row of a sequence
+  // of exactly one row (the others have no partials).
+  int64_t row = f;
+  if (p.cu_q) {
+    const int qa = p.cu_q[b], qe = p.cu_q[b + 1];
+    if (!(qa >= 0 && qe == qa + 1 && (int64_t)qe <= p.q_total)) return;
+    row = (int64_t)qa * p.H + (f - (int64_t)b * p.H);
+  }
+
   const int maxctx = p.MB * p.BS;
   const bool fixed = p.part_tokens > 0;
   const bool ok = ctx > 0 && ctx <= maxctx;
@@ -72,7 +81,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void reduce_kernel(const ReduceP
       const float fillv = ctx <= 0 ? 0.0f : __builtin_nanf("");
       if (r == 0) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) store_elem(p.out, p.out_dtype, f * D + 4 * c + e, fillv);
+        for (int e = 0; e < 4; ++e) store_elem(p.out, p.out_dtype, row * D + 4 * c + e, fillv);
       }
       return;
     }
@@ -119,7 +128,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void reduce_kernel(const ReduceP
   L = wave_sum(L);
   if (r == 0) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) store_elem(p.out, p.out_dtype, f * D + 4 * c + e, acc[e] / L);
+    for (int e = 0; e < 4; ++e) store_elem(p.out, p.out_dtype, row * D + 4 * c + e, acc[e] / L);
   }
 }
 

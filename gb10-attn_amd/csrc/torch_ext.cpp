@@ -110,26 +110,54 @@ at::Tensor op_paged_attention_v2(const at::Tensor& q, const at::Tensor& k, const
   return call_simple(&paged_attention_v2, q, k, v, bt, ctx, scale, 3, "[B, H, D]");
 }
 
+// Scratch from the caching allocator (stream-ordered), 256-byte aligned.
+struct Scratch {
+  at::Tensor hold;
+  void* ptr = nullptr;
+  size_t bytes = 0;
+};
+
+Scratch scratch_of(const at::Tensor& q, size_t bytes) {
+  TORCH_CHECK(bytes != (size_t)-1, pa_last_error());
+  Scratch s;
+  s.bytes = bytes;
+  if (bytes > 0) {
+    s.hold = at::empty({(int64_t)bytes + 256}, q.options().dtype(at::kByte));
+    s.ptr = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(s.hold.data_ptr()) + 255) & ~uintptr_t(255));
+  }
+  return s;
+}
+
+at::Tensor prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& bt,
+                   const at::Tensor& ctx, const at::Tensor* cu, int64_t max_q_len, double scale, double k_scale,
+                   double v_scale, bool fp32) {
+  Args a = cu ? prep(q, k, v, bt, ctx, 3, "[T, H, D]") : prep(q, k, v, bt, ctx, 4, "[B, S, H, D]");
+  at::Tensor cuq;
+  if (cu) cuq = cu->to(a.q.device(), at::kInt).contiguous();
+  c10::DeviceGuard guard(a.q.device());
+  at::Tensor out = at::empty(a.q.sizes(), a.q.options().dtype(at::kFloat));
+  pa_tensor_t o = view(out), qq = view(a.q), kk = view(a.k), vv = view(a.v), bb = view(a.bt), cc = view(a.ctx), uu;
+  if (cu) uu = view(cuq);
+  Scratch s = scratch_of(a.q, paged_attention_prefill_workspace_size(&qq, &kk, &bb, max_q_len));
+  check(paged_attention_prefill_split(&o, &qq, &kk, &vv, &bb, &cc, cu ? &uu : nullptr, max_q_len, scale, k_scale,
+                                      v_scale, fp32 ? 1 : 0, s.ptr, s.bytes, stream_of(a.q)));
+  return out;
+}
+
 at::Tensor op_paged_attention_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                                       const at::Tensor& bt, const at::Tensor& ctx, double scale) {
-  return call_simple(&paged_attention_prefill, q, k, v, bt, ctx, scale, 4, "[B, S, H, D]");
+  return prefill(q, k, v, bt, ctx, nullptr, 0, scale, 1.0, 1.0, true);
 }
 
 at::Tensor op_paged_attention_prefill_wmma(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                                            const at::Tensor& bt, const at::Tensor& ctx, double scale) {
-  return call_simple(&paged_attention_prefill_wmma, q, k, v, bt, ctx, scale, 4, "[B, S, H, D]");
+  return prefill(q, k, v, bt, ctx, nullptr, 0, scale, 1.0, 1.0, false);
 }
 
 at::Tensor op_paged_attention_prefill_wmma_scaled(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                                                   const at::Tensor& bt, const at::Tensor& ctx, double scale,
                                                   double k_scale, double v_scale) {
-  Args a = prep(q, k, v, bt, ctx, 4, "[B, S, H, D]");
-  c10::DeviceGuard guard(a.q.device());
-  at::Tensor out = at::empty(a.q.sizes(), a.q.options().dtype(at::kFloat));
-  pa_tensor_t o = view(out), qq = view(a.q), kk = view(a.k), vv = view(a.v), bb = view(a.bt), cc = view(a.ctx);
-  check(paged_attention_prefill_wmma_scaled(&o, &qq, &kk, &vv, &bb, &cc, scale, k_scale, v_scale,
-                                            stream_of(a.q)));
-  return out;
+  return prefill(q, k, v, bt, ctx, nullptr, 0, scale, k_scale, v_scale, false);
 }
 
 at::Tensor op_paged_attention_v3(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
@@ -138,15 +166,8 @@ at::Tensor op_paged_attention_v3(const at::Tensor& q, const at::Tensor& k, const
   c10::DeviceGuard guard(a.q.device());
   at::Tensor out = at::empty(a.q.sizes(), a.q.options().dtype(at::kFloat));
   pa_tensor_t o = view(out), qq = view(a.q), kk = view(a.k), vv = view(a.v), bb = view(a.bt), cc = view(a.ctx);
-  const size_t ws = paged_attention_v3_workspace_size(&qq, &kk, &bb, num_splits);
-  TORCH_CHECK(ws != (size_t)-1, pa_last_error());
-  at::Tensor scratch;
-  void* wp = nullptr;
-  if (ws > 0) {
-    scratch = at::empty({(int64_t)ws + 256}, a.q.options().dtype(at::kByte));
-    wp = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(scratch.data_ptr()) + 255) & ~uintptr_t(255));
-  }
-  check(paged_attention_v3(&o, &qq, &kk, &vv, &bb, &cc, scale, num_splits, wp, ws, stream_of(a.q)));
+  Scratch s = scratch_of(a.q, paged_attention_v3_workspace_size(&qq, &kk, &bb, num_splits));
+  check(paged_attention_v3(&o, &qq, &kk, &vv, &bb, &cc, scale, num_splits, s.ptr, s.bytes, stream_of(a.q)));
   return out;
 }
 
@@ -157,15 +178,8 @@ at::Tensor op_paged_attention_v3_scaled(const at::Tensor& q, const at::Tensor& k
   c10::DeviceGuard guard(a.q.device());
   at::Tensor out = at::empty(a.q.sizes(), a.q.options().dtype(at::kFloat));
   pa_tensor_t o = view(out), qq = view(a.q), kk = view(a.k), vv = view(a.v), bb = view(a.bt), cc = view(a.ctx);
-  const size_t ws = paged_attention_v3_workspace_size(&qq, &kk, &bb, num_splits);
-  TORCH_CHECK(ws != (size_t)-1, pa_last_error());
-  at::Tensor scratch;
-  void* wp = nullptr;
-  if (ws > 0) {
-    scratch = at::empty({(int64_t)ws + 256}, a.q.options().dtype(at::kByte));
-    wp = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(scratch.data_ptr()) + 255) & ~uintptr_t(255));
-  }
-  check(paged_attention_v3_scaled(&o, &qq, &kk, &vv, &bb, &cc, scale, k_scale, v_scale, num_splits, wp, ws,
+  Scratch s = scratch_of(a.q, paged_attention_v3_workspace_size(&qq, &kk, &bb, num_splits));
+  check(paged_attention_v3_scaled(&o, &qq, &kk, &vv, &bb, &cc, scale, k_scale, v_scale, num_splits, s.ptr, s.bytes,
                                   stream_of(a.q)));
   return out;
 }
@@ -174,15 +188,7 @@ at::Tensor op_paged_attention_prefill_varlen_scaled(const at::Tensor& q, const a
                                                     const at::Tensor& bt, const at::Tensor& ctx, const at::Tensor& cu,
                                                     int64_t max_q_len, double scale, double k_scale,
                                                     double v_scale) {
-  Args a = prep(q, k, v, bt, ctx, 3, "[T, H, D]");
-  at::Tensor cuq = cu.to(a.q.device(), at::kInt).contiguous();
-  c10::DeviceGuard guard(a.q.device());
-  at::Tensor out = at::empty(a.q.sizes(), a.q.options().dtype(at::kFloat));
-  pa_tensor_t o = view(out), qq = view(a.q), kk = view(a.k), vv = view(a.v), bb = view(a.bt), cc = view(a.ctx),
-              uu = view(cuq);
-  check(paged_attention_prefill_varlen_scaled(&o, &qq, &kk, &vv, &bb, &cc, &uu, max_q_len, scale, k_scale, v_scale,
-                                              stream_of(a.q)));
-  return out;
+  return prefill(q, k, v, bt, ctx, &cu, max_q_len, scale, k_scale, v_scale, false);
 }
 
 at::Tensor op_paged_attention_prefill_varlen(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,

@@ -105,29 +105,46 @@ def paged_attention_v2(q, k_cache, v_cache, block_tables, context_lens, scale, *
                         scale, out_dtype, out, 3, "[B, H, D]")
 
 
+def _scratch(need, dev):
+    """Split scratch from torch's caching allocator (None when the plan has no split)."""
+    if need == C.c_size_t(-1).value:
+        raise RuntimeError(last_error())
+    return torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+
+
+def _prefill(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, max_q_len, scale, out_dtype, out,
+             k_scale, v_scale, fp32):
+    varlen = cu_seqlens_q is not None
+    q, k_cache, v_cache, block_tables, context_lens = _prep(
+        q, k_cache, v_cache, block_tables, context_lens, 3 if varlen else 4,
+        "[T, H, D]" if varlen else "[B, S, H, D]")
+    cu = cu_seqlens_q.to(q.device, torch.int32).contiguous() if varlen else None
+    o = _out(q, out_dtype, out)
+    L = lib()
+    with torch.cuda.device(q.device):
+        qv, kv, bt = view(q), view(k_cache), view(block_tables)
+        ws = _scratch(L.paged_attention_prefill_workspace_size(C.byref(qv), C.byref(kv), C.byref(bt), int(max_q_len)),
+                      q.device)
+        check(L.paged_attention_prefill_split(
+            C.byref(view(o)), C.byref(qv), C.byref(kv), C.byref(view(v_cache)), C.byref(bt),
+            C.byref(view(context_lens)), C.byref(view(cu)) if varlen else None, int(max_q_len), float(scale),
+            float(k_scale), float(v_scale), int(fp32), ws.data_ptr() if ws is not None else None,
+            ws.numel() if ws is not None else 0, _stream(q.device)))
+    return o
+
+
 def paged_attention_prefill(q, k_cache, v_cache, block_tables, context_lens, scale, *,
                             out_dtype=torch.float32, out=None):
-    """kernels/paged_attn_prefill.h:13-15 -- causal chunked prefill, fp32 arithmetic."""
-    return _call_simple(lib().paged_attention_prefill, q, k_cache, v_cache, block_tables,
-                        context_lens, scale, out_dtype, out, 4, "[B, S, H, D]")
+    """kernels/paged_attn_prefill.h:13-15 -- causal chunked prefill, fp32 precision."""
+    return _prefill(q, k_cache, v_cache, block_tables, context_lens, None, 0, scale, out_dtype, out, 1.0, 1.0, True)
 
 
 def paged_attention_prefill_wmma(q, k_cache, v_cache, block_tables, context_lens, scale, *,
                                  out_dtype=torch.float32, out=None, k_scale=1.0, v_scale=1.0):
     """kernels/paged_attn_wmma.h:13-15 -- causal chunked prefill on MFMA (fp16/bf16/FP8 KV).
     k_scale / v_scale dequantise a scaled cache (paged_attention_prefill_wmma_scaled)."""
-    if k_scale == 1.0 and v_scale == 1.0:
-        return _call_simple(lib().paged_attention_prefill_wmma, q, k_cache, v_cache, block_tables,
-                            context_lens, scale, out_dtype, out, 4, "[B, S, H, D]")
-    q, k_cache, v_cache, block_tables, context_lens = _prep(
-        q, k_cache, v_cache, block_tables, context_lens, 4, "[B, S, H, D]")
-    o = _out(q, out_dtype, out)
-    with torch.cuda.device(q.device):
-        check(lib().paged_attention_prefill_wmma_scaled(
-            C.byref(view(o)), C.byref(view(q)), C.byref(view(k_cache)), C.byref(view(v_cache)),
-            C.byref(view(block_tables)), C.byref(view(context_lens)), float(scale), float(k_scale),
-            float(v_scale), _stream(q.device)))
-    return o
+    return _prefill(q, k_cache, v_cache, block_tables, context_lens, None, 0, scale, out_dtype, out, k_scale, v_scale,
+                    False)
 
 
 def paged_attention_prefill_varlen(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q,
@@ -137,16 +154,8 @@ def paged_attention_prefill_varlen(q, k_cache, v_cache, block_tables, context_le
     sequence b's q_len_b = cu_seqlens_q[b+1] - cu_seqlens_q[b] new tokens at
     rows cu_seqlens_q[b] .., positions context_lens[b] - q_len_b + r (causal).
     k_scale / v_scale dequantise a scaled cache (paged_attention_prefill_varlen_scaled)."""
-    q, k_cache, v_cache, block_tables, context_lens = _prep(
-        q, k_cache, v_cache, block_tables, context_lens, 3, "[T, H, D]")
-    cu = cu_seqlens_q.to(q.device, torch.int32).contiguous()
-    o = _out(q, out_dtype, out)
-    with torch.cuda.device(q.device):
-        check(lib().paged_attention_prefill_varlen_scaled(
-            C.byref(view(o)), C.byref(view(q)), C.byref(view(k_cache)), C.byref(view(v_cache)),
-            C.byref(view(block_tables)), C.byref(view(context_lens)), C.byref(view(cu)), int(max_q_len),
-            float(scale), float(k_scale), float(v_scale), _stream(q.device)))
-    return o
+    return _prefill(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, max_q_len, scale, out_dtype, out,
+                    k_scale, v_scale, False)
 
 
 def workspace_size(q, k_cache, block_tables, num_splits) -> int:

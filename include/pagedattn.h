@@ -264,6 +264,31 @@ int paged_attention_prefill_varlen_scaled(pa_tensor_t* out, const pa_tensor_t* q
                                           int64_t max_q_len, double scale, double k_scale, double v_scale,
                                           void* stream);
 
+/* The prefill entry points above with scratch for a context split: where a
+ * call's blocks of query rows leave most of the GPU idle (a few short chunks
+ * behind long contexts), each block's keys are cut into partitions of whole
+ * key tiles, computed by work-groups of their own and merged by a second
+ * launch (log-sum-exp rule).  cu_seqlens_q NULL: a uniform batch, q
+ * [B, S, H, D] (max_q_len unused), as paged_attention_prefill_wmma_scaled, or
+ * with fp32_precision as paged_attention_prefill (k_scale = v_scale = 1);
+ * otherwise a packed batch as paged_attention_prefill_varlen_scaled (its
+ * one-row sequences split as paged_attention_v3 plans it).
+ * workspace must be device memory of at least
+ * paged_attention_prefill_workspace_size(...) bytes, 256-byte aligned (NULL
+ * allowed when that is 0).  The reference's prefill has no split
+ * (kernels/paged_attn_prefill.cu:122-175). */
+int paged_attention_prefill_split(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k_cache,
+                                  const pa_tensor_t* v_cache, const pa_tensor_t* block_tables,
+                                  const pa_tensor_t* context_lens, const pa_tensor_t* cu_seqlens_q,
+                                  int64_t max_q_len, double scale, double k_scale, double v_scale,
+                                  int fp32_precision, void* workspace, size_t workspace_bytes, void* stream);
+
+/* Workspace bytes paged_attention_prefill_split needs for q [B, S, H, D], or
+ * q [T, H, D] and max_q_len, on the current device (0: no split is planned).
+ * Returns (size_t)-1 on invalid arguments. */
+size_t paged_attention_prefill_workspace_size(const pa_tensor_t* q, const pa_tensor_t* k_cache,
+                                              const pa_tensor_t* block_tables, int64_t max_q_len);
+
 /* KV-cache write ("reshape and cache"): token t's K and V rows, key[t] and
  * value[t] ([T, HKV, D], any non-negative token/head strides, 16-byte aligned
  * rows), go to block slot_mapping[t] / BS, row slot_mapping[t] % BS of

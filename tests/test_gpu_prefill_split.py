@@ -1,0 +1,91 @@
+"""Context split of the prefill (paged_attention_prefill_split, which the
+Python functions and the torch operators call): partitions of whole key tiles
+merged by a second launch, against the CPU oracle, at contexts around the
+partition and tile edges, in the 16-bit-weight, variable-length and
+fp32-precision kernels; poisoned and padded rows; the workspace checks."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from _helpers import close, to_dev, to_host
+from test_gpu_prefill import dev_args, prefill_case, want_of
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+@pytest.mark.parametrize("kv,qt", [("f16", "f32"), ("bf16", "bf16")])
+@pytest.mark.parametrize("entry", ["paged_attention_prefill_wmma", "paged_attention_prefill"])
+def test_prefill_split(pa, dev, D, kv, qt, entry):
+    """Contexts of one partition, of its edges and of many; a chunk longer than
+    its context (rows before it) and an empty one, in one batch."""
+    for S, BS, ctx in ((70, 16, [1537, 1024, 1023, 300, 64, 40, 0]), (65, 5, [2500])):
+        print("split", D, kv, entry, S, flush=True)
+        inp = prefill_case(len(ctx), S, 2, 1, D, BS, ctx, seed=D + S, kv=kv, qt=qt)
+        got = to_host(getattr(pa, entry)(*dev_args(inp, dev), 0.2))
+        assert "prefill_reduce_kernel" in pa.last_launch(), pa.last_launch()
+        close(got, want_of(inp, 0.2))
+
+
+def test_prefill_split_fp8_and_poison(pa, dev):
+    """An invalid block id reaches the rows that read its page whichever
+    partition holds it; a context beyond the table poisons its sequence."""
+    from test_gpu_prefill import _fp8, fp8_prefill_case
+    B, S, H, D, ctx = 3, 40, 2, 64, [2000, 1500, 1990]
+    inp, k8, v8, kf, vf = fp8_prefill_case(B, S, H, 2, D, 16, ctx, seed=4, qt="bf16", k_scale=0.05, v_scale=0.02)
+    bt, c = inp["bt"].copy(), inp["ctx"].copy()
+    bt[1, 92] = -3   # keys 1472..1487: rows from 1472 - 1460 on
+    bt[2, 0] = 10 ** 6
+    c[0] = bt.shape[1] * 16 + 1
+    print("split fp8 poison", flush=True)
+    got = to_host(pa.paged_attention_prefill_wmma(
+        to_dev(inp["q"], "bf16", dev), _fp8(k8, dev), _fp8(v8, dev), torch.from_numpy(bt).to(dev),
+        torch.from_numpy(c).to(dev), 0.125, k_scale=0.05, v_scale=0.02))
+    assert "prefill_reduce_kernel" in pa.last_launch(), pa.last_launch()
+    want = oracle.prefill(inp["q_f32"], kf, vf, inp["bt"], inp["ctx"], 0.125, "f32")
+    assert np.isnan(got[0]).all() and np.isnan(got[2]).all() and np.isnan(got[1, 12:]).all()
+    close(got[1, :12], want[1, :12])
+
+
+def test_varlen_split(pa, dev):
+    G, HKV, D = 3, 2, 64
+    lens, ctx = [13, 1, 0, 26, 70, 1], [1300, 30, 9, 2400, 900, 2000]
+    inp = oracle.paged_inputs(len(lens), 1, HKV, D, 16, ctx, seed=8, kv_dtype="bf16")
+    q = np.random.default_rng(8).standard_normal((sum(lens), G * HKV, D), dtype=np.float32)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    print("split varlen", flush=True)
+    got = to_host(pa.paged_attention_prefill_varlen(
+        to_dev(q, "f32", dev), to_dev(inp["k"], "bf16", dev), to_dev(inp["v"], "bf16", dev),
+        torch.from_numpy(inp["bt"]).to(dev), torch.from_numpy(inp["ctx"]).to(dev), torch.from_numpy(cu).to(dev),
+        70, 0.125))
+    # The one-row sequences split too: decode partitions, their merge, prefill partitions, theirs.
+    assert "; pa::reduce_kernel<64>; " in pa.last_launch() and "prefill_reduce_kernel" in pa.last_launch()
+    for b, n in enumerate(lens):
+        if n:
+            want = oracle.prefill(q[None, cu[b]:cu[b + 1]], inp["k"], inp["v"], inp["bt"][b:b + 1], inp["ctx"][b:b + 1],
+                                  0.125, "bf16")[0]
+            close(got[cu[b]:cu[b + 1]], want)
+
+
+def test_prefill_split_workspace_checks(pa, dev):
+    """A missing or short workspace is refused before any launch; without a
+    split the size is 0 and none is needed."""
+    L = pa.lib()
+    inp = prefill_case(1, 70, 2, 1, 64, 16, [2048], seed=1, kv="f16", qt="f16")
+    q, k, v, bt, c = dev_args(inp, dev)
+    out = torch.full(q.shape, 7.0, device=dev)
+    V = [pa.view(t) for t in (out, q, k, v, bt, c)]
+    need = L.paged_attention_prefill_workspace_size(C.byref(V[1]), C.byref(V[2]), C.byref(V[4]), 0)
+    assert need > 0 and need % 16 == 0
+    for ws, n in ((None, 0), (torch.empty(need, dtype=torch.uint8, device=dev), need - 1)):
+        rc = L.paged_attention_prefill_split(*[C.byref(x) for x in V], None, 0, 0.125, 1.0, 1.0, 0,
+                                             ws.data_ptr() if ws is not None else None, n, None)
+        assert rc == 3, rc
+    torch.cuda.synchronize()
+    assert bool((out == 7.0).all())
+    short = prefill_case(1, 70, 2, 1, 64, 16, [100], seed=1, kv="f16", qt="f16")
+    v3 = [pa.view(t) for t in dev_args(short, dev)]
+    assert L.paged_attention_prefill_workspace_size(C.byref(v3[0]), C.byref(v3[1]), C.byref(v3[3]), 0) == 0
