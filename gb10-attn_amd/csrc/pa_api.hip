@@ -499,15 +499,24 @@ PrefillParams prefill_params(const DecodeArgs& a, const int32_t* cu, int64_t T, 
   return pp;
 }
 
-// The matrix-core kernel serves paged_attention_prefill over 16-bit and FP8
-// caches for chunks of at least kPrefill32Rows rows; fp32 and fp64 caches,
-// shorter chunks and a q that is not 16-byte aligned run as a decode problem
-// per query row.  Contexts 64-4096, matrix kernel against decode kernel: at 64
-// rows 14.3 vs 15.0 us (one sequence of 12 heads, context 512), 15.2 vs 75.9
-// (eight sequences); at 16 rows 13.4 vs 11.1 and 14.4 vs 24.9.
-constexpr int kPrefill32Rows = 64;
+// Whether the matrix-core kernel serves a paged_attention_prefill call (16-bit
+// and FP8 caches, a 16-byte aligned q); else it runs as a decode problem per
+// query row.  It does when its context split is planned, when those decode
+// problems are kPrefill32Units work-groups or more, and for several rows of
+// groups of eight heads (whose decode problems run on the vector ALU).
+// Measured, decode kernel against matrix kernel, fp32 q: 12 heads of 64, one
+// row at context 4096 (split) 36.8 vs 14.9 us, at 512 8.7 vs 13.1; eight
+// sequences of 4 / 8 / 16 rows at 512 (384 / 768 / 1536 units) 14.2 vs 14.4,
+// 20.2 vs 14.4, 25.0 vs 14.6; 32/8 heads of 128, eight sequences of 8 / 16
+// rows (512 / 1024 units) 21.7 vs 22.0, 39.2 vs 23.5; 8/1 heads, two rows at
+// 64 / 512: 13.3 vs 10.5, 29.2 vs 20.3.
+constexpr int64_t kPrefill32Units = 768;
 bool prefill32_eligible(const DecodeArgs& a, const pa_tensor_t* q) {
-  return prefill_kv(a.kv_dtype) && a.p.Sq >= kPrefill32Rows && aligned16(q->data);
+  return prefill_kv(a.kv_dtype) && aligned16(q->data);
+}
+bool prefill32_pays(const DecodeArgs& a, const PrefillParams& pp) {
+  return pp.parts > 1 || (a.gc >= 8 && a.p.Sq > 1) ||
+         (int64_t)a.p.B * a.p.Sq * a.p.HKV * a.p.head_chunks >= kPrefill32Units;
 }
 
 // One direct decode launch (one partition per sequence): v1, v2 and the
@@ -523,7 +532,8 @@ int run_direct(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, con
   if (prefill && prefill32_eligible(a, q)) {
     PrefillParams pp = prefill_params(a, nullptr, 0, scale);
     if ((rc = bind_split(pp, false, ws))) return rc;
-    return hip_status(launch_prefill32(pp, a.kv_dtype, static_cast<hipStream_t>(stream)), "prefill kernel launch");
+    if (prefill32_pays(a, pp))
+      return hip_status(launch_prefill32(pp, a.kv_dtype, static_cast<hipStream_t>(stream)), "prefill kernel launch");
   }
   a.p.parts = 1;
   a.p.part_tokens = 0;

@@ -76,8 +76,8 @@ def test_prefill32(pa, dev, kv, qt, D):
     """Edges of the 32/64/128-row blocks and 32/64-key tiles; chunked, padded
     and empty sequences; both grid modes; page sizes that do not divide a tile."""
     for i, (B, S, H, HKV, BS, ctx, scale) in enumerate([
-            (3, 64, 4, 2, 16, [64, 160, 20], 1 / np.sqrt(D)), (2, 65, 2, 1, 5, [129, 64], -0.2),
-            (1, 129, 2, 2, 32, [129], 0.3), (2, 97, 2, 1, 16, [127, 0], 0.0)]):
+            (3, 64, 8, 4, 16, [64, 160, 20], 1 / np.sqrt(D)), (2, 65, 6, 6, 5, [129, 64], -0.2),
+            (1, 129, 6, 6, 32, [129], 0.3), (2, 97, 8, 4, 16, [127, 0], 0.0), (2, 3, 16, 2, 16, [63, 31], 0.1)]):
         print(f"prefill32 {kv} {qt} D={D} case {i}", flush=True)
         q, k, v, bt, c, k32, v32 = case(B, S, H, HKV, D, BS, ctx, kv, qt, D + i)
         got = run(pa, dev, q, k, v, bt, c, scale)
@@ -100,7 +100,7 @@ def test_prefill32_plain_mode(pa, dev, kv):
 def test_prefill32_q_range(pa, dev):
     """Rows of very large and very small q (the fp16 pieces are scaled by row)
     and rows that mix both; output types."""
-    q, k, v, bt, c, k32, v32 = case(1, 72, 2, 2, 64, 16, [100], "f16", "f32", 9)
+    q, k, v, bt, c, k32, v32 = case(1, 72, 12, 12, 64, 16, [100], "f16", "f32", 9)
     q[0, :10] *= 1e-30
     q[0, 10:20] *= 300.0
     q[0, 20:30, :, ::2] *= 1e-5
@@ -118,7 +118,7 @@ def test_prefill32_non_finite(pa, dev, kv):
     """Inf and NaN reach exactly the rows that attend them (a masked key's V is
     not multiplied into earlier rows), with the value a chain of fp32 products
     gives; an invalid block id poisons the rows that read its page."""
-    B, S, H, D, BS, ctx = 1, 100, 2, 64, 16, [150]
+    B, S, H, D, BS, ctx = 1, 100, 8, 64, 16, [150]
     q, k, v, bt, c, k32, v32 = case(B, S, H, H, D, BS, ctx, kv, "f32", 21)
 
     def put(x, x32, key, head, dim, val):
