@@ -45,8 +45,6 @@ hipError_t launch_decode_f32(const DecodeParams& p, int gc, hipStream_t stream);
 hipError_t launch_decode_f64(const DecodeParams& p, int gc, hipStream_t stream);
 hipError_t launch_decode_fp8(const DecodeParams& p, int gc, hipStream_t stream);
 
-thread_local int t_decode_fused = 0;
-
 hipError_t launch_decode(const DecodeParams& p, int kv_dtype, int gc, hipStream_t stream) {
   switch (kv_dtype) {
     case kF16: return launch_decode_f16(p, gc, stream);
@@ -316,6 +314,7 @@ int check_args(const pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* 
 }
 
 struct Plan {
+  bool explicit_parts;  // the caller's partitions (num_splits of ceil(ctx / num_splits) tokens)
   int64_t parts;
   int64_t part_tokens;  // 0 = reference count mode
   bool direct;
@@ -341,12 +340,14 @@ int make_plan(const DecodeParams& p, int gc, int kv_bytes, int64_t num_splits, P
   (void)gc;
   if (num_splits > 0) {
     if (num_splits > (1 << 20)) return fail(PA_ERR_INVALID_ARGUMENT, "num_splits too large");
+    plan->explicit_parts = true;
     plan->parts = num_splits;
     plan->part_tokens = 0;
     plan->direct = num_splits == 1;
     plan->hp = 0;
     return PA_OK;
   }
+  plan->explicit_parts = false;
   int cus = 0;
   int rc = device_cu_count(&cus);
   if (rc) return rc;
@@ -404,6 +405,40 @@ int plan_varlen_decode(const DecodeParams& p, int gc, int kv_bytes, Plan* plan) 
     plan->part_tokens = 0;
     plan->direct = true;
   }
+  return PA_OK;
+}
+
+// A call that only wants the merged output may compute it over any partitions
+// (the merge rule makes them one softmax).  From 16 partitions on (the
+// reference's chooser asks for 16 to 64 at 512 tokens and more; one query head
+// per KV head from 8, with rows of 1 KB from 4) it runs the library's own plan,
+// with no more partitions than the caller's count, whose workspace has been
+// checked.  64 partitions asked for, fp16
+// cache, 12 heads of 64: one sequence of 2048 tokens 16.4 -> 10.7 us, 16 of
+// them 26.1 -> 24.6 (the partition grids each paid a start-up per 32 tokens);
+// bf16, 32/8 heads of 128, 32 of 2048: 67.4 -> 57.8; 64/8 heads, 32 of 4096:
+// 177 -> 110 (the explicit partitions kept it off the matrix-core kernel).
+// The library's plan ran no slower at any of 25 batch and context sizes of
+// six head counts, but for 7 within 15 % where its own plan is not the best.
+bool own_plan_pays(const DecodeArgs& a, int64_t num_splits) {
+  const int64_t from = a.gc > 1 ? 16 : a.p.D * dtype_bytes(a.kv_dtype) < 1024 ? 8 : 4;
+  return num_splits >= from;
+}
+int own_plan(const DecodeArgs& a, int64_t num_splits, Plan* plan) {
+  Plan own;
+  int rc;
+  if ((rc = make_plan(a.p, a.gc, dtype_bytes(a.kv_dtype), 0, &own))) return rc;
+  if (own.parts > num_splits) {  // as many whole 128-token steps as keep within num_splits
+    const int64_t maxctx = (int64_t)a.p.MB * a.p.BS;
+    own.part_tokens = ((maxctx + num_splits - 1) / num_splits + 127) / 128 * 128;
+    own.parts = (maxctx + own.part_tokens - 1) / own.part_tokens;
+    if (own.parts <= 1) {
+      own.parts = 1;
+      own.part_tokens = 0;
+      own.direct = true;
+    }
+  }
+  *plan = own;
   return PA_OK;
 }
 
@@ -595,34 +630,15 @@ int run_v3(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const p
     return fail(PA_ERR_WORKSPACE, "workspace too small: need %zu bytes, got %zu", need, ws ? ws_bytes : 0);
   if (need > 0 && (reinterpret_cast<uintptr_t>(ws) & 255) != 0)
     return fail(PA_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+  if (phases == kBoth && own_plan_pays(a, num_splits) && (rc = own_plan(a, num_splits, &plan))) return rc;
   a.p.parts = (int)plan.parts;
   a.p.part_tokens = (int)plan.part_tokens;
   a.p.direct = plan.direct ? 1 : 0;
-  // Explicit splits into short chunks (the reference's own count at long
-  // contexts: 64 splits of 32 tokens at ctx 2048) run with a partition per
-  // wave or per token slot, each written as its own partials.  A call that
-  // wants the output too, over groups of one query head per KV head chunk,
-  // fuses when decode_fuse_rounds() allows it and one work-group per (row,
-  // head) at the narrowest packing still fills the GPU: that work-group
-  // serves every partition of its unit in rounds, merges each partition's
-  // partials into the output in registers (they are not written), and the
-  // reduce launch is skipped (config 2 at 64 splits: partition kernel +
-  // reduce 79.0 us per call, fused 65.6 us).
+  // Explicit splits into short chunks that write partials (pa_v3_partition,
+  // few partitions) run with a partition per wave or per token slot.
   const int64_t maxctx = (int64_t)a.p.MB * a.p.BS;
-  a.p.wave_parts = num_splits > 0 && !plan.direct && (maxctx + plan.parts - 1) / plan.parts <= kWavePartTokens;
+  a.p.wave_parts = plan.explicit_parts && !plan.direct && (maxctx + plan.parts - 1) / plan.parts <= kWavePartTokens;
   a.p.hp = plan.hp;
-  a.p.fuse_final = 0;
-  if (a.p.wave_parts && phases == kBoth && a.gc == 1) {
-    int cus = 0;
-    if ((rc = device_cu_count(&cus))) return rc;
-    const int kvb = dtype_bytes(a.kv_dtype);
-    const int hp = pack_for(a.p, kvb, 1, cus);
-    if ((int64_t)a.p.B * a.p.Sq * (a.p.HKV / hp) * a.p.head_chunks >= cus &&
-        decode_fuse_rounds(plan.parts, a.p.MB, a.p.BS, decode_tpi(a.p.D, hp, kvb)) > 0) {
-      a.p.fuse_final = 1;
-      a.p.hp = hp;
-    }
-  }
   if (a.p.hp == 0) {
     int cus = 0;
     if ((rc = device_cu_count(&cus))) return rc;
@@ -634,15 +650,14 @@ int run_v3(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const p
   // repay): config 3's ragged batch at 8 splits (partitions up to 4096
   // tokens) 5.33 -> 6.17 TB/s; at 64 splits (up to 512) -2 %, and config 2's
   // uniform batch at 8 or 64 splits -3.7 %, hence the bound.
-  a.p.seq_order = num_splits > 0 && !plan.direct && a.p.B <= 64 && a.p.Sq == 1 &&
+  a.p.seq_order = plan.explicit_parts && !plan.direct && a.p.B <= 64 && a.p.Sq == 1 &&
                   (maxctx + plan.parts - 1) / plan.parts >= kLongestFirstTokens ? 1 : 0;
   if (!plan.direct) bind_workspace(&a.p, ws, plan);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  t_decode_fused = 0;
   if (phases & kPartition) {
     if ((rc = hip_status(launch_decode(a.p, a.kv_dtype, a.gc, s), "partition kernel launch"))) return rc;
   }
-  if ((phases & kReduce) && !plan.direct && !t_decode_fused) {
+  if ((phases & kReduce) && !plan.direct) {
     const ReduceParams r = reduce_params(a.p);
     if ((rc = hip_status(launch_reduce(r, s), "reduce kernel launch"))) return rc;
   }

@@ -201,14 +201,13 @@ void decode_kernel(const DecodeParams p) {
   // Short explicit partitions (one is a few wave tiles, and a work-group per
   // partition would pay its start-up for each).  Wave-partition mode:
   // work-group `grp` serves partitions grp * NW + w, one per wave w.
-  // Slot-partition mode: it serves `rounds` rounds of NW * TPI partitions,
-  // round r's grp * gparts + r * NW * TPI + w * TPI + s for token slot s of
-  // wave w: a slot's lanes stream their own partition's tokens, so the
-  // wave's slot streams are the partials themselves, with no cross-slot
+  // Slot-partition mode: partitions grp * NW * TPI + w * TPI + s for token
+  // slot s of wave w: a slot's lanes stream their own partition's tokens, so
+  // the wave's slot streams are the partials themselves, with no cross-slot
   // combine per partition.
   const bool wpm = p.wave_parts == kWavePart;
   const bool spm = p.wave_parts == kSlotPart;
-  const int gparts = spm ? NW * TPI * p.rounds : wpm ? NW : 1;  // partitions per work-group
+  const int gparts = spm ? NW * TPI : wpm ? NW : 1;  // partitions per work-group
   const int ngrp = (p.parts + gparts - 1) / gparts;
   int part, z, grp = 0;  // part: per lane in the slot-partition mode
   if (compact_grid(p)) {
@@ -266,9 +265,7 @@ void decode_kernel(const DecodeParams p) {
   const bool fixed = p.part_tokens > 0;
   const bool ok = ctx > 0 && ctx_b <= maxctx;
   const int nparts = fixed ? (ok ? (ctx + p.part_tokens - 1) / p.part_tokens : 0) : p.parts;
-  // (fuse_final: a slot-partition work-group that covers every partition of
-  // its unit, GC == 1, also merges them and writes the output.)
-  const bool final_here = p.direct || (fixed && nparts <= 1) || p.fuse_final;
+  const bool final_here = p.direct || (fixed && nparts <= 1);
 
   if (!ok) {
     // Zero rows for an empty context, NaN rows for one longer than the table.
@@ -725,11 +722,9 @@ void decode_kernel(const DecodeParams p) {
   if (spm) {
     // The work-group's block-table entries in one staged chunk (the host
     // enables the mode only when they fit).  Each slot streams its own
-    // partition of each round, NI consecutive tokens per tile (a token past
-    // its end reads the masked safe row); the tile count is the chunk's,
-    // wave-uniform, rounded up to even.  The two-tile pipeline runs on
-    // across rounds: a round's first tile is issued before the previous
-    // round's last is consumed.
+    // partition, NI consecutive tokens per tile (a token past its end reads
+    // the masked safe row); the tile count is the chunk's, wave-uniform,
+    // rounded up to even.
     const int cp = T0 < T1 ? (int)fastdiv((uint32_t)T0, p.bs_div) : 0;
     if (T0 < T1) {
       const int np = (int)fastdiv((uint32_t)(T1 - 1), p.bs_div) + 1 - cp;
@@ -741,30 +736,17 @@ void decode_kernel(const DecodeParams p) {
       }
       __syncthreads();
     }
-    const int R = p.rounds;
-    const int nt = ((chunk + NI - 1) / NI + 1) & ~1;  // tiles per round (even)
-    // Fused output (GC == 1): each slot's partitions merged as they complete
-    // (log-sum-exp rule), then the wave's slots and the waves as below.  A
-    // bad block id poisons its own partition's partial and the output.
-    float mT = kNegBig, lT = 0.0f, aT[VEC];
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) aT[e] = 0.0f;
-    int bad_all = 0;
-    int cr = 0;  // round being consumed
+    const int nt = ((chunk + NI - 1) / NI + 1) & ~1;  // tiles (even)
     auto finish = [&]() __attribute__((always_inline)) {
       rebase();
       // This slot's partition: its partials from its lanes (dims dsub * VEC
-      // .. of head hl), m and l from those of dsub 0.  The fused form keeps
-      // them in registers only: the workspace is the split's scratch, and
-      // the partials' writes (3 % of the bytes, 4-byte m and l stores among
-      // them) took config 2 at 64 splits from 0.77 to 0.68 of 8 TB/s.
-      const int pr = part + cr * NW * TPI;
-      if (pr < nparts && !p.fuse_final) {
+      // .. of head hl), m and l from those of dsub 0.
+      if (part < nparts) {
 #pragma unroll
         for (int g = 0; g < GC; ++g) {
           if (g0 + g >= p.G) continue;
           const int h = (kvh * HP + hl) * p.G + g0 + g;
-          const int64_t pidx = ((int64_t)b * p.H + h) * p.parts + pr;
+          const int64_t pidx = ((int64_t)b * p.H + h) * p.parts + part;
 #pragma unroll
           for (int e = 0; e < VEC; ++e) p.ws_acc[pidx * D + dsub * VEC + e] = acc[g][e] * p.vscale;
           if (dsub == 0) {
@@ -773,79 +755,35 @@ void decode_kernel(const DecodeParams p) {
           }
         }
       }
-      if constexpr (GC == 1) {
-        if (p.fuse_final) {
-          const float mn = fmaxf(mT, m[0]);
-          const float ca = fast_exp2(mT - mn), cb = fast_exp2(m[0] - mn);
-          lT = lT * ca + l[0] * cb;
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) aT[e] = aT[e] * ca + acc[0][e] * cb;
-          mT = mn;
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < GC; ++g) {
-        m[g] = kNegBig;
-        mx[g] = kNegBig;
-        l[g] = 0.0f;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) acc[g][e] = 0.0f;
-      }
-      m_own = kNegBig;
-      mx_own = kNegBig;
-      l_own = 0.0f;
-      bad_all |= bad;
-      bad = 0;
-      ++cr;
     };
     if (T0 < T1) {
-      // Issue position (round ir, token offset iu); past the last round a
-      // tile reads the masked safe row of the last round's partition.  Each
-      // tile carries the bad flag of its own loads, taken at consume time.
-      int ir = 0, iu = 0;
+      // Tile at token offset u of the partition; each tile carries the bad
+      // flag of its own loads, taken at consume time.  (Past the end a tile
+      // reads the masked safe row.)
+      const int r0 = min(part * chunk, ctx), r1 = min(r0 + chunk, ctx);
+      int u = 0;
       auto iss = [&](Tile& T, int& tb) __attribute__((always_inline)) {
-        const int pr = part + min(ir, R - 1) * NW * TPI;
-        const int r0 = min(pr * chunk, ctx), r1 = min(r0 + chunk, ctx);
-        const int u = ir < R ? iu : chunk;
         const int keep = bad;
         bad = 0;
         issue_at([&](int i) { return r0 + u + i; }, cp, r1, T);
         tb = bad;
         bad = keep;
-        iu += NI;
-        if (iu >= nt * NI) {
-          iu = 0;
-          ++ir;
-        }
+        u += NI;
       };
-      const int ntot = nt * R;
       Tile A, B;
-      int ba, bb, cu = 0;
+      int ba, bb;
       iss(A, ba);
-      for (int j = 0; j < ntot; j += 2) {
+      for (int j = 0; j < nt; j += 2) {
         iss(B, bb);
         bad |= ba;
         consume(A);
         iss(A, ba);
         bad |= bb;
         consume(B);
-        cu += 2;
-        if (cu == nt) {
-          finish();
-          cu = 0;
-        }
       }
-    } else {
-      for (int r = 0; r < R; ++r) finish();  // empty partitions: m = -3e38, l = 0
     }
-    bad = bad_all;
-    if constexpr (GC != 1) return;
-    if (!p.fuse_final) return;  // work-group uniform
-    m[0] = mT;
-    mx[0] = mT;
-    l[0] = lT;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) acc[0][e] = aT[e];
+    finish();  // (an empty partition: m = -3e38, l = 0)
+    return;
   } else {
     const bool fast = (p.BS % TPI) == 0 && (t0 % TPI) == 0;
     if (T0 < T1) {
@@ -1009,25 +947,16 @@ hipError_t launch_decode_one(const DecodeParams& p, int64_t blocks, hipStream_t 
 template <typename KV, int D, int GC, int HP = 1>
 hipError_t launch_decode_dg(const DecodeParams& p0, hipStream_t stream) {
   DecodeParams p = p0;
-  // Short explicit partitions.  A call whose host plan fuses
-  // (decode_fuse_rounds(), GC == 1) takes the slot-partition mode in rounds:
-  // one work-group per unit.  Otherwise one partition per token slot when
-  // every slot of a work-group has one (parts >= kDecodeWaves * TPI) and the
+  // Short explicit partitions: one partition per token slot when every slot
+  // of a work-group has one (parts >= kDecodeWaves * TPI) and the
   // work-group's pages fit one staged block-table chunk; else one per wave.
   constexpr int TPI = DecodeShapeOf<KV, D, GC, HP>::TPI;
-  const int fr = GC == 1 && p.fuse_final && p.wave_parts ? decode_fuse_rounds(p.parts, p.MB, p.BS, TPI) : 0;
-  p.fuse_final = fr > 0 ? 1 : 0;
-  p.rounds = 1;
-  if (fr > 0) {
-    p.wave_parts = kSlotPart;
-    p.rounds = fr;
-    t_decode_fused = 1;
-  } else if (p.wave_parts) {
+  if (p.wave_parts) {
     const int64_t chunk_max = ((int64_t)p.MB * p.BS + p.parts - 1) / p.parts;
     const int64_t pages = ((int64_t)kDecodeWaves * TPI * chunk_max + p.BS - 1) / p.BS + 1;
     p.wave_parts = p.parts >= kDecodeWaves * TPI && pages <= kBtChunk ? kSlotPart : kWavePart;
   }
-  const int64_t gparts = p.wave_parts == kSlotPart ? (int64_t)kDecodeWaves * TPI * p.rounds
+  const int64_t gparts = p.wave_parts == kSlotPart ? (int64_t)kDecodeWaves * TPI
                                                    : p.wave_parts ? kDecodeWaves : 1;
   const int64_t groups = (p.parts + gparts - 1) / gparts;
   const int64_t blocks = (int64_t)p.B * p.Sq * (p.HKV / HP) * p.head_chunks * groups;
