@@ -39,6 +39,8 @@ void note_launch(const char* fmt, ...) {
   g_launches += buf;
 }
 
+bool decode_mfma_f16(const DecodeParams& p, int gc);
+bool decode_mfma_bf16(const DecodeParams& p, int gc);
 hipError_t launch_decode_f16(const DecodeParams& p, int gc, hipStream_t stream);
 hipError_t launch_decode_bf16(const DecodeParams& p, int gc, hipStream_t stream);
 hipError_t launch_decode_f32(const DecodeParams& p, int gc, hipStream_t stream);
@@ -54,6 +56,10 @@ hipError_t launch_decode(const DecodeParams& p, int kv_dtype, int gc, hipStream_
     case kFP8: return launch_decode_fp8(p, gc, stream);
     default: return hipErrorInvalidValue;
   }
+}
+// Whether the matrix-core decode kernel serves the call.
+bool decode_on_matrix_cores(const DecodeParams& p, int kv_dtype, int gc) {
+  return kv_dtype == kF16 ? decode_mfma_f16(p, gc) : kv_dtype == kBF16 && decode_mfma_bf16(p, gc);
 }
 }  // namespace pa
 
@@ -337,7 +343,6 @@ int pack_for(const DecodeParams& p, int kv_bytes, int64_t splits, int cus) {
 // workspace-size query runs without one); its packing is chosen at launch
 // (hp = 0 here).
 int make_plan(const DecodeParams& p, int gc, int kv_bytes, int64_t num_splits, Plan* plan) {
-  (void)gc;
   if (num_splits > 0) {
     if (num_splits > (1 << 20)) return fail(PA_ERR_INVALID_ARGUMENT, "num_splits too large");
     plan->explicit_parts = true;
@@ -385,6 +390,26 @@ int make_plan(const DecodeParams& p, int gc, int kv_bytes, int64_t num_splits, P
   plan->part_tokens = nparts > 1 ? ptok : 0;
   plan->direct = nparts <= 1;
   plan->hp = hp;
+  // A split whose heads can be packed takes as many partitions as bring the
+  // grid of the widest rows to four work-groups per CU, of at least 512 tokens
+  // (1024 of an FP8 cache): wide rows and an even end of the launch both pay
+  // more than the longer partial pass.  bf16, 32/8 heads of 128, contexts
+  // ragged over [256, 8192]: 32 sequences 105 -> 98 us, 16 58 -> 50; 64 equal
+  // contexts of 4096: 190 -> 181.  fp16, 16 heads of 128, 32
+  // sequences of 2048 / 4096: 100 -> 90, 188 -> 171.  Not where 512-token
+  // partitions leave that grid under two per CU (12 heads of 64, 16 sequences
+  // of 4096: 41.2 -> 43.1), nor at 256 tokens (FP8, 32/8 heads, 32 of 2048:
+  // 40.7 -> 42.9).
+  if (nparts > 1 && hi > lo) {
+    // (Sq is 1 here; the size query leaves it, and B may be, 0.)
+    const int64_t packed = std::max<int64_t>(1, (int64_t)p.B * (p.HKV / hi) * ((p.G + gc - 1) / gc));
+    const int64_t want = std::min((4 * (int64_t)cus + packed - 1) / packed, maxctx / (kv_bytes == 1 ? 1024 : 512));
+    if (want > nparts && packed * want >= 2 * (int64_t)cus) {
+      plan->part_tokens = ((maxctx + want - 1) / want + 127) / 128 * 128;
+      plan->parts = (maxctx + plan->part_tokens - 1) / plan->part_tokens;
+      if (packed * plan->parts >= (int64_t)cus * knobs().wgs_per_cu) plan->hp = hi;
+    }
+  }
   return PA_OK;
 }
 
@@ -592,6 +617,7 @@ ReduceParams reduce_params(const DecodeParams& p) {
   r.out_dtype = p.out_dtype;
   r.parts = p.parts;
   r.part_tokens = p.part_tokens;
+  r.uniform_whole = p.uniform_whole;
   r.cu_q = p.cu_q;
   r.q_total = p.q_total;
   return r;
@@ -653,6 +679,13 @@ int run_v3(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const p
   a.p.seq_order = plan.explicit_parts && !plan.direct && a.p.B <= 64 && a.p.Sq == 1 &&
                   (maxctx + plan.parts - 1) / plan.parts >= kLongestFirstTokens ? 1 : 0;
   if (!plan.direct) bind_workspace(&a.p, ws, plan);
+  // Partitions of the library's own plan on the matrix-core kernel: a batch of
+  // nearly equal contexts that fills the GPU uncut is not cut (part_len).
+  if (phases == kBoth && plan.part_tokens > 0 && a.p.B <= 64 && decode_on_matrix_cores(a.p, a.kv_dtype, a.gc)) {
+    int cus = 0;
+    if ((rc = device_cu_count(&cus))) return rc;
+    a.p.uniform_whole = (int64_t)a.p.B * a.p.HKV * a.p.head_chunks >= cus ? 1 : 0;
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (phases & kPartition) {
     if ((rc = hip_status(launch_decode(a.p, a.kv_dtype, a.gc, s), "partition kernel launch"))) return rc;

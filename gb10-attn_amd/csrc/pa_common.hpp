@@ -63,6 +63,7 @@ struct DecodeParams {
   int32_t pprio;        // 1: the whole grid is resident at once; waves lower their priority as they progress
   int32_t wave_parts;   // explicit splits into short chunks: 1 from the host (the launcher picks the
                         // mode: a partition per wave or per token slot); 0 otherwise
+  int32_t uniform_whole;  // part_len(): nearly equal contexts are not cut (B <= 64)
   int32_t seq_order;    // explicit split into long partitions, B <= 64, Sq = 1: sequences dispatched
                         // longest first
   FastDiv bs_div;
@@ -84,6 +85,7 @@ struct ReduceParams {
   int32_t out_dtype;
   int32_t parts;
   int32_t part_tokens;
+  int32_t uniform_whole;
   const int32_t* cu_q;  // variable-length batches: as DecodeParams
   int64_t q_total;
 };

@@ -45,20 +45,21 @@ namespace pa {
 __device__ inline bool compact_grid(const DecodeParams& p) {
   return p.part_tokens > 0 && p.Sq == 1 && p.B <= 64 && p.cu_q == nullptr;
 }
-// Unit `id` of the compacted numbering -> (z, part); false past the last one.
+// Unit `id` of the compacted numbering of partitions of ptok tokens -> (z,
+// part); false past the last one.
 // Whole partitions come first, sequence by sequence (a context out of range
 // is one unit: it writes its row), then each sequence's shorter last
 // partition, longest first: the dispatcher hands out work-groups in id
 // order, so the launch ends on its shortest units.  Config 3 (1044 units on
 // 512 slots, partitions of 13 to 2048 tokens) had ended with half the slots
 // idle for its last ~15 %.
-__device__ inline bool compact_unit(const DecodeParams& p, int id, int lane, int& z, int& part) {
+__device__ inline bool compact_unit(const DecodeParams& p, int ptok, int id, int lane, int& z, int& part) {
   const int maxctx = p.MB * p.BS;
   const int c = lane < p.B ? p.context_lens[lane] : 0;
   const bool valid = lane < p.B && c > 0 && c <= maxctx;
-  const int whole = valid ? c / p.part_tokens : 0;
+  const int whole = valid ? c / ptok : 0;
   const int nfull = lane < p.B ? (valid ? whole : 1) : 0;   // units of whole partitions
-  const int rem = valid ? c - whole * p.part_tokens : 0;     // tokens of the last partition if shorter (0: none)
+  const int rem = valid ? c - whole * ptok : 0;     // tokens of the last partition if shorter (0: none)
   int incl = nfull;  // inclusive prefix sum over sequences 0..lane
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -211,7 +212,7 @@ void decode_kernel(const DecodeParams p) {
   const int ngrp = (p.parts + gparts - 1) / gparts;
   int part, z, grp = 0;  // part: per lane in the slot-partition mode
   if (compact_grid(p)) {
-    if (!compact_unit(p, id, lane, z, part)) return;  // work-group uniform
+    if (!compact_unit(p, p.part_tokens, id, lane, z, part)) return;  // work-group uniform
   } else if (wpm || spm) {
     grp = id % ngrp;
     z = id / ngrp;

@@ -332,6 +332,28 @@ __device__ inline float group_sum(float v) {
   return v;
 }
 
+// Partition length of a batch of up to 64 sequences: part_tokens, or with
+// `whole` set (DecodeParams::uniform_whole) the whole context where the lengths
+// are nearly equal.  Such a batch needs no cut for balance, and each cut costs
+// its work-groups' start-up and a pass over the partials: 32 sequences of 8192
+// tokens, 64/8 heads of 128, bf16: 197 -> 188 us; ragged ones keep their partitions
+// (uncut 133 us against 107).  Wave-uniform; the same in every kernel of a call.
+__device__ inline int part_len(int part_tokens, int whole, const int32_t* context_lens, int B, int maxctx) {
+  if (!whole) return part_tokens;
+  const int lane = threadIdx.x & 63;
+  const int c = lane < B ? context_lens[lane] : 0;
+  const int v = c > 0 && c <= maxctx ? c : 0;
+  int mx = v;
+  float sum = (float)v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    mx = max(mx, __shfl_xor(mx, o, 64));
+    sum += __shfl_xor(sum, o, 64);
+  }
+  mx = __builtin_amdgcn_readfirstlane(mx);
+  return __builtin_amdgcn_readfirstlane(sum >= 0.9f * (float)mx * (float)B ? 1 : 0) ? max(maxctx, part_tokens) : part_tokens;
+}
+
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 }  // namespace pa

@@ -69,12 +69,13 @@ __global__ __launch_bounds__(64 * kReduceWaves) void reduce_kernel(const ReduceP
   }
 
   const int maxctx = p.MB * p.BS;
-  const bool fixed = p.part_tokens > 0;
+  const int ptok = part_len(p.part_tokens, p.uniform_whole, p.context_lens, p.B, maxctx);
+  const bool fixed = ptok > 0;
   const bool ok = ctx > 0 && ctx <= maxctx;
   int n;
   if (fixed) {
     if (!ok) return;  // the partition kernel wrote this row
-    n = (ctx + p.part_tokens - 1) / p.part_tokens;
+    n = (ctx + ptok - 1) / ptok;
     if (n <= 1) return;
   } else {
     if (!ok) {

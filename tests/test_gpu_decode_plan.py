@@ -1,0 +1,67 @@
+"""The library's own decode plan where it replaces or refines a call's split,
+against the CPU oracle: explicit counts from 16 partitions on (fewer planned,
+as many, and more than asked for), packed splits, and batches of nearly equal
+contexts on the matrix-core kernel, which are not cut."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from _helpers import close, decode_case, dev_inputs, oracle_decode_rows, to_host
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,H,HKV,D,ctx,S", [
+    (1, 8, 1, 64, [8192], 16),             # the plan wants more partitions: held to 16
+    (3, 8, 8, 128, [3000, 1, 0], 64),      # fewer than asked
+    (2, 12, 4, 32, [700, 5000], 17),       # odd group, ragged
+    (16, 16, 16, 64, [4096] * 16, 64),     # packed heads
+    (40, 8, 8, 32, [600] * 40, 8),         # uncut
+])
+@pytest.mark.parametrize("kv", ["f16", "bf16"])
+def test_explicit_count_on_own_plan(pa, dev, B, H, HKV, D, ctx, S, kv):
+    inp = decode_case(B, H, HKV, D, 16, ctx, seed=B + S, kv=kv, q=kv)
+    q, k, v, bt, c = dev_inputs(inp, dev)
+    print("own plan", B, H, HKV, D, S, kv, flush=True)
+    got = to_host(pa.paged_attention_v3(q, k, v, bt, c, 0.1, S))
+    close(got, oracle_decode_rows(inp["q_f32"], inp["k"], inp["v"], inp["bt"], inp["ctx"], 0.1, kv))
+    # The explicit split's workspace is still asked for.
+    need, V = pa.workspace_size(q, k, bt, S), pa.view
+    out = torch.empty((B, H, D), device=dev)
+    views = [V(t) for t in (out, q, k, v, bt, c)]
+    rc = pa.lib().paged_attention_v3(*[C.byref(x) for x in views], 0.1, S, None, 0, None)
+    assert need > 0 and rc == 3
+
+
+@pytest.mark.parametrize("kv", ["f16", "bf16"])
+@pytest.mark.parametrize("lens", ["equal", "nearly", "ragged", "empty and beyond"])
+def test_equal_contexts_uncut(pa, dev, kv, lens):
+    """A work-group per (sequence, KV head) or more fills the GPU, groups of
+    eight: equal contexts run whole, others in partitions, by the same call."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    HKV, G, D, B = 8, 8, 64, -(-cus // 8)
+    assert B <= 64
+    n = np.full(B, 3008)
+    if lens == "nearly":
+        n -= np.arange(B) % 300
+    elif lens == "ragged":
+        n = np.random.default_rng(1).integers(1, 3009, B)
+        n[3] = 3008
+    elif lens == "empty and beyond":
+        n[5], n[7] = 0, 17
+    inp = decode_case(B, HKV * G, HKV, D, 16, n.tolist(), seed=3, kv=kv, q=kv, mb=188)
+    q, k, v, bt, c = dev_inputs(inp, dev)
+    ctx = inp["ctx"].copy()
+    if lens == "empty and beyond":
+        ctx[7] = 188 * 16 + 1
+        c = torch.from_numpy(ctx).to(dev)
+    print("uncut", lens, kv, flush=True)
+    got = to_host(pa.paged_attention_v3(q, k, v, bt, c, 0.125, 0))
+    assert "decode_mfma_kernel" in pa.last_launch() and "reduce_kernel" in pa.last_launch(), pa.last_launch()
+    if lens == "empty and beyond":
+        assert np.all(got[5] == 0.0) and np.isnan(got[7]).all()
+        got[7] = 0.0
+        ctx[7] = 0
+    close(got, oracle_decode_rows(inp["q_f32"], inp["k"], inp["v"], inp["bt"], ctx, 0.125, kv))
