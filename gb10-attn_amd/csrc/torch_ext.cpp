@@ -22,6 +22,8 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
+#include <optional>
+
 #include "../../include/pagedattn.h"
 
 namespace {
@@ -128,20 +130,53 @@ Scratch scratch_of(const at::Tensor& q, size_t bytes) {
   return s;
 }
 
+// The prefill entry points into `out` (a new fp32 tensor when null).
 at::Tensor prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& bt,
                    const at::Tensor& ctx, const at::Tensor* cu, int64_t max_q_len, double scale, double k_scale,
-                   double v_scale, bool fp32) {
+                   double v_scale, bool fp32, const at::Tensor* given = nullptr) {
   Args a = cu ? prep(q, k, v, bt, ctx, 3, "[T, H, D]") : prep(q, k, v, bt, ctx, 4, "[B, S, H, D]");
   at::Tensor cuq;
   if (cu) cuq = cu->to(a.q.device(), at::kInt).contiguous();
   c10::DeviceGuard guard(a.q.device());
-  at::Tensor out = at::empty(a.q.sizes(), a.q.options().dtype(at::kFloat));
+  at::Tensor out = given ? *given : at::empty(a.q.sizes(), a.q.options().dtype(at::kFloat));
   pa_tensor_t o = view(out), qq = view(a.q), kk = view(a.k), vv = view(a.v), bb = view(a.bt), cc = view(a.ctx), uu;
   if (cu) uu = view(cuq);
   Scratch s = scratch_of(a.q, paged_attention_prefill_workspace_size(&qq, &kk, &bb, max_q_len));
   check(paged_attention_prefill_split(&o, &qq, &kk, &vv, &bb, &cc, cu ? &uu : nullptr, max_q_len, scale, k_scale,
                                       v_scale, fp32 ? 1 : 0, s.ptr, s.bytes, stream_of(a.q)));
   return out;
+}
+
+// The Python functions' calls (ops.py): into the caller's output of any served
+// type, with its workspace where it holds the split.
+void op_prefill_out(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& bt,
+                    const at::Tensor& ctx, const std::optional<at::Tensor>& cu, int64_t max_q_len, double scale,
+                    double k_scale, double v_scale, bool fp32, const at::Tensor& out) {
+  prefill(q, k, v, bt, ctx, cu.has_value() ? &*cu : nullptr, max_q_len, scale, k_scale, v_scale, fp32, &out);
+}
+
+void op_decode_out(int64_t version, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                   const at::Tensor& bt, const at::Tensor& ctx, double scale, int64_t num_splits, double k_scale,
+                   double v_scale, const at::Tensor& out, const std::optional<at::Tensor>& workspace) {
+  Args a = prep(q, k, v, bt, ctx, 3, "[B, H, D]");
+  c10::DeviceGuard guard(a.q.device());
+  pa_tensor_t o = view(out), qq = view(a.q), kk = view(a.k), vv = view(a.v), bb = view(a.bt), cc = view(a.ctx);
+  if (version < 3) {
+    check((version == 1 ? paged_attention : paged_attention_v2)(&o, &qq, &kk, &vv, &bb, &cc, scale, stream_of(a.q)));
+    return;
+  }
+  const size_t need = paged_attention_v3_workspace_size(&qq, &kk, &bb, num_splits);
+  TORCH_CHECK(need != (size_t)-1, pa_last_error());
+  const bool theirs = workspace.has_value() && (size_t)workspace->numel() >= need;
+  Scratch s;
+  if (theirs) {
+    s.ptr = workspace->data_ptr();
+    s.bytes = (size_t)workspace->numel();
+  } else {
+    s = scratch_of(a.q, need);
+  }
+  check(paged_attention_v3_scaled(&o, &qq, &kk, &vv, &bb, &cc, scale, k_scale, v_scale, num_splits, s.ptr, s.bytes,
+                                  stream_of(a.q)));
 }
 
 at::Tensor op_paged_attention_prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
@@ -223,6 +258,12 @@ void op_write_kv(at::Tensor& k_cache, at::Tensor& v_cache, const at::Tensor& key
   op_write_kv_scaled(k_cache, v_cache, key, value, slot_mapping, 1.0, 1.0);
 }
 
+void op_write_kv_into(const at::Tensor& k_cache, const at::Tensor& v_cache, const at::Tensor& key,
+                      const at::Tensor& value, const at::Tensor& slot_mapping, double k_scale, double v_scale) {
+  at::Tensor k = k_cache, v = v_cache;
+  op_write_kv_scaled(k, v, key, value, slot_mapping, k_scale, v_scale);
+}
+
 }  // namespace
 
 TORCH_LIBRARY(gb10_attn, m) {
@@ -235,6 +276,13 @@ TORCH_LIBRARY(gb10_attn, m) {
   m.def("paged_attention_v3_scaled(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
         "Tensor context_lens, float scale, int num_splits, float k_scale, float v_scale) -> Tensor",
         &op_paged_attention_v3_scaled);
+  m.def("decode_out(int version, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor context_lens, "
+        "float scale, int num_splits, float k_scale, float v_scale, Tensor(a!) out, Tensor? workspace) -> ()");
+  m.def("prefill_out(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor context_lens, "
+        "Tensor? cu_seqlens_q, int max_q_len, float scale, float k_scale, float v_scale, bool fp32, "
+        "Tensor(a!) out) -> ()");
+  m.def("write_kv_into(Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor key, Tensor value, Tensor slot_mapping, "
+        "float k_scale, float v_scale) -> ()");
   m.def("choose_num_splits(int num_seqs, int num_heads, int max_context) -> int", &op_choose_num_splits);
   m.def("paged_attention_prefill(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
         "Tensor context_lens, float scale) -> Tensor", &op_paged_attention_prefill);
@@ -254,4 +302,12 @@ TORCH_LIBRARY(gb10_attn, m) {
   m.def("write_kv_scaled(Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor key, Tensor value, Tensor slot_mapping, "
         "float k_scale, float v_scale) -> ()",
         &op_write_kv_scaled);
+}
+
+// The Python functions' operators have a GPU kernel only: under torch.compile
+// they end the graph, as the functions always have, and run eagerly.
+TORCH_LIBRARY_IMPL(gb10_attn, CUDA, m) {
+  m.impl("decode_out", &op_decode_out);
+  m.impl("prefill_out", &op_prefill_out);
+  m.impl("write_kv_into", &op_write_kv_into);
 }

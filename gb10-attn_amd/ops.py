@@ -15,8 +15,8 @@ views (e.g. one layer of a larger pool) without a copy.  Rows of a sequence
 with context_lens <= 0 are zeros; context_lens beyond the block table or
 out-of-range block ids give NaN rows (the reference reads out of bounds).
 
-PyTorch only supplies device memory and streams here; all arithmetic runs in
-the HIP kernels behind include/pagedattn.h.
+PyTorch only supplies device memory, streams and the native call layer here;
+all arithmetic runs in the HIP kernels behind include/pagedattn.h.
 """
 from __future__ import annotations
 
@@ -25,7 +25,7 @@ import ctypes as C
 import torch
 
 from ._lib import (DTYPE_BF16, DTYPE_F16, DTYPE_F32, DTYPE_F64, DTYPE_FP8, DTYPE_I32, DTYPE_I64,
-                   PaTensor, check, last_error, lib)
+                   LIB_PATH, PaTensor, check, last_error, lib)
 
 _DT = {
     torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16,
@@ -48,29 +48,11 @@ def _kv_ok(t: torch.Tensor) -> bool:
     return all((t.stride(i) * es) % 16 == 0 or t.shape[i] == 1 for i in range(3))
 
 
-def _prep(q, k_cache, v_cache, block_tables, context_lens, qdim, what):
+def _on_gpu(q, k_cache, v_cache):
     if not q.is_cuda:
         raise RuntimeError("q must be on CUDA")
     if not (k_cache.is_cuda and v_cache.is_cuda):
         raise RuntimeError("kv cache must be on CUDA")
-    if q.dim() != qdim:
-        raise RuntimeError(f"q must be {what}")
-    if k_cache.dim() != 4:
-        raise RuntimeError("k_cache must be [NB, BS, H, D]")
-    q = q.contiguous()
-    # Strided K/V views are read in place; anything the kernels cannot
-    # address directly is made contiguous, as the reference does for all inputs.
-    if not _kv_ok(k_cache):
-        k_cache = k_cache.contiguous()
-    if not _kv_ok(v_cache):
-        v_cache = v_cache.contiguous()
-    block_tables = block_tables.to(torch.int32).contiguous()
-    context_lens = context_lens.to(torch.int32).contiguous()
-    return q, k_cache, v_cache, block_tables, context_lens
-
-
-def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
 
 
 def _out(q, out_dtype, out):
@@ -79,58 +61,37 @@ def _out(q, out_dtype, out):
     return torch.empty(q.shape, dtype=out_dtype, device=q.device)
 
 
-def _call_simple(fn, q, k_cache, v_cache, block_tables, context_lens, scale, out_dtype, out,
-                 qdim, what):
-    q, k_cache, v_cache, block_tables, context_lens = _prep(
-        q, k_cache, v_cache, block_tables, context_lens, qdim, what)
+# The calls go through libpagedattn_torch.so (csrc/torch_ext.cpp), which builds
+# the C-ABI's tensor views, checks and scratch natively: a tiny decode took
+# 25 us of host time through ctypes and 6 through it.
+def _decode(version, q, k_cache, v_cache, block_tables, context_lens, scale, num_splits, k_scale, v_scale, out_dtype,
+            out, workspace):
+    _on_gpu(q, k_cache, v_cache)
     o = _out(q, out_dtype, out)
-    with torch.cuda.device(q.device):
-        check(fn(C.byref(view(o)), C.byref(view(q)), C.byref(view(k_cache)), C.byref(view(v_cache)),
-                 C.byref(view(block_tables)), C.byref(view(context_lens)), float(scale),
-                 _stream(q.device)))
+    torch_ops().decode_out(version, q, k_cache, v_cache, block_tables, context_lens, float(scale), int(num_splits),
+                           float(k_scale), float(v_scale), o, workspace)
+    return o
+
+
+def _prefill(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, max_q_len, scale, out_dtype, out,
+             k_scale, v_scale, fp32):
+    _on_gpu(q, k_cache, v_cache)
+    o = _out(q, out_dtype, out)
+    torch_ops().prefill_out(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, int(max_q_len),
+                            float(scale), float(k_scale), float(v_scale), fp32, o)
     return o
 
 
 def paged_attention(q, k_cache, v_cache, block_tables, context_lens, scale, *,
                     out_dtype=torch.float32, out=None):
     """kernels/paged_attn_v1.h:13-15 -- decode, q [B,H,D] -> out [B,H,D]."""
-    return _call_simple(lib().paged_attention, q, k_cache, v_cache, block_tables, context_lens,
-                        scale, out_dtype, out, 3, "[B, H, D]")
+    return _decode(1, q, k_cache, v_cache, block_tables, context_lens, scale, 0, 1.0, 1.0, out_dtype, out, None)
 
 
 def paged_attention_v2(q, k_cache, v_cache, block_tables, context_lens, scale, *,
                        out_dtype=torch.float32, out=None):
     """kernels/paged_attn_v2.h:13-15 -- online-softmax decode."""
-    return _call_simple(lib().paged_attention_v2, q, k_cache, v_cache, block_tables, context_lens,
-                        scale, out_dtype, out, 3, "[B, H, D]")
-
-
-def _scratch(need, dev):
-    """Split scratch from torch's caching allocator (None when the plan has no split)."""
-    if need == C.c_size_t(-1).value:
-        raise RuntimeError(last_error())
-    return torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-
-
-def _prefill(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, max_q_len, scale, out_dtype, out,
-             k_scale, v_scale, fp32):
-    varlen = cu_seqlens_q is not None
-    q, k_cache, v_cache, block_tables, context_lens = _prep(
-        q, k_cache, v_cache, block_tables, context_lens, 3 if varlen else 4,
-        "[T, H, D]" if varlen else "[B, S, H, D]")
-    cu = cu_seqlens_q.to(q.device, torch.int32).contiguous() if varlen else None
-    o = _out(q, out_dtype, out)
-    L = lib()
-    with torch.cuda.device(q.device):
-        qv, kv, bt = view(q), view(k_cache), view(block_tables)
-        ws = _scratch(L.paged_attention_prefill_workspace_size(C.byref(qv), C.byref(kv), C.byref(bt), int(max_q_len)),
-                      q.device)
-        check(L.paged_attention_prefill_split(
-            C.byref(view(o)), C.byref(qv), C.byref(kv), C.byref(view(v_cache)), C.byref(bt),
-            C.byref(view(context_lens)), C.byref(view(cu)) if varlen else None, int(max_q_len), float(scale),
-            float(k_scale), float(v_scale), int(fp32), ws.data_ptr() if ws is not None else None,
-            ws.numel() if ws is not None else 0, _stream(q.device)))
-    return o
+    return _decode(2, q, k_cache, v_cache, block_tables, context_lens, scale, 0, 1.0, 1.0, out_dtype, out, None)
 
 
 def paged_attention_prefill(q, k_cache, v_cache, block_tables, context_lens, scale, *,
@@ -176,24 +137,8 @@ def paged_attention_v3(q, k_cache, v_cache, block_tables, context_lens, scale, n
     num_splits <= 0 lets the library plan the split from the CU count.
     k_scale / v_scale dequantise a scaled cache (e.g. torch.float8_e4m3fn):
     attention runs on k_cache * k_scale and v_cache * v_scale."""
-    q, k_cache, v_cache, block_tables, context_lens = _prep(
-        q, k_cache, v_cache, block_tables, context_lens, 3, "[B, H, D]")
-    o = _out(q, out_dtype, out)
-    need = workspace_size(q, k_cache, block_tables, num_splits)
-    if workspace is None or workspace.numel() < need:
-        workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
-        if k_scale == 1.0 and v_scale == 1.0:
-            check(lib().paged_attention_v3(
-                C.byref(view(o)), C.byref(view(q)), C.byref(view(k_cache)), C.byref(view(v_cache)),
-                C.byref(view(block_tables)), C.byref(view(context_lens)), float(scale),
-                int(num_splits), workspace.data_ptr(), workspace.numel(), _stream(q.device)))
-        else:
-            check(lib().paged_attention_v3_scaled(
-                C.byref(view(o)), C.byref(view(q)), C.byref(view(k_cache)), C.byref(view(v_cache)),
-                C.byref(view(block_tables)), C.byref(view(context_lens)), float(scale), float(k_scale),
-                float(v_scale), int(num_splits), workspace.data_ptr(), workspace.numel(), _stream(q.device)))
-    return o
+    return _decode(3, q, k_cache, v_cache, block_tables, context_lens, scale, num_splits, k_scale, v_scale, out_dtype,
+                   out, workspace)
 
 
 def choose_num_splits(num_seqs: int, num_heads: int, max_context: int) -> int:
@@ -238,10 +183,7 @@ def write_kv(k_cache, v_cache, key, value, slot_mapping, k_scale=1.0, v_scale=1.
     if slot_mapping.dtype not in (torch.int32, torch.int64):
         slot_mapping = slot_mapping.to(torch.int64)
     slot_mapping = slot_mapping.to(key.device).contiguous()
-    with torch.cuda.device(key.device):
-        check(lib().pa_write_kv_scaled(C.byref(view(k_cache)), C.byref(view(v_cache)), C.byref(view(key)),
-                                       C.byref(view(value)), C.byref(view(slot_mapping)), float(k_scale),
-                                       float(v_scale), _stream(key.device)))
+    torch_ops().write_kv_into(k_cache, v_cache, key, value, slot_mapping, float(k_scale), float(v_scale))
 
 
 def write_kv_blocks(kv_pool, block_ids, start, k, v, k_scale=1.0, v_scale=1.0):
@@ -264,16 +206,21 @@ def write_kv_blocks(kv_pool, block_ids, start, k, v, k_scale=1.0, v_scale=1.0):
                  k_scale, v_scale)
 
 
+_ops = None
+
+
 def torch_ops():
     """The same launchers as PyTorch operators, torch.ops.gb10_attn.* (built from
     csrc/torch_ext.cpp into libpagedattn_torch.so): the reference's exact
     torch::Tensor signatures for callers that bind them from C++ or TorchScript,
     with no Python/ctypes work per call.  Raises ImportError when not built."""
-    from ._lib import LIB_PATH
-    path = LIB_PATH.with_name("libpagedattn_torch.so")
-    if not path.exists():
-        raise ImportError(f"{path} is missing: build it with __graft_entry__.build()")
-    if not hasattr(torch.ops, "gb10_attn") or not hasattr(torch.ops.gb10_attn, "paged_attention_v3"):
-        torch.ops.load_library(str(path))
-    return torch.ops.gb10_attn
-
+    global _ops
+    if _ops is None:
+        lib()  # (its ImportError names the missing library)
+        path = LIB_PATH.with_name("libpagedattn_torch.so")
+        if not path.exists():
+            raise ImportError(f"{path} is missing: build it with __graft_entry__.build()")
+        if not hasattr(torch.ops.gb10_attn, "paged_attention_v3"):
+            torch.ops.load_library(str(path))
+        _ops = torch.ops.gb10_attn
+    return _ops
