@@ -16,19 +16,28 @@ static hipError_t launch_p32_q(const PrefillParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Key-split mode (64 packed query rows per work-group) or the plain one (128):
+// see key_split_pays(); up to 64 rows take it too (half of the plain mode's
+// waves would have none).  At D = 128 q in several pieces takes it always: the
+// plain mode's two row tiles per wave overflow the registers there (60 to 100
+// spilled, none to 45 in the key-split mode): fp32 q, fp16 cache, 12 heads,
+// S = 4096 321 -> 128 us, eight of 1024 rows 151 -> 100, 32/8 heads, eight
+// 256-row chunks at 4096 457 -> 296; bf16 355 -> 165, 173 -> 127, 574 -> 397.
 template <typename KV, int D, int kQP>
 static hipError_t launch_p32(const PrefillParams& p, hipStream_t stream) {
   if constexpr (PfShape<D>::MT == 2) {
-    // Key-split mode (64 query rows per work-group) for grids of few
-    // work-groups, and for up to 64 rows (half of the plain mode's waves would
-    // have none).
-    static std::atomic<int64_t> cache[64];
-    int64_t cus = 0, per_cu = 0;
-    residency(prefill32_kernel<KV, D, kQP, false>, cache, &cus, &per_cu);
-    const int64_t plain = (int64_t)p.B * p.H * ((p.S + PfShape<D>::QB - 1) / PfShape<D>::QB);
-    if (p.S <= 64 || (cus > 0 && plain < cus)) return launch_p32_q<KV, D, kQP, true>(p, stream);
+    if constexpr (D == 128 && kQP > 1) {
+      return launch_p32_q<KV, D, kQP, true>(p, stream);
+    } else {
+      static std::atomic<int64_t> cache[64];
+      int64_t cus = 0, per_cu = 0;
+      residency(prefill32_kernel<KV, D, kQP, true>, cache, &cus, &per_cu);
+      const int64_t rows = (int64_t)p.S * p.gp, QB = PfShape<D>::QB;
+      if (rows <= 64 || key_split_pays((int64_t)p.B * p.HG * ((rows + QB - 1) / QB), cus, per_cu))
+        return launch_p32_q<KV, D, kQP, true>(p, stream);
+    }
   }
-  return launch_p32_q<KV, D, kQP, false>(p, stream);
+  if constexpr (!(D == 128 && kQP > 1)) return launch_p32_q<KV, D, kQP, false>(p, stream);
 }
 
 template <typename KV, int kQP>

@@ -87,14 +87,45 @@ def test_prefill32(pa, dev, kv, qt, D):
 
 @pytest.mark.parametrize("kv", ["f16", "bf16"])
 def test_prefill32_plain_mode(pa, dev, kv):
-    """A grid of at least a work-group per CU (128 rows per work-group)."""
+    """A grid of two work-groups per CU (128 rows per work-group)."""
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    H = -(-cus // 4)
-    q, k, v, bt, c, k32, v32 = case(2, 130, H, 1, 64, 16, [130, 200], kv, "f32", 5)
+    H = cus // 2
+    q, k, v, bt, c, k32, v32 = case(2, 130, H, H, 64, 16, [130, 200], kv, "f32", 5)
     print("plain mode", kv, flush=True)
     got = run(pa, dev, q, k, v, bt, c, 0.125)
     assert pa.last_launch().endswith("false>"), pa.last_launch()
-    close64(got[:, :, :2], attention64(q[:, :, :2].contiguous(), k32, v32, bt, c, 0.125))
+    close64(got[:, :, :2], attention64(q[:, :, :2].contiguous(), k32[:, :, :2], v32[:, :, :2], bt, c, 0.125))
+
+
+@pytest.mark.parametrize("fn,D,qt,per_cu", [("paged_attention_prefill", 64, "f16", 3),
+                                            ("paged_attention_prefill_wmma", 64, "f16", 3),
+                                            ("paged_attention_prefill_wmma", 64, "f32", 3),
+                                            ("paged_attention_prefill", 128, "f16", 2),
+                                            ("paged_attention_prefill_wmma", 128, "f16", 2),
+                                            ("paged_attention_prefill", 128, "f32", None)])
+@pytest.mark.parametrize("over", [0, 1])
+def test_key_split_bound(pa, dev, fn, D, qt, per_cu, over):
+    """The largest grid whose halves are resident at once (per_cu of them per
+    CU) takes the key-split mode, the next one the plain mode; at D = 128 q in
+    pieces always takes the key-split mode.  Heads of every part of the grid
+    against attention in 64 bits; the 16-bit weights of the matrix-core form
+    round by 2^-12 each, 2.5e-4 at most."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    H = cus * (per_cu or 3) // 4 + over  # two 128-row blocks per head
+    q, k, v, bt, c, k32, v32 = case(1, 130, H, H, D, 16, [140], "f16", qt, 6)
+    print("key split bound", fn, D, qt, H, flush=True)
+    got = to_host(getattr(pa, fn)(q.to(dev), k.to(dev), v.to(dev), torch.from_numpy(bt).to(dev),
+                                  torch.from_numpy(c).to(dev), 0.1))
+    split = per_cu is None or not over
+    assert pa.last_launch().endswith("true>" if split else "false>"), pa.last_launch()
+    for h in (0, H // 2, H - 1):
+        one = slice(h, h + 1)
+        want = attention64(q[:, :, one].contiguous(), k32[:, :, one], v32[:, :, one], bt, c, 0.1)
+        if fn == "paged_attention_prefill":
+            close64(got[:, :, one], want)
+        else:
+            err = float((torch.from_numpy(got[:, :, one]).double() - want).norm() / want.norm())
+            assert err < 2.5e-4, err
 
 
 def test_prefill32_q_range(pa, dev):
