@@ -559,8 +559,8 @@ PrefillParams prefill_params(const DecodeArgs& a, const int32_t* cu, int64_t T, 
   return pp;
 }
 
-// Whether the matrix-core kernel serves a paged_attention_prefill call (16-bit
-// and FP8 caches, a 16-byte aligned q); else it runs as a decode problem per
+// Whether the matrix-core kernel serves a paged_attention_prefill call (bf16,
+// FP8 and ungrouped fp16 caches, a 16-byte aligned q); else it runs as a decode problem per
 // query row.  It does when its context split is planned, when those decode
 // problems are kPrefill32Units work-groups or more, and for several rows of
 // groups of eight heads (whose decode problems run on the vector ALU).
@@ -571,8 +571,12 @@ PrefillParams prefill_params(const DecodeArgs& a, const int32_t* cu, int64_t T, 
 // rows (512 / 1024 units) 21.7 vs 22.0, 39.2 vs 23.5; 8/1 heads, two rows at
 // 64 / 512: 13.3 vs 10.5, 29.2 vs 20.3.
 constexpr int64_t kPrefill32Units = 768;
+// Groups over fp16 caches keep the decode kernel: its packed P.V carries their
+// weights as fp16 pairs (1.3e-4 from 64 bits; the matrix kernel 1.7e-7), and the
+// calls' results stay what they were to the fp32 tolerance.  (8/2 heads of 128,
+// 75 us against 19 there.)
 bool prefill32_eligible(const DecodeArgs& a, const pa_tensor_t* q) {
-  return prefill_kv(a.kv_dtype) && aligned16(q->data);
+  return prefill_kv(a.kv_dtype) && !(a.kv_dtype == kF16 && a.gc > 1) && aligned16(q->data);
 }
 bool prefill32_pays(const DecodeArgs& a, const PrefillParams& pp) {
   return pp.parts > 1 || (a.gc >= 8 && a.p.Sq > 1) ||
