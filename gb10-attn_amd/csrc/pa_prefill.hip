@@ -31,9 +31,11 @@ static hipError_t launch_pp(const PrefillParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Key-split mode: see key_split_pays(); a variable-length batch takes it when
-// the plain grid (blocks of 128 query rows) has fewer work-groups than CUs
+// Key-split mode when the plain grid (blocks of 128 query rows) has fewer
+// work-groups than CUs: chunks of a long context
 // (the reference's 512-token chunk at context 2048: 192 work-groups, +19 %).
+// Above that, twice the tiles cost more than the shorter chains save
+// (config 4a, 768 work-groups: -17 %).
 // The choice counts the work-groups that have rows to serve: a uniform
 // batch's B * ceil(S / rows) per head; a variable-length batch brings T rows
 // in all (its grid is sized by the longest sequence, and the work-groups past
@@ -43,20 +45,15 @@ static hipError_t launch_pp(const PrefillParams& p, hipStream_t stream) {
 template <typename KV, int D>
 static hipError_t launch_pf(const PrefillParams& p, hipStream_t stream) {
   if constexpr (PfShape<D>::MT == 2) {
-    static std::atomic<int64_t> cache[2][64];
+    static std::atomic<int64_t> cache[64];
     int64_t cus = 0, per_cu = 0;
-    if (p.q_split) {
-      residency(prefill_mfma_kernel<KV, D, true, true>, cache[1], &cus, &per_cu);
-    } else {
-      residency(prefill_mfma_kernel<KV, D, false, true>, cache[0], &cus, &per_cu);
-    }
+    residency(prefill_mfma_kernel<KV, D, false, false>, cache, &cus, &per_cu);
     auto busy = [&](int rows) {
       const int64_t grid = (int64_t)p.B * ((p.S + rows - 1) / rows);
       return (int64_t)p.H * (p.cu_q ? std::min<int64_t>(grid, (p.q_total + rows - 1) / rows) : grid);
     };
-    const int64_t rows = (int64_t)p.S * p.gp, QB = PfShape<D>::QB;
-    if (p.cu_q ? cus > 0 && busy(PfShape<D>::QB) < cus
-               : rows <= 64 || key_split_pays((int64_t)p.B * p.HG * ((rows + QB - 1) / QB), cus, per_cu))
+    const int64_t plain = busy(PfShape<D>::QB);
+    if ((cus > 0 && plain < cus) || (!p.cu_q && (int64_t)p.S * p.gp <= 64))
       return p.q_split ? launch_pf_q<KV, D, true, true>(p, stream) : launch_pf_q<KV, D, false, true>(p, stream);
     // The 8-wave kernel (one work-group per CU) for grids of at least two
     // of its work-groups per CU; below that its 256-row blocks leave CUs

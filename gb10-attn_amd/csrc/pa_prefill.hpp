@@ -1802,16 +1802,15 @@ static int64_t pf_grid(F kernel, std::atomic<int64_t> (&cache)[64], int QB, Pref
   return units;
 }
 
-// Whether `plain` blocks of 128 packed rows run faster as twice as many
-// key-split ones of 64 (per_cu of them resident per CU): where all of those are
-// resident at once, up to three per CU.  384 plain blocks on 256 CUs take two
-// blocks' time, 768 halves at three per CU one and a half.  fp16, D = 64, 12
-// heads: S = 4096 67.7 -> 54.8 us, three 1024-row chunks at 2048 38.4 -> 31.4; 24
-// heads, four 512-row chunks at 4096 88.9 -> 85.2 (fp32 precision 121 -> 106); D
-// = 32 68.9 -> 58.9.  Two per CU (D = 128): 256 blocks, one prompt of 1024 rows
-// of 32/8 heads, 30.2 -> 24.7 (fp32 precision 49.0 -> 32.6); but 384, 24 heads,
-// four chunks at 4096, 137 -> 183.  Past that the halves only pay their second
-// reading of K and V (D = 64, 448 blocks, fp32 precision: 34.5 -> 40.6).
+// Whether `plain` blocks of 128 packed rows of the fp32-precision prefill run
+// faster as twice as many key-split ones of 64 (per_cu of them resident per CU):
+// where all of those are resident at once, up to three per CU.  384 plain blocks
+// on 256 CUs take two blocks' time, 768 halves at three per CU one and a half.
+// fp16, D = 64: 12 heads, S = 4096 91.2 -> 74.1 us; 24 heads, four 512-row
+// chunks at 4096 121 -> 106.  Two per CU (D = 128, bf16 q): 256 blocks, one prompt
+// of 1024 rows of 32/8 heads, 55 -> 35; but 384, 24 heads, fp16, four chunks at
+// 4096, 209 -> 234.  Past that the halves only pay their second reading of K and V
+// (D = 64, 448 blocks: 34.5 -> 40.6).
 inline bool key_split_pays(int64_t plain, int64_t cus, int64_t per_cu) {
   return 2 * plain <= cus * std::clamp<int64_t>(per_cu, 2, 3);
 }
