@@ -623,7 +623,9 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p) {
       l *= corr;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) o[dt] *= corr;
-      const float negm = m == -__builtin_inff() ? 0.0f : -m;
+      // (The weights carry the matrix pass's scale: partitions of a context split
+      // that took either pass are merged.)
+      const float negm = (m == -__builtin_inff() ? 0.0f : -m) + kXBias;
 #pragma unroll 1
       for (int r = 0; r < 16; ++r) {
         const int key0 = mt * 32 + 8 * (r >> 2) + (r & 3);  // lane half 0's key; half 1's is 4 further

@@ -165,3 +165,33 @@ def test_prefill32_non_finite(pa, dev, kv):
     bad[0, 5] = 10 ** 6  # keys 80..95: rows whose own keys include one of them
     got = run(pa, dev, q, k, v, bad, c, 0.125)
     assert np.isnan(got[0, 30:]).all() and np.isfinite(got[0, :30, :]).all()
+
+
+@pytest.mark.parametrize("kv", ["f16", "bf16", "fp8"])
+@pytest.mark.parametrize("D", [64, 256])
+def test_prefill32_split_non_finite(pa, dev, kv, D):
+    """Inf and NaN in one partition of a context split: that partition's sums
+    come from another pass than its neighbours' and merge in the same units.
+    Head 0 has them in the keys of the last rows of a block only, head 1 in one
+    dim of an early key, head 2 nowhere."""
+    B, S, H, BS, ctx = 1, 70, 3, 16, [2500]
+    q, k, v, bt, c, k32, v32 = case(B, S, H, H, D, BS, ctx, kv, "f32", 22)
+
+    def put(x, x32, key, head, dim, val):
+        page, row = int(bt[0, key // BS]), key % BS
+        if kv == "fp8":
+            x.view(torch.uint8)[page, row, head, dim] = 0x7f  # NaN
+            val = float("nan")
+        else:
+            x[page, row, head, dim] = val
+        x32[page, row, head, dim] = val
+
+    put(v, v32, 2490, 0, 3, float("inf"))
+    put(k, k32, 2496, 0, 9, float("nan"))
+    put(v, v32, 100, 1, 7, float("nan"))
+    print("split non-finite", kv, D, flush=True)
+    got = run(pa, dev, q, k, v, bt, c, 0.125)
+    assert "prefill_reduce_kernel" in pa.last_launch(), pa.last_launch()
+    want = attention64(q, k32, v32, bt, c, 0.125)
+    for h in range(H):
+        close64(got[:, :, h], want[:, :, h])
