@@ -257,7 +257,11 @@ __device__ __forceinline__ bool pf_unit(const PrefillParams& p, int64_t x, int l
       for (int c = 0; c < kVlMaxSeqs / 64; ++c) mine += nbk[c];
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) mine += __shfl_xor(mine, o, 64);
-      const int64_t total = (int64_t)mine * p.HG;
+      // No more than the grid and the workspace hold: a cu_q whose ranges overlap
+      // ([0, 512, 0, 512] of 512 rows) has more rows than T.  The units past them
+      // stay unserved, as past the end of the unsplit kernel's grid.
+      const int64_t rows = (int64_t)mine * p.HG;
+      const int64_t total = rows < p.units ? rows : p.units;
       if (x >= total * p.parts) return false;
       part = (int)(x / total);
       x -= part * total;

@@ -91,3 +91,32 @@ def test_prefill_split_workspace_checks(pa, dev):
     short = prefill_case(1, 70, 2, 1, 64, 16, [100], seed=1, kv="f16", qt="f16")
     v3 = [pa.view(t) for t in dev_args(short, dev)]
     assert L.paged_attention_prefill_workspace_size(C.byref(v3[0]), C.byref(v3[1]), C.byref(v3[3]), 0) == 0
+
+
+def test_varlen_split_overlapping_ranges(pa, dev):
+    """Ranges that overlap (each in itself well formed) number more blocks than
+    the workspace and the grid are sized for: what does not fit is not served,
+    and nothing beyond the workspace is written.  Sequences 0 and 2 are the same
+    rows, keys and values, so the rows that are served have one result."""
+    L, H, D, S, n = pa.lib(), 12, 64, 512, 2048
+    inp = oracle.paged_inputs(1, 1, H, D, 16, [n], seed=12, kv_dtype="f16")
+    q = np.random.default_rng(12).standard_normal((S, H, D), dtype=np.float32)
+    dq = to_dev(q, "f32", dev)
+    t = [torch.full((S, H, D), 7.0, device=dev), dq, to_dev(inp["k"], "f16", dev), to_dev(inp["v"], "f16", dev),
+         torch.from_numpy(np.repeat(inp["bt"], 3, 0)).to(dev), torch.full((3,), n, dtype=torch.int32, device=dev),
+         torch.tensor([0, S, 0, S], dtype=torch.int32, device=dev)]
+    V = [pa.view(x) for x in t]
+    need = L.paged_attention_prefill_workspace_size(C.byref(V[1]), C.byref(V[2]), C.byref(V[4]), S)
+    assert need > 0
+    guard = 1 << 20
+    ws = torch.full((need + 2 * guard,), 0xA5, dtype=torch.uint8, device=dev)
+    print("overlapping ranges", flush=True)
+    pa.check(L.paged_attention_prefill_split(*[C.byref(x) for x in V], S, 0.125, 1.0, 1.0, 0, ws.data_ptr() + guard,
+                                             need, torch.cuda.current_stream().cuda_stream))
+    assert "prefill_reduce_kernel" in pa.last_launch(), pa.last_launch()
+    assert bool((ws[:guard] == 0xA5).all()) and bool((ws[guard + need:] == 0xA5).all())
+    got = to_host(t[0])
+    # 132 units of 64 rows and a head: blocks 7 .. 3 of both sequences, block 2 of one.
+    want = oracle.prefill(q[None], inp["k"], inp["v"], inp["bt"], inp["ctx"], 0.125, "f16")[0]
+    close(got[128:], want[128:])
+    assert np.all(got[:128] == 7.0)
