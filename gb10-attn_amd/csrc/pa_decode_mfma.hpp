@@ -18,7 +18,8 @@
 //    global_load_lds_dwordx4 and is read transposed (ds_read_b64_tr_b16);
 //    the probabilities never leave registers.  P is carried as a 16-bit
 //    hi + lo pair (two products; ~22/16-bit significand for fp16/bf16), and q
-//    likewise when it does not arrive in the KV type, so the result keeps the
+//    likewise when it does not arrive in the KV type (fp16 pairs of a row
+//    scaled by a power of two, so any finite fp32 q is served), so the result keeps the
 //    fp32-softmax precision of the reference's decode (kernels/paged_attn_v3.cu:93-111).
 //  * Two tiles in flight per wave (K in registers, V in a double-buffered LDS
 //    area); rows past the partition end, or on pages with an invalid block id,
@@ -171,11 +172,34 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) 
   const bool qlive = col < GC && g0 + col < p.G;
   const bool split_q = SQ && p.q_dtype != KV::kCode;
   u32x4_t qf[KS], qlo[KS];
+  float qscale = p.qscale;  // (per lane: its head column's, with the inverse of q's scale)
   {
     const int64_t qb = ((int64_t)z * p.H + kvh * p.G + g0 + (qlive ? col : 0)) * D + kg * 8;
     float xq[KS][8];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) load_elems<8>(p.q, p.q_dtype, qb + 32 * ks, xq[ks]);
+    // fp16 pieces have fp16's range: the head's row is scaled by the power of two
+    // that puts its largest element in [2^14, 2^15) (an fp32 element past 65504
+    // would be Inf - Inf), and its scores by the inverse.  Inf keeps its scale.
+    if constexpr (SQ && !kBf16) {
+      float mxq = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) mxq = fmaxf(mxq, __builtin_fabsf(xq[ks][e]));
+      }
+      mxq = fmaxf(mxq, __shfl_xor(mxq, 16, 64));
+      mxq = fmaxf(mxq, __shfl_xor(mxq, 32, 64));
+      const int ex = (int)(__builtin_bit_cast(uint32_t, mxq) >> 23) - 127;
+      const int k = ex > 127 ? 0 : max(-113, min(100, 14 - ex));
+      const float up = __builtin_bit_cast(float, (uint32_t)(127 + k) << 23);
+      qscale *= __builtin_bit_cast(float, (uint32_t)(127 - k) << 23);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xq[ks][e] *= up;
+      }
+    }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       uint32_t w[4], wl[4];
@@ -191,7 +215,6 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) 
       qlo[ks] = u32x4_t{wl[0], wl[1], wl[2], wl[3]};
     }
   }
-  const float qscale = p.qscale;
 
   const char* kbase = static_cast<const char*>(p.k) + (int64_t)kvh * p.k_sh * 2;
   const char* vbase = static_cast<const char*>(p.v) + (int64_t)kvh * p.v_sh * 2;

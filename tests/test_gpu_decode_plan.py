@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from _helpers import close, decode_case, dev_inputs, oracle_decode_rows, to_host
+from test_gpu_prefill32 import attention64, case
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +66,28 @@ def test_equal_contexts_uncut(pa, dev, kv, lens):
         got[7] = 0.0
         ctx[7] = 0
     close(got, oracle_decode_rows(inp["q_f32"], inp["k"], inp["v"], inp["bt"], ctx, 0.125, kv))
+
+
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+@pytest.mark.parametrize("S", [0, 16])
+def test_matrix_decode_q_range(pa, dev, D, S):
+    """fp32 q beyond fp16's range, large and small elements mixed in a row,
+    tiny and zero rows, over an fp16 cache with groups of eight.  Tolerance: q
+    and the weights carry 22 bits each, and a score of up to 30 log2 units moves
+    its weight by 30 * 2^-22 of itself: 1e-5."""
+    ctx = [700, 1, 2049]
+    q, k, v, bt, c, k32, v32 = case(3, 1, 16, 2, D, 16, ctx, "f16", "f32", D + S)
+    q[0, 0, :8] *= 3e5
+    q[0, 0, 8:, ::2] *= 1e6
+    q[1, 0] *= 1e-30
+    q[2, 0, 3] = 0.0
+    q[2, 0, 4:9] *= 1e30
+    print("q range", D, S, flush=True)
+    for b, scale in ((0, 2e-7), (1, 0.1), (2, 2e-31)):
+        one = slice(b, b + 1)
+        got = to_host(pa.paged_attention_v3(q[one, 0].to(dev), k.to(dev), v.to(dev), torch.from_numpy(bt[one]).to(dev),
+                                            torch.from_numpy(c[one]).to(dev), scale, S))
+        assert "decode_mfma_kernel" in pa.last_launch(), pa.last_launch()
+        want = attention64(q[one], k32, v32, bt[one], c[one], scale)[:, 0]
+        err = float((torch.from_numpy(got).double() - want).norm() / want.norm())
+        assert err < 1e-5, (b, err)
