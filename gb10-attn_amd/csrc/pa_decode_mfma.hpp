@@ -439,7 +439,7 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) 
     const int h = kvh * p.G + g0 + g;
     if (final_here) {
       store_elem(p.out, p.out_dtype, ((int64_t)z * p.H + h) * D + d,
-                 bad ? __builtin_nanf("") : (L > 0.0f ? A * p.vscale / L : 0.0f));
+                 bad ? __builtin_nanf("") : A * p.vscale / L);
     } else {
       const int64_t pidx = ((int64_t)b * p.H + h) * p.parts + part;
       p.ws_acc[pidx * D + d] = A * p.vscale;

@@ -91,3 +91,24 @@ def test_matrix_decode_q_range(pa, dev, D, S):
         want = attention64(q[one], k32, v32, bt[one], c[one], scale)[:, 0]
         err = float((torch.from_numpy(got).double() - want).norm() / want.norm())
         assert err < 1e-5, (b, err)
+
+
+@pytest.mark.parametrize("kv", ["f16", "bf16"])
+@pytest.mark.parametrize("S", [0, 1, 16])
+def test_matrix_decode_non_finite_scores(pa, dev, kv, S):
+    """A NaN or +Inf score makes its row NaN, as on the vector kernel, and so do
+    scores that are all -Inf; -Inf among others is a weight of 0."""
+    q, k, v, bt, c, k32, v32 = case(4, 1, 16, 2, 64, 16, [40, 40, 1, 700], kv, kv, 5)
+    q[:, :, :, 2] = q[:, :, :, 2].abs() + 1  # (the sign of the scores below)
+    for b, key, head, val in ((0, 7, 0, "nan"), (1, 30, 1, "inf"), (2, 0, 0, "-inf"), (3, 300, 1, "-inf")):
+        page = int(bt[b, key // 16])
+        k[page, key % 16, head, 2] = float(val)
+        k32[page, key % 16, head, 2] = float(val)
+    print("non-finite scores", kv, S, flush=True)
+    got = to_host(pa.paged_attention_v3(q[:, 0].to(dev), k.to(dev), v.to(dev), torch.from_numpy(bt).to(dev),
+                                        torch.from_numpy(c).to(dev), 0.125, S))
+    assert "decode_mfma" in pa.last_launch(), pa.last_launch()
+    want = attention64(q, k32, v32, bt, c, 0.125)[:, 0].float().numpy()
+    assert np.isnan(want[0, :8]).all() and np.isnan(want[2, :8]).all() and np.isfinite(want[3]).all()
+    close(got, want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
