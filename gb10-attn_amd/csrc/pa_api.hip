@@ -660,7 +660,10 @@ int run_v3(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const p
     return fail(PA_ERR_WORKSPACE, "workspace too small: need %zu bytes, got %zu", need, ws ? ws_bytes : 0);
   if (need > 0 && (reinterpret_cast<uintptr_t>(ws) & 255) != 0)
     return fail(PA_ERR_WORKSPACE, "workspace must be 256-byte aligned");
-  if (phases == kBoth && own_plan_pays(a, num_splits) && (rc = own_plan(a, num_splits, &plan))) return rc;
+  if (phases == kBoth && own_plan_pays(a, num_splits)) {
+    if ((rc = own_plan(a, num_splits, &plan))) return rc;
+    a.p.fp32_weights = 1;  // as the explicit partitions' kernel
+  }
   a.p.parts = (int)plan.parts;
   a.p.part_tokens = (int)plan.part_tokens;
   a.p.direct = plan.direct ? 1 : 0;

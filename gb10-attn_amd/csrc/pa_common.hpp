@@ -64,6 +64,7 @@ struct DecodeParams {
   int32_t wave_parts;   // explicit splits into short chunks: 1 from the host (the launcher picks the
                         // mode: a partition per wave or per token slot); 0 otherwise
   int32_t uniform_whole;  // part_len(): nearly equal contexts are not cut (B <= 64)
+  int32_t fp32_weights;   // matrix-core decode over a bf16 cache: weights (and fp32 q) in 24 bits, not 16
   int32_t seq_order;    // explicit split into long partitions, B <= 64, Sq = 1: sequences dispatched
                         // longest first
   FastDiv bs_div;

@@ -96,16 +96,39 @@ __device__ inline int dm_vpos(int r, int cc) {
 constexpr float kDmLazy = 8.0f;  // raise the running max only past 2^8
 
 
+// x in three bf16 pieces, cut toward zero: their sum is the fp32 value.  A piece
+// that is 0 becomes the smallest normal of x's sign where x is 2^26 times that or
+// more, so an Inf times the pieces is Inf, as in fp32 (0 * Inf is NaN).
+__device__ inline void cut3(float x, float (&pc)[3]) {
+  const float least = __builtin_fabsf(x) >= 0x1p-100f ? __builtin_copysignf(0x1p-126f, x) : 0.0f;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const float c = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xffff0000u);
+    pc[i] = c == 0.0f ? least : c;
+    x -= c;
+  }
+}
+__device__ inline uint32_t pack_hi(float x, float y) {  // the upper halves of two floats
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, y), __builtin_bit_cast(uint32_t, x), 0x07060302u);
+}
+
 // SQ: q may need the hi + lo split (q's dtype is not the cache's).  A
 // separate instance for q of the cache's dtype keeps the run-time test out of
 // the k-step loop, where it put a branch between consecutive MFMAs.
-template <typename KV, int D, int GC, bool SQ>
-__global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) {
+// EX (bf16 caches, DecodeParams::fp32_weights): weights and a split q as three
+// bf16 pieces, 24 bits, where hi + lo hold 16: explicit split counts, whose own
+// partitions run on the vector kernel with fp32 weights, keep their precision.
+// 64 partitions asked for, 64/8 heads of 128, fp32 q, error against 64 bits at 2048
+// tokens: partitions 2.6e-7, hi + lo 3.3e-6, three pieces 2.2e-7; 32 sequences of
+// 2048 tokens: partitions 122 us, three pieces 53.6 (the loads bound it).
+template <typename KV, int D, int GC, bool SQ, bool EX>
+__device__ __forceinline__ void decode_mfma_body(const DecodeParams& p) {
   using Sh = DmShape<D>;
   constexpr int KT = Sh::KT, KS = Sh::KS, NDT = Sh::NDT, NCH = Sh::NCH, TPD = Sh::TPD, NDMA = Sh::NDMA;
   constexpr int NW = 4;
   constexpr bool kBf16 = KV::kCode == kBF16;
   static_assert(GC <= 16, "the GQA group is one 16-column MFMA n-tile");
+  static_assert(!EX || kBf16, "fp16 pieces are hi + lo");
 
   // Per-wave double-buffered V tiles; reused for the cross-wave merge.
   __shared__ __attribute__((aligned(16))) uint16_t s_v[NW][2][Sh::TILE];
@@ -171,7 +194,7 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) 
   // in the KV type (hi + lo when q is another type).
   const bool qlive = col < GC && g0 + col < p.G;
   const bool split_q = SQ && p.q_dtype != KV::kCode;
-  u32x4_t qf[KS], qlo[KS];
+  u32x4_t qf[KS], qlo[KS], qx[EX && SQ ? KS : 1];
   float qscale = p.qscale;  // (per lane: its head column's, with the inverse of q's scale)
   {
     const int64_t qb = ((int64_t)z * p.H + kvh * p.G + g0 + (qlive ? col : 0)) * D + kg * 8;
@@ -202,17 +225,27 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) 
     }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      uint32_t w[4], wl[4];
+      uint32_t w[4], wl[4], wx[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float x0 = qlive ? xq[ks][2 * j] : 0.0f;
         const float x1 = qlive ? xq[ks][2 * j + 1] : 0.0f;
+        if constexpr (EX && SQ) {
+          float a[3], b[3];
+          cut3(x0, a);
+          cut3(x1, b);
+          w[j] = pack_hi(a[0], b[0]);
+          wl[j] = pack_hi(a[1], b[1]);
+          wx[j] = pack_hi(a[2], b[2]);
+          continue;
+        }
         w[j] = pack2m<kBf16>(x0, x1);
         const float2_t r = unpack2m<kBf16>(w[j]);
         wl[j] = pack2m<kBf16>(x0 - r[0], x1 - r[1]);
       }
       qf[ks] = u32x4_t{w[0], w[1], w[2], w[3]};
       qlo[ks] = u32x4_t{wl[0], wl[1], wl[2], wl[3]};
+      if constexpr (EX && SQ) qx[ks] = u32x4_t{wx[0], wx[1], wx[2], wx[3]};
     }
   }
 
@@ -298,8 +331,24 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) 
       st[mt] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
+        if constexpr (EX) continue;
         st[mt] = mfma16<kBf16>(T.k[mt][ks], qf[ks], st[mt]);
         if (split_q) st[mt] = mfma16<kBf16>(T.k[mt][ks], qlo[ks], st[mt]);
+      }
+      if constexpr (EX) {  // small pieces first, two chains: fewer roundings of the whole score
+        float4_t sb = float4_t{0.f, 0.f, 0.f, 0.f};
+        if constexpr (SQ) {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) st[mt] = mfma16<kBf16>(T.k[mt][ks], qx[ks], st[mt]);
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) st[mt] = mfma16<kBf16>(T.k[mt][ks], qlo[ks], st[mt]);
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          float4_t& acc = ks & 1 ? sb : st[mt];
+          acc = mfma16<kBf16>(T.k[mt][ks], qf[ks], acc);
+        }
+        if constexpr (KS > 1) st[mt] += sb;
       }
     }
     // Scores in log2 units (any sign of the scale).  Lane (col, kg) holds
@@ -333,20 +382,32 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) 
     }
     const float negm = m == -__builtin_inff() ? 0.0f : -m;
     // P^T operand: slots 0..3 = m-tile 0 (tokens kg*4 + i), 4..7 = m-tile 1.
-    uint32_t w[4], wl[4];
+    uint32_t w[4], wl[4], wx[4];
+    float lt = 0.0f;  // EX: the tile's weights
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const float p0 = fast_exp2(st[mt][2 * j] + negm);
         const float p1 = fast_exp2(st[mt][2 * j + 1] + negm);
-        l += p0 + p1;
+        if constexpr (!EX) l += p0 + p1;
+        if constexpr (EX) {
+          lt += p0 + p1;
+          float a[3], b[3];
+          cut3(p0, a);
+          cut3(p1, b);
+          w[mt * 2 + j] = pack_hi(a[0], b[0]);
+          wl[mt * 2 + j] = pack_hi(a[1], b[1]);
+          wx[mt * 2 + j] = pack_hi(a[2], b[2]);
+          continue;
+        }
         const uint32_t h = pack2m<kBf16>(p0, p1);
         const float2_t r = unpack2m<kBf16>(h);
         w[mt * 2 + j] = h;
         wl[mt * 2 + j] = pack2m<kBf16>(p0 - r[0], p1 - r[1]);
       }
     }
+    if constexpr (EX) l += lt;
     const u32x4_t pb = u32x4_t{w[0], w[1], w[2], w[3]};
     const u32x4_t pl = u32x4_t{wl[0], wl[1], wl[2], wl[3]};
     // V^T operand of dim tile dt: rows kg*4 + (col/4) and 16 + kg*4 + (col/4),
@@ -361,8 +422,14 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) 
           (lds_short4m_t*)(cv + (r0 + 16) * D + (dm_vpos<D>(r0 + 16, c >> 3) << 3) + (c & 7)));
       const uint64_t lo64 = __builtin_bit_cast(uint64_t, lo), hi64 = __builtin_bit_cast(uint64_t, hi);
       const u32x4_t a = u32x4_t{(uint32_t)lo64, (uint32_t)(lo64 >> 32), (uint32_t)hi64, (uint32_t)(hi64 >> 32)};
-      o[dt] = mfma16<kBf16>(a, pb, o[dt]);
-      o[dt] = mfma16<kBf16>(a, pl, o[dt]);
+      if constexpr (EX) {  // (the tile's products summed on their own: O is rounded once per 32 keys)
+        float4_t ot = mfma16<kBf16>(a, u32x4_t{wx[0], wx[1], wx[2], wx[3]}, float4_t{0.f, 0.f, 0.f, 0.f});
+        ot = mfma16<kBf16>(a, pl, ot);
+        o[dt] += mfma16<kBf16>(a, pb, ot);
+      } else {
+        o[dt] = mfma16<kBf16>(a, pb, o[dt]);
+        o[dt] = mfma16<kBf16>(a, pl, o[dt]);
+      }
     }
   };
 
@@ -451,15 +518,30 @@ __global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) 
   }
 }
 
+template <typename KV, int D, int GC, bool SQ>
+__global__ __launch_bounds__(256) void decode_mfma_kernel(const DecodeParams p) {
+  decode_mfma_body<KV, D, GC, SQ, false>(p);
+}
+
+template <typename KV, int D, int GC, bool SQ>
+__global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void decode_mfma32_kernel(const DecodeParams p) {
+  decode_mfma_body<KV, D, GC, SQ, true>(p);
+}
+
 template <typename KV, int D, int GC>
 hipError_t launch_decode_mfma_dg(const DecodeParams& p, hipStream_t stream) {
   const int64_t blocks = (int64_t)p.B * p.Sq * p.HKV * p.head_chunks * p.parts;
   const bool sq = p.q_dtype != KV::kCode;
-  note_launch("pa::decode_mfma_kernel<%s, %d, %d, %s>", KV::kName, D, GC, sq ? "true" : "false");
-  if (!sq)
-    hipLaunchKernelGGL((decode_mfma_kernel<KV, D, GC, false>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
-  else
-    hipLaunchKernelGGL((decode_mfma_kernel<KV, D, GC, true>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+  auto kernel = sq ? decode_mfma_kernel<KV, D, GC, true> : decode_mfma_kernel<KV, D, GC, false>;
+  const char* name = "decode_mfma_kernel";
+  if constexpr (KV::kCode == kBF16) {
+    if (p.fp32_weights) {
+      kernel = sq ? decode_mfma32_kernel<KV, D, GC, true> : decode_mfma32_kernel<KV, D, GC, false>;
+      name = "decode_mfma32_kernel";
+    }
+  }
+  note_launch("pa::%s<%s, %d, %d, %s>", name, KV::kName, D, GC, sq ? "true" : "false");
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 

@@ -112,3 +112,41 @@ def test_matrix_decode_non_finite_scores(pa, dev, kv, S):
     assert np.isnan(want[0, :8]).all() and np.isnan(want[2, :8]).all() and np.isfinite(want[3]).all()
     close(got, want)
     assert np.array_equal(np.isnan(got), np.isnan(want))
+
+
+@pytest.mark.parametrize("kv,qt", [("bf16", "f32"), ("bf16", "f16"), ("bf16", "bf16"), ("f16", "f32"), ("f16", "f16")])
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+def test_explicit_count_precision(pa, dev, kv, qt, D):
+    """Explicit counts over groups of eight: fp32 weights (bf16 caches: three
+    bf16 pieces; fp16: 22 bits).  Tolerance: N(0, 1) scores of up to 8 carry a
+    rounding of 8 * 2^-24 (fp16 pieces 2^-22) and sums a few 2^-24: 1e-6."""
+    ctx = [700, 1, 2049, 64]
+    q, k, v, bt, c, k32, v32 = case(4, 1, 16, 2, D, 16, ctx, kv, qt, D)
+    print("explicit precision", kv, qt, D, flush=True)
+    got = to_host(pa.paged_attention_v3(q[:, 0].to(dev), k.to(dev), v.to(dev), torch.from_numpy(bt).to(dev),
+                                        torch.from_numpy(c).to(dev), D ** -0.5, 64))
+    assert ("decode_mfma32_kernel" if kv == "bf16" else "decode_mfma_kernel") in pa.last_launch(), pa.last_launch()
+    want = attention64(q, k32, v32, bt, c, D ** -0.5)[:, 0]
+    err = float((torch.from_numpy(got).double() - want).norm() / want.norm())
+    print(f"error {err:.2e}", flush=True)
+    assert err < 1e-6, err
+
+
+@pytest.mark.parametrize("qt", ["f32", "bf16"])
+def test_explicit_count_infinities(pa, dev, qt):
+    """Inf in K and V over a bf16 cache reaches the outputs as a chain of fp32
+    products carries it."""
+    q, k, v, bt, c, k32, v32 = case(2, 1, 16, 2, 64, 16, [500, 40], "bf16", qt, 3)
+    for x, x32, b, key, head, dim, val in ((v, v32, 0, 123, 0, 5, float("inf")), (v, v32, 0, 200, 1, 7, float("-inf")),
+                                           (v, v32, 1, 3, 1, 9, float("inf")), (k, k32, 1, 11, 0, 2, float("inf"))):
+        page = int(bt[b, key // 16])
+        x[page, key % 16, head, dim] = val
+        x32[page, key % 16, head, dim] = val
+    print("infinities", qt, flush=True)
+    got = to_host(pa.paged_attention_v3(q[:, 0].to(dev), k.to(dev), v.to(dev), torch.from_numpy(bt).to(dev),
+                                        torch.from_numpy(c).to(dev), 0.125, 64))
+    want = attention64(q, k32, v32, bt, c, 0.125)[:, 0].float().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    assert np.array_equal(got[np.isinf(got)], want[np.isinf(want)])
+    fine = np.isfinite(want)
+    close(got[fine], want[fine])
