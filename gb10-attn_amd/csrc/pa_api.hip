@@ -687,11 +687,15 @@ int run_v3(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const p
                   (maxctx + plan.parts - 1) / plan.parts >= kLongestFirstTokens ? 1 : 0;
   if (!plan.direct) bind_workspace(&a.p, ws, plan);
   // Partitions of the library's own plan on the matrix-core kernel: a batch of
-  // nearly equal contexts that fills the GPU uncut is not cut (part_len).
+  // nearly equal contexts is not cut (part_len) where whole contexts give every
+  // CU the same number of units, but for a sixteenth.  64/8 heads of 128, bf16,
+  // context 8192, cut -> uncut: 256 units on 256 CUs 188 -> 180 us, 480 365 -> 347,
+  // 512 378 -> 362; but 264 214 -> 282, 384 283 -> 315, 448 (heads of 64) 188 -> 194.
   if (phases == kBoth && plan.part_tokens > 0 && a.p.B <= 64 && decode_on_matrix_cores(a.p, a.kv_dtype, a.gc)) {
     int cus = 0;
     if ((rc = device_cu_count(&cus))) return rc;
-    a.p.uniform_whole = (int64_t)a.p.B * a.p.HKV * a.p.head_chunks >= cus ? 1 : 0;
+    const int64_t units = (int64_t)a.p.B * a.p.HKV * a.p.head_chunks, rounds = (units + cus - 1) / cus;
+    a.p.uniform_whole = units >= cus && 16 * units >= 15 * rounds * cus ? 1 : 0;
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (phases & kPartition) {

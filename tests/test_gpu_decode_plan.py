@@ -37,12 +37,14 @@ def test_explicit_count_on_own_plan(pa, dev, B, H, HKV, D, ctx, S, kv):
 
 
 @pytest.mark.parametrize("kv", ["f16", "bf16"])
-@pytest.mark.parametrize("lens", ["equal", "nearly", "ragged", "empty and beyond"])
+@pytest.mark.parametrize("lens", ["equal", "nearly", "ragged", "empty and beyond", "one more"])
 def test_equal_contexts_uncut(pa, dev, kv, lens):
     """A work-group per (sequence, KV head) or more fills the GPU, groups of
-    eight: equal contexts run whole, others in partitions, by the same call."""
+    eight: equal contexts run whole, others in partitions, by the same call; so
+    do equal ones whose units leave a round of the GPU mostly empty.  Partitions
+    write the workspace, whole contexts do not."""
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    HKV, G, D, B = 8, 8, 64, -(-cus // 8)
+    HKV, G, D, B = 8, 8, 64, -(-cus // 8) + (lens == "one more")
     assert B <= 64
     n = np.full(B, 3008)
     if lens == "nearly":
@@ -59,7 +61,9 @@ def test_equal_contexts_uncut(pa, dev, kv, lens):
         ctx[7] = 188 * 16 + 1
         c = torch.from_numpy(ctx).to(dev)
     print("uncut", lens, kv, flush=True)
-    got = to_host(pa.paged_attention_v3(q, k, v, bt, c, 0.125, 0))
+    ws = torch.full((pa.workspace_size(q, k, bt, 0),), 0xA5, dtype=torch.uint8, device=dev)
+    got = to_host(pa.paged_attention_v3(q, k, v, bt, c, 0.125, 0, workspace=ws))
+    assert bool((ws == 0xA5).all()) == (lens in ("equal", "nearly", "empty and beyond"))
     assert "decode_mfma_kernel" in pa.last_launch() and "reduce_kernel" in pa.last_launch(), pa.last_launch()
     if lens == "empty and beyond":
         assert np.all(got[5] == 0.0) and np.isnan(got[7]).all()
