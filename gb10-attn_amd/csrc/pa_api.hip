@@ -390,21 +390,19 @@ int make_plan(const DecodeParams& p, int gc, int kv_bytes, int64_t num_splits, P
   plan->part_tokens = nparts > 1 ? ptok : 0;
   plan->direct = nparts <= 1;
   plan->hp = hp;
-  // A split whose heads can be packed takes as many partitions as bring the
-  // grid of the widest rows to four work-groups per CU, of at least 512 tokens
-  // (1024 of an FP8 cache): wide rows and an even end of the launch both pay
-  // more than the longer partial pass.  bf16, 32/8 heads of 128, contexts
-  // ragged over [256, 8192]: 32 sequences 105 -> 98 us, 16 58 -> 50; 64 equal
-  // contexts of 4096: 190 -> 181.  fp16, 16 heads of 128, 32
-  // sequences of 2048 / 4096: 100 -> 90, 188 -> 171.  Not where 512-token
-  // partitions leave that grid under two per CU (12 heads of 64, 16 sequences
-  // of 4096: 41.2 -> 43.1), nor at 256 tokens (FP8, 32/8 heads, 32 of 2048:
-  // 40.7 -> 42.9).
-  if (nparts > 1 && hi > lo) {
+  // A split of one-head groups of 128 elements and more takes as many partitions
+  // as give every CU four work-groups of the widest rows, of at least 512 tokens
+  // (1024 of an FP8 cache), where they come out even: wide rows and an even end
+  // of the launch both pay more than the longer partial pass.  16 heads of 128,
+  // fp16: 32 sequences of 2048 / 4096 96.2 -> 91.8 us, 181 -> 172; 16 of 8192
+  // 182 -> 171.  Not where the partitions do not divide the CUs (12 heads of 64, 32
+  // sequences of 8192: 127 -> 134), nor for groups of four (32/8 heads of 128, 32
+  // of 4096: 95 -> 100; 8/2 heads, FP8, 131 ragged to 12684: 145 -> 190).
+  if (nparts > 1 && hi > lo && p.G == 1 && p.D >= 128) {
     // (Sq is 1 here; the size query leaves it, and B may be, 0.)
-    const int64_t packed = std::max<int64_t>(1, (int64_t)p.B * (p.HKV / hi) * ((p.G + gc - 1) / gc));
-    const int64_t want = std::min((4 * (int64_t)cus + packed - 1) / packed, maxctx / (kv_bytes == 1 ? 1024 : 512));
-    if (want > nparts && packed * want >= 2 * (int64_t)cus) {
+    const int64_t packed = std::max<int64_t>(1, (int64_t)p.B * (p.HKV / hi)), even = 4 * (int64_t)cus;
+    const int64_t want = even / packed;
+    if (even % packed == 0 && want > nparts && want <= maxctx / (kv_bytes == 1 ? 1024 : 512)) {
       plan->part_tokens = ((maxctx + want - 1) / want + 127) / 128 * 128;
       plan->parts = (maxctx + plan->part_tokens - 1) / plan->part_tokens;
       if (packed * plan->parts >= (int64_t)cus * knobs().wgs_per_cu) plan->hp = hi;

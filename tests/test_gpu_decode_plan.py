@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
     (1, 8, 1, 64, [8192], 16),             # the plan wants more partitions: held to 16
     (3, 8, 8, 128, [3000, 1, 0], 64),      # fewer than asked
     (2, 12, 4, 32, [700, 5000], 17),       # odd group, ragged
-    (16, 16, 16, 64, [4096] * 16, 64),     # packed heads
+    (16, 16, 16, 128, [4096] * 16, 64),    # packed heads
+    (16, 16, 16, 64, [4096] * 16, 64),
     (40, 8, 8, 32, [600] * 40, 8),         # uncut
 ])
 @pytest.mark.parametrize("kv", ["f16", "bf16"])
@@ -154,3 +155,26 @@ def test_explicit_count_infinities(pa, dev, qt):
     assert np.array_equal(got[np.isinf(got)], want[np.isinf(want)])
     fine = np.isfinite(want)
     close(got[fine], want[fine])
+
+
+@pytest.mark.parametrize("B,H,HKV,D,ctx,packed", [
+    (32, 16, 16, 128, 4096, 4), (16, 16, 16, 128, 8192, 8),   # four work-groups of two heads per CU
+    (16, 16, 16, 128, 2048, 0), (32, 12, 12, 64, 8192, 0), (32, 32, 8, 128, 4096, 0), (24, 16, 16, 128, 8192, 0)])
+def test_packed_split_rule(pa, dev, B, H, HKV, D, ctx, packed):
+    """Which splits take the partitions of packed heads (a share of 256 CUs each,
+    evenly); the others are pa_plan_partitions'.  Sizes only: nothing is launched."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    if cus != 256:
+        pytest.skip("sizes chosen for 256 CUs")
+    ptr, MB = torch.empty(64, device=dev).data_ptr(), ctx // 16
+    T = type(pa.view(torch.empty(1)))
+    q = T.make(ptr, 1, (B, H, D), (H * D, D, 1))
+    k = T.make(ptr, 1, (B * MB, 16, HKV, D), (16 * HKV * D, HKV * D, D, 1))
+    bt = T.make(ptr, 4, (B, MB), (MB, 1))
+    size = pa.lib().paged_attention_v3_workspace_size(C.byref(q), C.byref(k), C.byref(bt), 0)
+    tok, n = C.c_int64(), C.c_int64()
+    pa.check(pa.lib().pa_plan_partitions(B, H, HKV, D, ctx, cus, C.byref(tok), C.byref(n)))
+    parts = packed or n.value
+    rows = B * H * parts
+    up = lambda x: (x + 255) // 256 * 256
+    assert size == up(rows * D * 4) + 2 * up(rows * 4), (size / (B * H * (D + 2) * 4), parts)
