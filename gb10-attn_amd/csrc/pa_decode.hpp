@@ -135,12 +135,14 @@ using DecodeShapeOf = DecodeShape<KV, D * HP, (GC == 1 && HP == 1) ? 2 : 0>;
 // heads two (above); the FP8 group of four at D = 128 packed two KV heads
 // to a work-group three, which it fits with one spilled register outside
 // the loop (170 registers otherwise: FP8 config 3 4550 -> 4753 GB/s); groups of
-// two three, left to itself the allocator has tipped bf16 caches with fp32 q into
-// two (12/6 heads of 64, 8 sequences of 2048: 15.2 -> 19.2 us); larger groups one.
+// two three, and four over FP8, left to itself the allocator has tipped bf16 caches
+// with fp32 q into two (12/6 heads of 64, 8 sequences of 2048: 15.2 -> 19.2 us) and
+// FP8 into three (128 ragged to 8192 at 16 splits: 159 -> 179); larger groups one.
 template <typename KV, int D, int GC, int HP, int DQ>
 constexpr int decode_waves_per_eu() {
   if (GC > 4) return 1;
   if (KV::kCode == kFP8 && GC == 4 && HP == 2 && D == 128 && DQ != 0) return 3;
+  if (GC == 2 && KV::kCode == kFP8 && DQ != 0) return 4;
   if (GC == 2 && D <= 128 && KV::kCode != kFP8) return 3;
   return 2;
 }
