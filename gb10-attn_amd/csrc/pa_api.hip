@@ -436,24 +436,35 @@ int plan_varlen_decode(const DecodeParams& p, int gc, int kv_bytes, Plan* plan) 
 // reference's chooser asks for 16 to 64 at 512 tokens and more; one query head
 // per KV head from 8, with rows of 1 KB from 4) it runs the library's own plan,
 // with no more partitions than the caller's count, whose workspace has been
-// checked.  64 partitions asked for, fp16
-// cache, 12 heads of 64: one sequence of 2048 tokens 16.4 -> 10.7 us, 16 of
-// them 26.1 -> 24.6 (the partition grids each paid a start-up per 32 tokens);
-// bf16, 32/8 heads of 128, 32 of 2048: 67.4 -> 57.8; 64/8 heads, 32 of 4096:
-// 177 -> 110 (the explicit partitions kept it off the matrix-core kernel).
-// The library's plan ran no slower at any of 25 batch and context sizes of
-// six head counts, but for 7 within 15 % where its own plan is not the best.
-bool own_plan_pays(const DecodeArgs& a, int64_t num_splits) {
-  const int64_t from = a.gc > 1 ? 16 : a.p.D * dtype_bytes(a.kv_dtype) < 1024 ? 8 : 4;
-  return num_splits >= from;
-}
-int own_plan(const DecodeArgs& a, int64_t num_splits, Plan* plan) {
+// checked, where that is faster than the caller's.  Own plan against explicit
+// partitions (of `chunk` tokens), the reference's counts:
+//  * Groups of eight over 16-bit caches, on the matrix cores: 1.4 to 5 times as
+//    fast at every size (64/8 heads of 128, 32 of 4096: 181 -> 96 us).
+//  * One-head groups whose uncut units fill the GPU, where the partitions of a unit
+//    are one work-group's slots (rounds of them, up to 4080 tokens): uncut, or
+//    split with packed heads (12 heads of 64, 64 of 512: 1.22).  Without packed
+//    heads the split loses to uncut (16 heads of 128, 16 of 2048: 52 and 46 us).
+//  * Larger groups whose units fill the GPU, uncut or in the compacted grid (up to
+//    64 sequences): 1.05 to 1.4 at chunks of up to 64 tokens (groups of eight over
+//    FP8: 32), down to 0.8 past that (16/4 heads of 64, 32 of 4096 at 16: 33 and 40 us).
+//  * Fewer units from 1024 tokens on, where the partitions leave half of the CUs
+//    idle (three quarters where they pack heads, seven eighths in groups of eight):
+//    1.05 to 2.7 (12 heads of 64, one of 2048: 16.4 -> 10.7 us).  With more work-
+//    groups than that down to 0.68 (8/1 heads, FP8, 64 of 4096: 48 and 71 us), for
+//    nearly a full GPU 0.8 to 1.05 (16 heads of 64, 13 of 4096: 44 and 55; 12 heads,
+//    16 of 2048 25.6 and 24.7, ragged 19.2 and 21.4), and not where the own plan is
+//    uncut (16 heads of 128, 4 of 512: 12.1 and 14.0).
+int own_plan(const DecodeArgs& a, int64_t num_splits, int cus, Plan* plan, bool* pays) {
+  const int kvb = dtype_bytes(a.kv_dtype);
+  const DecodeParams& p = a.p;
+  const int64_t maxctx = (int64_t)p.MB * p.BS, chunk = (maxctx + num_splits - 1) / num_splits;
+  *pays = false;
+  if (num_splits < (a.gc > 1 ? 16 : p.D * kvb < 1024 ? 8 : 4)) return PA_OK;
   Plan own;
   int rc;
-  if ((rc = make_plan(a.p, a.gc, dtype_bytes(a.kv_dtype), 0, &own))) return rc;
+  if ((rc = make_plan(p, a.gc, kvb, 0, &own))) return rc;
   if (own.parts > num_splits) {  // as many whole 128-token steps as keep within num_splits
-    const int64_t maxctx = (int64_t)a.p.MB * a.p.BS;
-    own.part_tokens = ((maxctx + num_splits - 1) / num_splits + 127) / 128 * 128;
+    own.part_tokens = (chunk + 127) / 128 * 128;
     own.parts = (maxctx + own.part_tokens - 1) / own.part_tokens;
     if (own.parts <= 1) {
       own.parts = 1;
@@ -461,7 +472,42 @@ int own_plan(const DecodeArgs& a, int64_t num_splits, Plan* plan) {
       own.direct = true;
     }
   }
-  *plan = own;
+  DecodeParams d = p;
+  d.parts = (int)own.parts;
+  d.part_tokens = (int)own.part_tokens;
+  if (decode_on_matrix_cores(d, a.kv_dtype, a.gc)) {
+    *pays = true;
+    *plan = own;
+    return PA_OK;
+  }
+  // Partitions a work-group serves at hp packed heads in the slot mode, and whether
+  // the pages of n of them fit its block-table stage.
+  auto slots = [&](int64_t hp) {
+    const int64_t lanes = (int64_t)p.D * hp * kvb / (kvb == 1 ? 8 : 16);
+    return kDecodeWaves * (lanes >= 64 ? 1 : 64 / lanes);
+  };
+  auto fit = [&](int64_t n) { return (n * chunk + p.BS - 1) / p.BS + 1 <= kBtChunk; };
+  const int64_t heads = (int64_t)p.B * p.head_chunks * p.HKV;
+  const int lo = decode_pack_min(p.D, kvb, p.G, p.HKV, p.k_sh);
+  const int64_t units = heads / lo;
+  if (a.gc == 1 && units >= cus) {
+    const int hp = pack_for(p, kvb, 1, cus);
+    const int64_t n = slots(hp), rounds = (num_splits + n - 1) / n;
+    *pays = chunk <= kWavePartTokens && heads / hp >= cus && num_splits >= n && rounds <= 8 && fit(rounds * n);
+    if (!own.direct && own.hp <= lo) {
+      own.parts = 1;
+      own.part_tokens = 0;
+      own.direct = true;
+    }
+  } else if (units >= cus) {
+    *pays = (own.direct || p.B <= 64) && chunk <= (a.gc < 8 ? 64 : 32);
+  } else if (!own.direct && chunk <= 128 && maxctx >= 1024) {
+    const int hp = pack_for(p, kvb, num_splits, cus);
+    const int64_t n = num_splits >= slots(hp) && fit(slots(hp)) ? slots(hp) : kDecodeWaves;
+    const int64_t wgs = heads / hp * ((num_splits + n - 1) / n);
+    *pays = a.gc >= 8 ? 8 * wgs <= cus : hp > 1 ? 4 * wgs <= cus : 2 * wgs < cus;
+  }
+  if (*pays) *plan = own;
   return PA_OK;
 }
 
@@ -658,9 +704,11 @@ int run_v3(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k, const p
     return fail(PA_ERR_WORKSPACE, "workspace too small: need %zu bytes, got %zu", need, ws ? ws_bytes : 0);
   if (need > 0 && (reinterpret_cast<uintptr_t>(ws) & 255) != 0)
     return fail(PA_ERR_WORKSPACE, "workspace must be 256-byte aligned");
-  if (phases == kBoth && own_plan_pays(a, num_splits)) {
-    if ((rc = own_plan(a, num_splits, &plan))) return rc;
-    a.p.fp32_weights = 1;  // as the explicit partitions' kernel
+  if (phases == kBoth && num_splits > 1) {
+    int cus = 0;
+    bool own = false;
+    if ((rc = device_cu_count(&cus)) || (rc = own_plan(a, num_splits, cus, &plan, &own))) return rc;
+    a.p.fp32_weights = own ? 1 : 0;  // as the explicit partitions' kernel
   }
   a.p.parts = (int)plan.parts;
   a.p.part_tokens = (int)plan.part_tokens;

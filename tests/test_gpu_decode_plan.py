@@ -178,3 +178,43 @@ def test_packed_split_rule(pa, dev, B, H, HKV, D, ctx, packed):
     rows = B * H * parts
     up = lambda x: (x + 255) // 256 * 256
     assert size == up(rows * D * 4) + 2 * up(rows * 4), (size / (B * H * (D + 2) * 4), parts)
+
+
+@pytest.mark.parametrize("kv,B,H,HKV,D,ctx,S,own", [
+    ("f16", 1, 12, 12, 64, 2048, 64, True),     # a few units
+    ("f16", 16, 12, 12, 64, 2048, 64, False),   # nearly a full GPU
+    ("f16", 64, 12, 12, 64, 512, 16, False),    # (16 partitions: half of a work-group's slots)
+    ("f16", 64, 12, 12, 64, 512, 64, True),     # rounds of slots, uncut
+    ("f16", 64, 12, 12, 64, 4096, 64, False),   # more pages than a work-group stages
+    ("f16", 4, 16, 16, 128, 512, 32, False),    # uncut, but a few units
+    ("f16", 32, 32, 8, 128, 1024, 32, True),    # groups of four that fill the GPU
+    ("f16", 32, 32, 8, 128, 2048, 16, False),   # chunks of 128 tokens
+    ("fp8", 8, 64, 8, 128, 1024, 32, False),    # groups of eight on the vector kernel
+    ("bf16", 8, 64, 8, 128, 1024, 32, True)])   # and on the matrix cores
+def test_explicit_count_route(pa, dev, kv, B, H, HKV, D, ctx, S, own):
+    """Which explicit counts run the library's plan: the caller's own partitions
+    write their partial sums to the end of the workspace.  Both are the attention
+    of the same rows."""
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("sizes chosen for 256 CUs")
+    MB = ctx // 16
+    g = torch.Generator(device=dev).manual_seed(1)
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16, "fp8": torch.float8_e4m3fn}[kv]
+    q = torch.randn((B, H, D), device=dev, generator=g).half() if kv != "bf16" else torch.randn(
+        (B, H, D), device=dev, generator=g).bfloat16()
+    k, v = (torch.randn((B * MB, 16, HKV, D), device=dev, generator=g).half().to(dt) for _ in range(2))
+    bt = torch.randperm(B * MB, device=dev, generator=g).int().view(B, MB)
+    c = torch.full((B,), ctx, dtype=torch.int32, device=dev)
+    need = pa.workspace_size(q, k, bt, S)
+    ws = torch.full((need,), 0xA5, dtype=torch.uint8, device=dev)
+    rows = B * H * S
+    last = (rows * D * 4 + 255) // 256 * 256 + (rows * 4 + 255) // 256 * 256 + rows * 4 - 4
+    print("route", kv, B, H, HKV, D, ctx, S, flush=True)
+    got = pa.paged_attention_v3(q, k, v, bt, c, 0.1, S, workspace=ws)
+    assert bool((ws[last:last + 4] == 0xA5).all()) == own, pa.last_launch()
+    want = torch.empty_like(got)
+    V = [pa.view(t) for t in (want, q, k, v, bt, c)]
+    st = torch.cuda.current_stream().cuda_stream
+    pa.check(pa.lib().pa_v3_partition(*[C.byref(x) for x in V], 0.1, S, ws.data_ptr(), need, st))
+    pa.check(pa.lib().pa_v3_reduce(*[C.byref(V[i]) for i in (0, 1, 2, 4, 5)], S, ws.data_ptr(), need, st))
+    close(to_host(got), to_host(want))
