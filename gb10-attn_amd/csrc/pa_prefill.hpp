@@ -209,6 +209,19 @@ __device__ inline int swv(int row, int cc) {
   return row * D + (vpos<D>(row, cc) << 3);
 }
 
+// The i-th head group that sequence b's work-groups take.  Pairs reach the 8 XCDs
+// round robin, so with eight packed KV heads each XCD kept to one of them: its K and
+// V rows lie a whole token row apart and share few of the L2's channels.  The heads'
+// order therefore moves on with the sequence.  8-wave kernel, fp16, 64/8 heads of
+// 128, one block per query head before packing -> packed in a fixed order -> this:
+// 8 prompts of 256 rows 42 -> 58 -> 36 us, 16 prompts 80 -> 104 -> 69 us; 32/8 heads,
+// 16 prompts of 512 rows 94 -> 96 -> 83 us.
+__device__ __forceinline__ int pf_turn(const PrefillParams& p, int b, int i) {
+  if (p.gp == 1) return i;
+  i += (int)(((uint32_t)b * (uint32_t)p.HG >> 3) % (uint32_t)p.HG);
+  return i >= p.HG ? i - p.HG : i;
+}
+
 // Work-group x -> partition (context split, the slow index) and unit (b, head
 // group, block of QB packed rows); false past the last unit of a compacted
 // grid (work-group uniform).
@@ -290,8 +303,8 @@ __device__ __forceinline__ bool pf_unit(const PrefillParams& p, int64_t x, int l
     }
     if (fb < 0) return false;
     qt = ft;
-    hg = fh;
     b = fb;
+    hg = pf_turn(p, b, fh);
   } else {
     if constexpr (kPart) {
       part = (int)(x / p.units);
@@ -304,8 +317,8 @@ __device__ __forceinline__ bool pf_unit(const PrefillParams& p, int64_t x, int l
     }
     qt = nq - 1 - (int)(x / nbh);
     const int64_t bh = x % nbh;
-    hg = (int)(bh % p.HG);
     b = (int)(bh / p.HG);
+    hg = pf_turn(p, b, (int)(bh % p.HG));
   }
   return true;
 }
@@ -1234,8 +1247,8 @@ void prefill_pp_kernel(const PrefillParams p) {
   }
   const int qt = nq - 1 - (int)(x / nbh);
   const int64_t bh = x % nbh;
-  const int hg = (int)(bh % p.HG);
   const int b = (int)(bh / p.HG);
+  const int hg = pf_turn(p, b, (int)(bh % p.HG));
   const int h0 = hg * p.gp;  // first query head of the unit
   const int kvh = h0 / p.G;
 

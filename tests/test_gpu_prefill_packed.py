@@ -55,3 +55,22 @@ def test_packed_rows_varlen(pa, dev):
             want = oracle.prefill(q[None, cu[b]:cu[b + 1]], inp["k"], inp["v"], inp["bt"][b:b + 1], inp["ctx"][b:b + 1],
                                   0.125, "f16")[0]
             close(got[cu[b]:cu[b + 1]], want)
+
+
+@pytest.mark.parametrize("HKV", [3, 8])
+@pytest.mark.parametrize("rows,ctx", [(65, 70), (16, 1500)])
+def test_packed_heads_turn(pa, dev, HKV, rows, ctx):
+    """The order of a sequence's packed heads moves on with the sequence: every
+    sequence and head is served once, in a uniform and a variable-length batch
+    that wrap around the heads, also where contexts are split (16 rows)."""
+    G, D, B = 4, 32, 11
+    inp = prefill_case(B, rows, HKV * G, HKV, D, 16, [ctx + 3 * b for b in range(B)], seed=HKV + rows, kv="f16", qt="f16")
+    want = want_of(inp, 0.2)
+    args = dev_args(inp, dev)
+    print("heads turn", HKV, rows, ctx, flush=True)
+    close(to_host(pa.paged_attention_prefill_wmma(*args, 0.2)), want)
+    close(to_host(pa.paged_attention_prefill(*args, 0.2)), want)
+    cu = torch.arange(B + 1, dtype=torch.int32, device=dev) * rows
+    q, *rest = args
+    got = pa.paged_attention_prefill_varlen(q.reshape(B * rows, HKV * G, D), *rest, cu, rows, 0.2)
+    close(to_host(got).reshape(want.shape), want)
