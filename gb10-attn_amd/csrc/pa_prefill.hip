@@ -36,12 +36,17 @@ static hipError_t launch_pp(const PrefillParams& p, hipStream_t stream) {
 // (the reference's 512-token chunk at context 2048: 192 work-groups, +19 %).
 // Above that, twice the tiles cost more than the shorter chains save
 // (config 4a, 768 work-groups: -17 %).
-// The choice counts the work-groups that have rows to serve: a uniform
-// batch's B * ceil(S / rows) per head; a variable-length batch brings T rows
-// in all (its grid is sized by the longest sequence, and the work-groups past
-// a sequence's rows exit at once), so about ceil(T / rows) of its blocks carry
-// work.  (A mixed batch of 64 decode rows and four 256-row chunks had taken
-// the 8-wave kernel for its 816-block grid: 48 blocks with rows, on 256 CUs.)
+// The choice counts the blocks that have rows to serve as if each query head had
+// its own: a uniform batch's B * ceil(S / rows) per head; a variable-length batch
+// brings T rows in all (its grid is sized by the longest sequence, and the
+// work-groups past a sequence's rows exit at once), so about ceil(T / rows) of its
+// blocks carry work.  (A mixed batch of 64 decode rows and four 256-row chunks had
+// taken the 8-wave kernel for its 816-block grid: 48 blocks with rows, on 256 CUs.)
+// A group's heads are packed into shared blocks, so where the rows of a head do not
+// fill a block the launch has fewer of them, down to count / gp.  fp16, 64/8 heads
+// of 128, one block per query head -> packed, 8-wave / 4-wave: 16 prompts of 32 rows
+// 32 -> 14.4 / 11.4 us (64 blocks), of 64 rows at 564 tokens 78 -> 33.3 / 33.7 us,
+// of 128 rows 46 -> 33.8 / 29.4 us; 4 prompts of 512 rows 49 -> 40 / 42 us.
 template <typename KV, int D>
 static hipError_t launch_pf(const PrefillParams& p, hipStream_t stream) {
   if constexpr (PfShape<D>::MT == 2) {
@@ -55,9 +60,9 @@ static hipError_t launch_pf(const PrefillParams& p, hipStream_t stream) {
     const int64_t plain = busy(PfShape<D>::QB);
     if ((cus > 0 && plain < cus) || (!p.cu_q && (int64_t)p.S * p.gp <= 64))
       return p.q_split ? launch_pf_q<KV, D, true, true>(p, stream) : launch_pf_q<KV, D, false, true>(p, stream);
-    // The 8-wave kernel (one work-group per CU) for grids of at least two
-    // of its work-groups per CU; below that its 256-row blocks leave CUs
-    // idle at the end of the launch (config 4a: 384 work-groups, -20 %).
+    // The 8-wave kernel (one work-group per CU) from two of its blocks per CU on;
+    // with fewer and one head to a block its 256-row blocks leave CUs idle at the
+    // end of the launch (config 4a: 384 work-groups, -20 %).
     if constexpr (KV::kCode == kF16 || KV::kCode == kBF16 || KV::kCode == kFP8) {
       const int64_t pp_units = busy(kPpRows);
       if (!p.q_split && p.MB <= kPfBtStage && cus > 0 && pp_units >= 2 * cus) return launch_pp<KV, D>(p, stream);
