@@ -607,13 +607,22 @@ PrefillParams prefill_params(const DecodeArgs& a, const int32_t* cu, int64_t T, 
 // FP8 and ungrouped fp16 caches, a 16-byte aligned q); else it runs as a decode problem per
 // query row.  It does when its context split is planned, when those decode
 // problems are kPrefill32Units work-groups or more, and for several rows of
-// groups of eight heads (whose decode problems run on the vector ALU).
+// groups of eight heads (whose decode problems run on the vector ALU), with these
+// exceptions, where a decode problem is short or a matrix block long.  Below 256
+// tokens the count is of query rows and grows with D (a block's setup and its
+// masked keys weigh more than the few keys of a row); D = 256 splits only from
+// 1024 tokens or 512 work-groups on; and at D = 128 over a bf16 cache q in three
+// pieces spills registers in the split kernel, so one to three rows take it only
+// where its grid is small.
 // Measured, decode kernel against matrix kernel, fp32 q: 12 heads of 64, one
 // row at context 4096 (split) 36.8 vs 14.9 us, at 512 8.7 vs 13.1; eight
 // sequences of 4 / 8 / 16 rows at 512 (384 / 768 / 1536 units) 14.2 vs 14.4,
 // 20.2 vs 14.4, 25.0 vs 14.6; 32/8 heads of 128, eight sequences of 8 / 16
 // rows (512 / 1024 units) 21.7 vs 22.0, 39.2 vs 23.5; 8/1 heads, two rows at
-// 64 / 512: 13.3 vs 10.5, 29.2 vs 20.3.
+// 64 / 512: 13.3 vs 10.5, 29.2 vs 20.3.  The exceptions: 8 heads of 256, 128 rows
+// at 128 14.7 vs 28.6, four sequences of 32 at 32 10.5 vs 17.9, one to four rows
+// at 513 (split) 20-25 vs 27-33; 16 heads of 128, eight sequences of 8 rows at 8
+// 8.7 vs 12.7; over bf16, eight rows of 1 / 2 at 4096 (split) 80 vs 125, 90 vs 125.
 constexpr int64_t kPrefill32Units = 768;
 // Groups over fp16 caches keep the decode kernel: its packed P.V carries their
 // weights as fp16 pairs (1.3e-4 from 64 bits; the matrix kernel 1.7e-7), and the
@@ -623,8 +632,19 @@ bool prefill32_eligible(const DecodeArgs& a, const pa_tensor_t* q) {
   return prefill_kv(a.kv_dtype) && !(a.kv_dtype == kF16 && a.gc > 1) && aligned16(q->data);
 }
 bool prefill32_pays(const DecodeArgs& a, const PrefillParams& pp) {
-  return pp.parts > 1 || (a.gc >= 8 && a.p.Sq > 1) ||
-         (int64_t)a.p.B * a.p.Sq * a.p.HKV * a.p.head_chunks >= kPrefill32Units;
+  const int64_t units = (int64_t)a.p.B * a.p.Sq * a.p.HKV * a.p.head_chunks;
+  const int64_t maxctx = (int64_t)a.p.MB * a.p.BS;
+  if (pp.parts > 1) {
+    if (a.p.D == 256 && maxctx < 1024 && units < 512) return false;
+    if (a.kv_dtype == kBF16 && pp.q_dtype != kBF16 && a.p.D == 128 && a.p.Sq < 4) {
+      const int QB = pf_split_rows(a.p.D);
+      return (int64_t)pp.B * pp.HG * (((int64_t)pp.S * pp.gp + QB - 1) / QB) <= 32;
+    }
+    return true;
+  }
+  if (a.gc >= 8 && a.p.Sq > 1 && maxctx >= 64) return true;
+  if (maxctx >= 256) return units >= kPrefill32Units;
+  return (int64_t)a.p.B * a.p.Sq * a.p.H >= std::min<int64_t>(24 * a.p.D, 4096);
 }
 
 // One direct decode launch (one partition per sequence): v1, v2 and the

@@ -74,7 +74,9 @@ def close64(got, want):
 @pytest.mark.parametrize("D", [32, 64, 128, 256])
 def test_prefill32(pa, dev, kv, qt, D):
     """Edges of the 32/64/128-row blocks and 32/64-key tiles; chunked, padded
-    and empty sequences; both grid modes; page sizes that do not divide a tile."""
+    and empty sequences; both grid modes; page sizes that do not divide a tile.
+    Short contexts take the matrix kernel from a number of rows that grows with D."""
+    n = {32: 1, 64: 2, 128: 4, 256: 6}[D]
     for i, (B, S, H, HKV, BS, ctx, scale) in enumerate([
             (3, 64, 8, 4, 16, [64, 160, 20], 1 / np.sqrt(D)), (2, 65, 6, 6, 5, [129, 64], -0.2),
             (1, 129, 6, 6, 32, [129], 0.3), (2, 97, 8, 4, 16, [127, 0], 0.0), (2, 3, 16, 2, 16, [63, 31], 0.1)]):
@@ -82,7 +84,7 @@ def test_prefill32(pa, dev, kv, qt, D):
         HKV = H if kv == "f16" else HKV  # (groups over fp16 caches run on the decode kernel)
         S = max(S, 65) if kv == "f16" and i == 4 else S  # (three rows of ungrouped heads too)
         ctx = [max(n, S - 2) for n in ctx] if kv == "f16" and i == 4 else ctx
-        q, k, v, bt, c, k32, v32 = case(B, S, H, HKV, D, BS, ctx, kv, qt, D + i)
+        q, k, v, bt, c, k32, v32 = case(B * n, S, H, HKV, D, BS, ctx * n, kv, qt, D + i)
         got = run(pa, dev, q, k, v, bt, c, scale)
         assert "prefill32_kernel" in pa.last_launch(), pa.last_launch()
         close64(got, attention64(q, k32, v32, bt, c, scale))
@@ -126,7 +128,7 @@ def test_key_split_bound(pa, dev, fn, D, qt, per_cu, over):
 def test_prefill32_q_range(pa, dev):
     """Rows of very large and very small q (the fp16 pieces are scaled by row)
     and rows that mix both; output types."""
-    q, k, v, bt, c, k32, v32 = case(1, 72, 12, 12, 64, 16, [100], "f16", "f32", 9)
+    q, k, v, bt, c, k32, v32 = case(2, 72, 12, 12, 64, 16, [100, 81], "f16", "f32", 9)
     q[0, :10] *= 1e-30
     q[0, 10:20] *= 300.0
     q[0, 20:30, :, ::2] *= 1e-5
@@ -134,6 +136,7 @@ def test_prefill32_q_range(pa, dev):
     print("q range", flush=True)
     want = attention64(q, k32, v32, bt, c, 0.01)
     close64(run(pa, dev, q, k, v, bt, c, 0.01), want)
+    assert "prefill32_kernel" in pa.last_launch(), pa.last_launch()
     for ot, tol in ((torch.float16, 2 ** -11), (torch.bfloat16, 2 ** -8)):
         got = run(pa, dev, q, k, v, bt, c, 0.01, out_dtype=ot)
         assert float((torch.from_numpy(got).double() - want).norm() / want.norm()) < tol
@@ -144,7 +147,7 @@ def test_prefill32_non_finite(pa, dev, kv):
     """Inf and NaN reach exactly the rows that attend them (a masked key's V is
     not multiplied into earlier rows), with the value a chain of fp32 products
     gives; an invalid block id poisons the rows that read its page."""
-    B, S, H, D, BS, ctx = 1, 100, 8, 64, 16, [150]
+    B, S, H, D, BS, ctx = 1, 100, 16, 64, 16, [150]
     q, k, v, bt, c, k32, v32 = case(B, S, H, H, D, BS, ctx, kv, "f32", 21)
 
     def put(x, x32, key, head, dim, val):
@@ -161,6 +164,7 @@ def test_prefill32_non_finite(pa, dev, kv):
     put(k, k32, 140, 1, 9, float("-inf"))
     print("non-finite", kv, flush=True)
     close64(run(pa, dev, q, k, v, bt, c, 0.125), attention64(q, k32, v32, bt, c, 0.125))
+    assert "prefill32_kernel" in pa.last_launch(), pa.last_launch()
     bad = bt.copy()
     bad[0, 5] = 10 ** 6  # keys 80..95: rows whose own keys include one of them
     got = run(pa, dev, q, k, v, bad, c, 0.125)
@@ -195,3 +199,20 @@ def test_prefill32_split_non_finite(pa, dev, kv, D):
     want = attention64(q, k32, v32, bt, c, 0.125)
     for h in range(H):
         close64(got[:, :, h], want[:, :, h])
+
+
+@pytest.mark.parametrize("D,kv,H,B,S,ctx,matrix", [
+    (256, "bf16", 8, 1, 128, 128, False), (256, "bf16", 8, 4, 128, 128, True), (64, "bf16", 12, 1, 127, 127, False),
+    (64, "bf16", 12, 1, 128, 128, True), (256, "f16", 8, 1, 3, 900, False), (256, "f16", 8, 1, 3, 1100, True),
+    (128, "bf16", 16, 8, 2, 4096, False), (128, "bf16", 16, 2, 2, 4096, True), (128, "bf16", 16, 8, 4, 4096, True),
+    (128, "fp8", 16, 8, 2, 4096, True)])
+def test_prefill32_rule(pa, dev, D, kv, H, B, S, ctx, matrix):
+    """Short contexts, D = 256 and three-piece splits take the matrix kernel only
+    where it is the faster one; both sides of each bound against 64 bits."""
+    q, k, v, bt, c, k32, v32 = case(B, S, H, H, D, 16, [ctx] * B, kv, "f32", D + ctx)
+    print("prefill32 rule", D, kv, H, B, S, ctx, flush=True)
+    got = run(pa, dev, q, k, v, bt, c, 0.1)
+    assert ("prefill32" in pa.last_launch()) == matrix, pa.last_launch()
+    for h in (0, H - 1):
+        one = slice(h, h + 1)
+        close64(got[:, :, one], attention64(q[:, :, one].contiguous(), k32[:, :, one], v32[:, :, one], bt, c, 0.1))
