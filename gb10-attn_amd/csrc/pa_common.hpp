@@ -150,8 +150,12 @@ inline int64_t pf_compact_units(const PrefillParams& p, int QB) {
 // 0.86, D = 128 1.3), two take 1.25-1.35 times that between them, and a third
 // or fourth adds nothing: so a grid is brought to at most two work-groups per
 // CU, and only where the shorter chains save more than the second launch and
-// the partial sums cost (5-7 us; a variable-length
-// batch, whose grid holds idle work-groups, 12).  B = 1, S = 16, context 12288: 12 heads of
+// the partial sums cost (5-7 us; a variable-length batch, whose grid holds idle
+// work-groups and whose prompts may be shorter than its longest context, 12, and 20
+// where the partitions outnumber the CUs: 90 decode rows and six chunks of 128 at
+// context 1024, fp16, unsplit / split: 8/1 heads of 128 71 / 78 us, 8/2 heads
+// 51 / 56; at 4096 217 / 143 and 156 / 118).  The times are those of 16-bit weights;
+// fp32 weights and the 32-key tiles of D = 256 take longer.  B = 1, S = 16, context 12288: 12 heads of
 // 64 150 -> 20 us, 32/8 heads of 128 242 -> 27 us; B = 1, S = 64, context
 // 1024: 17.5 -> 12.5 and 27.8 -> 15.7; B = 1, S = 512, context 8192, 32/8
 // heads (256 blocks, two partitions): 161 -> 111.  Without the two bounds
@@ -173,7 +177,7 @@ inline size_t plan_prefill_split(PrefillParams& p, bool varlen, int cus) {
   int64_t n = 2 * (int64_t)cus / busy;
   if (n > key_tiles / kPfMinPartTiles) n = key_tiles / kPfMinPartTiles;
   const double tile_us = p.D <= 64 ? 0.86 : 1.3;
-  if (n < 2 || (double)key_tiles * tile_us * (1.0 - 1.35 / (double)n) < (varlen ? 12.0 : 7.0)) return 0;
+  if (n < 2 || (double)key_tiles * tile_us * (1.0 - 1.35 / (double)n) < (varlen ? (n * busy > cus ? 20.0 : 12.0) : 7.0)) return 0;
   p.part_tiles = (int32_t)((key_tiles + n - 1) / n);
   p.parts = (int32_t)((key_tiles + p.part_tiles - 1) / p.part_tiles);
   return (size_t)units * p.parts * QB * (p.D + 2) * 4;

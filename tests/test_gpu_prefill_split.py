@@ -120,3 +120,23 @@ def test_varlen_split_overlapping_ranges(pa, dev):
     want = oracle.prefill(q[None], inp["k"], inp["v"], inp["bt"], inp["ctx"], 0.125, "f16")[0]
     close(got[128:], want[128:])
     assert np.all(got[:128] == 7.0)
+
+
+@pytest.mark.parametrize("npf,mb,split", [(6, 64, False), (6, 128, True), (2, 64, True)])
+def test_varlen_split_rule(pa, dev, npf, mb, split):
+    """A variable-length batch whose partitions outnumber the CUs splits only from
+    longer contexts on; every sequence against the oracle."""
+    HKV, G, D, S = 2, 4, 128, 128
+    lens = [1] * 4 + [S] * npf
+    ctx = [33, 7, 64, 1] + [mb * 16 - 5 * i for i in range(npf)]
+    inp = oracle.paged_inputs(len(lens), 1, HKV, D, 16, ctx, seed=9, kv_dtype="f16")
+    q = oracle.quantize(np.random.default_rng(9).standard_normal((sum(lens), G * HKV, D), dtype=np.float32), "f16")
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    print("varlen split rule", npf, mb, flush=True)
+    got = to_host(pa.paged_attention_prefill_varlen(
+        to_dev(q, "f16", dev), to_dev(inp["k"], "f16", dev), to_dev(inp["v"], "f16", dev),
+        torch.from_numpy(inp["bt"]).to(dev), torch.from_numpy(inp["ctx"]).to(dev), torch.from_numpy(cu).to(dev), S, 0.1))
+    assert ("prefill_reduce_kernel" in pa.last_launch()) == split, pa.last_launch()
+    for b in range(len(lens)):
+        close(got[cu[b]:cu[b + 1]], oracle.prefill(q[None, cu[b]:cu[b + 1]], inp["k"], inp["v"], inp["bt"][b:b + 1],
+                                                   inp["ctx"][b:b + 1], 0.1, "f16")[0])
