@@ -418,12 +418,16 @@ int make_plan(const DecodeParams& p, int gc, int kv_bytes, int64_t num_splits, P
 // row and one 64-row chunk at context 8000 292 -> 55 us (decode and prefill
 // split), eight rows and three chunks of ragged contexts to 4000 98 -> 68;
 // sixteen rows and two 512-row chunks at 2048, below the bound, 102 -> 106.
+// Not in groups of eight whose units fill the GPU: these rows run on the vector
+// ALU, and cut contexts took 0.72 to 0.96 of the speed of whole ones over ragged
+// contexts to 8192 (64/8 heads of 128, FP8, 78 rows and two chunks of 512: 584 and
+// 811 us; fp16, 59 rows: 649 and 727), 0.88 to 1.24 over equal ones.
 int plan_varlen_decode(const DecodeParams& p, int gc, int kv_bytes, Plan* plan) {
   int cus = 0, rc;
   if ((rc = make_plan(p, gc, kv_bytes, 0, plan)) || plan->direct) return rc;
   if ((rc = device_cu_count(&cus))) return rc;
   const double rows = (double)p.MB * p.BS * p.D / 64.0, units = (double)p.B * p.HKV * ((p.G + gc - 1) / gc);
-  if (rows * rows * cus < 8.0 * (double)knobs().split_pay * units) {
+  if (rows * rows * cus < 8.0 * (double)knobs().split_pay * units || (gc >= 8 && units >= cus)) {
     plan->parts = 1;
     plan->part_tokens = 0;
     plan->direct = true;
