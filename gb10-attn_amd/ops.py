@@ -63,13 +63,84 @@ def _out(q, out_dtype, out):
 
 # The calls go through libpagedattn_torch.so (csrc/torch_ext.cpp), which builds
 # the C-ABI's tensor views, checks and scratch natively: a tiny decode took
-# 25 us of host time through ctypes and 6 through it.
+# 25 us of host time through ctypes and 6 through it.  Where only libpagedattn.so
+# was built, the same three calls go to it through ctypes.
+def _prep(q, k_cache, v_cache, block_tables, context_lens, qdim, what):
+    if q.dim() != qdim:
+        raise RuntimeError(f"q must be {what}")
+    if k_cache.dim() != 4:
+        raise RuntimeError("k_cache must be [NB, BS, H, D]")
+    # Strided K/V views are read in place; anything the kernels cannot
+    # address directly is made contiguous, as the reference does for all inputs.
+    return (q.contiguous(), k_cache if _kv_ok(k_cache) else k_cache.contiguous(),
+            v_cache if _kv_ok(v_cache) else v_cache.contiguous(),
+            block_tables.to(q.device, torch.int32).contiguous(), context_lens.to(q.device, torch.int32).contiguous())
+
+
+def _stream(dev: torch.device) -> int:
+    return torch.cuda.current_stream(dev).cuda_stream
+
+
+def _scratch(nbytes, dev):
+    if nbytes == C.c_size_t(-1).value:
+        raise RuntimeError(last_error())
+    return torch.empty(nbytes, dtype=torch.uint8, device=dev)  # (the allocator aligns to 512 bytes)
+
+
+class _CAbi:
+    @staticmethod
+    def decode_out(version, q, k_cache, v_cache, block_tables, context_lens, scale, num_splits, k_scale, v_scale, out,
+                   workspace):
+        args = _prep(q, k_cache, v_cache, block_tables, context_lens, 3, "[B, H, D]")
+        q, k, _, bt, _ = args
+        six = [C.byref(view(t)) for t in (out, *args)]
+        with torch.cuda.device(q.device):
+            if version < 3:
+                check((lib().paged_attention if version == 1 else lib().paged_attention_v2)(*six, scale,
+                                                                                          _stream(q.device)))
+                return
+            need = lib().paged_attention_v3_workspace_size(six[1], six[2], six[4], num_splits)
+            if workspace is None or workspace.numel() < need:
+                workspace = _scratch(need, q.device)
+            check(lib().paged_attention_v3_scaled(*six, scale, k_scale, v_scale, num_splits, workspace.data_ptr(),
+                                                  workspace.numel(), _stream(q.device)))
+
+    @staticmethod
+    def prefill_out(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, max_q_len, scale, k_scale, v_scale,
+                    fp32, out):
+        cu = cu_seqlens_q
+        args = _prep(q, k_cache, v_cache, block_tables, context_lens, *((4, "[B, S, H, D]") if cu is None
+                                                                        else (3, "[T, H, D]")))
+        q = args[0]
+        six = [C.byref(view(t)) for t in (out, *args)]
+        if cu is not None:
+            cu = cu.to(q.device, torch.int32).contiguous()
+        with torch.cuda.device(q.device):
+            ws = _scratch(lib().paged_attention_prefill_workspace_size(six[1], six[2], six[4], max_q_len), q.device)
+            check(lib().paged_attention_prefill_split(*six, None if cu is None else C.byref(view(cu)), max_q_len, scale,
+                                                      k_scale, v_scale, int(fp32), ws.data_ptr(), ws.numel(),
+                                                      _stream(q.device)))
+
+    @staticmethod
+    def write_kv_into(k_cache, v_cache, key, value, slot_mapping, k_scale, v_scale):
+        with torch.cuda.device(key.device):
+            check(lib().pa_write_kv_scaled(*(C.byref(view(t)) for t in (k_cache, v_cache, key, value, slot_mapping)),
+                                           k_scale, v_scale, _stream(key.device)))
+
+
+def _native():
+    if _ops is None and not _torch_path().exists():
+        lib()  # (its ImportError names the missing library)
+        return _CAbi
+    return torch_ops()
+
+
 def _decode(version, q, k_cache, v_cache, block_tables, context_lens, scale, num_splits, k_scale, v_scale, out_dtype,
             out, workspace):
     _on_gpu(q, k_cache, v_cache)
     o = _out(q, out_dtype, out)
-    torch_ops().decode_out(version, q, k_cache, v_cache, block_tables, context_lens, float(scale), int(num_splits),
-                           float(k_scale), float(v_scale), o, workspace)
+    _native().decode_out(version, q, k_cache, v_cache, block_tables, context_lens, float(scale), int(num_splits),
+                         float(k_scale), float(v_scale), o, workspace)
     return o
 
 
@@ -77,8 +148,8 @@ def _prefill(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, max_
              k_scale, v_scale, fp32):
     _on_gpu(q, k_cache, v_cache)
     o = _out(q, out_dtype, out)
-    torch_ops().prefill_out(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, int(max_q_len),
-                            float(scale), float(k_scale), float(v_scale), fp32, o)
+    _native().prefill_out(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, int(max_q_len),
+                          float(scale), float(k_scale), float(v_scale), fp32, o)
     return o
 
 
@@ -133,8 +204,10 @@ def paged_attention_v3(q, k_cache, v_cache, block_tables, context_lens, scale, n
                        out_dtype=torch.float32, out=None, workspace=None, k_scale=1.0, v_scale=1.0):
     """kernels/paged_attn_v3.h:13-16 -- context-split decode + separate LSE reduce.
 
-    num_splits > 0 cuts each sequence exactly as the reference does;
-    num_splits <= 0 lets the library plan the split from the CU count.
+    num_splits > 0 cuts each sequence as the reference does, except where the
+    library's own partitions, no more than those, were measured to be faster;
+    the merge makes either one softmax.  num_splits <= 0 lets the library plan
+    the split from the CU count.
     k_scale / v_scale dequantise a scaled cache (e.g. torch.float8_e4m3fn):
     attention runs on k_cache * k_scale and v_cache * v_scale."""
     return _decode(3, q, k_cache, v_cache, block_tables, context_lens, scale, num_splits, k_scale, v_scale, out_dtype,
@@ -183,7 +256,7 @@ def write_kv(k_cache, v_cache, key, value, slot_mapping, k_scale=1.0, v_scale=1.
     if slot_mapping.dtype not in (torch.int32, torch.int64):
         slot_mapping = slot_mapping.to(torch.int64)
     slot_mapping = slot_mapping.to(key.device).contiguous()
-    torch_ops().write_kv_into(k_cache, v_cache, key, value, slot_mapping, float(k_scale), float(v_scale))
+    _native().write_kv_into(k_cache, v_cache, key, value, slot_mapping, float(k_scale), float(v_scale))
 
 
 def write_kv_blocks(kv_pool, block_ids, start, k, v, k_scale=1.0, v_scale=1.0):
@@ -209,6 +282,10 @@ def write_kv_blocks(kv_pool, block_ids, start, k, v, k_scale=1.0, v_scale=1.0):
 _ops = None
 
 
+def _torch_path():
+    return LIB_PATH.with_name("libpagedattn_torch.so")
+
+
 def torch_ops():
     """The same launchers as PyTorch operators, torch.ops.gb10_attn.* (built from
     csrc/torch_ext.cpp into libpagedattn_torch.so): the reference's exact
@@ -217,7 +294,7 @@ def torch_ops():
     global _ops
     if _ops is None:
         lib()  # (its ImportError names the missing library)
-        path = LIB_PATH.with_name("libpagedattn_torch.so")
+        path = _torch_path()
         if not path.exists():
             raise ImportError(f"{path} is missing: build it with __graft_entry__.build()")
         if not hasattr(torch.ops.gb10_attn, "paged_attention_v3"):

@@ -59,3 +59,34 @@ def test_python_calls_inside_compile(pa, dev):
     want = layer(q)
     assert torch.equal(torch.compile(layer, backend="eager")(q), want)
     assert torch.equal(layer(q.clone().requires_grad_()).detach(), want)
+
+
+def test_python_calls_without_operator_library(pa, dev, monkeypatch, tmp_path):
+    """With libpagedattn.so alone the functions give the same results."""
+    import sys
+    ops = sys.modules[pa.paged_attention.__module__]
+    q, k, v, bt, c = dev_inputs(decode_case(3, 8, 2, 64, 16, [2000, 1, 700], seed=2, kv="bf16", q="bf16"), dev)
+    a = dev_args(prefill_case(2, 70, 4, 2, 64, 16, [70, 1100], seed=1, kv="f16", qt="f16"), dev)
+    cu = torch.tensor([0, 70, 140], device=dev)
+    k8 = torch.randn((5, 16, 2, 64), device=dev).to(torch.float8_e4m3fn)
+    key = torch.randn((7, 2, 64), device=dev)
+
+    def calls():
+        kc, vc = torch.zeros_like(k8), torch.zeros_like(k8)
+        pa.write_kv(kc, vc, key, key.flip(0), torch.arange(7, device=dev) * 3, 0.5, 0.25)
+        return [pa.paged_attention(q, k, v, bt, c, 0.1), pa.paged_attention_v2(q, k, v, bt, c, 0.1),
+                pa.paged_attention_v3(q, k, v, bt.long(), c.long(), 0.1, 0, out_dtype=torch.bfloat16),
+                pa.paged_attention_v3(q, k, v, bt, c, 0.1, 5, k_scale=0.5, v_scale=2.0),
+                pa.paged_attention_prefill_wmma(*a, 0.2), pa.paged_attention_prefill(*a, 0.2),
+                pa.paged_attention_prefill_varlen(a[0].reshape(140, 4, 64), *a[1:], cu, 70, 0.2),
+                kc.view(torch.uint8), vc.view(torch.uint8)]
+
+    print("without the operator library", flush=True)
+    want = calls()
+    monkeypatch.setattr(ops, "_ops", None)
+    monkeypatch.setattr(ops, "_torch_path", lambda: tmp_path / "none.so")
+    assert ops._native() is ops._CAbi
+    for x, y in zip(calls(), want):
+        assert x.dtype == y.dtype and torch.equal(x, y)
+    with pytest.raises(RuntimeError, match=r"q must be \[B, H, D\]"):
+        pa.paged_attention_v2(q[0], k, v, bt, c, 0.1)
