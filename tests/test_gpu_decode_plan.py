@@ -1,6 +1,6 @@
 """The library's own decode plan where it replaces or refines a call's split,
-against the CPU oracle: explicit counts from 16 partitions on (fewer planned,
-as many, and more than asked for), packed splits, and batches of nearly equal
+against the CPU oracle: explicit counts it may replace (fewer planned, as many,
+and more than asked for) where it is the faster, packed splits, and batches of nearly equal
 contexts on the matrix-core kernel, which are not cut."""
 import ctypes as C
 
