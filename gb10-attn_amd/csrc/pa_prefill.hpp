@@ -222,6 +222,17 @@ __device__ __forceinline__ int pf_turn(const PrefillParams& p, int b, int i) {
   return i >= p.HG ? i - p.HG : i;
 }
 
+// Sum over the wave, in scalar registers: rotations within rows of 16 lanes, then one
+// lane of each row.
+__device__ __forceinline__ int pf_wave_sum(int s) {
+  s += __builtin_amdgcn_update_dpp(0, s, 0x128, 0xf, 0xf, false);  // row_ror:8
+  s += __builtin_amdgcn_update_dpp(0, s, 0x124, 0xf, 0xf, false);
+  s += __builtin_amdgcn_update_dpp(0, s, 0x122, 0xf, 0xf, false);
+  s += __builtin_amdgcn_update_dpp(0, s, 0x121, 0xf, 0xf, false);
+  return __builtin_amdgcn_readlane(s, 0) + __builtin_amdgcn_readlane(s, 16) + __builtin_amdgcn_readlane(s, 32) +
+         __builtin_amdgcn_readlane(s, 48);
+}
+
 // Work-group x -> partition (context split, the slow index) and unit (b, head
 // group, block of QB packed rows); false past the last unit of a compacted
 // grid (work-group uniform).
@@ -251,7 +262,7 @@ __device__ __forceinline__ bool pf_unit(const PrefillParams& p, int64_t x, int l
     // (decode rows of a mixed batch, blocks past a short sequence's rows)
     // exiting only after a memory round trip, and spread the working ones
     // across the launch.  Per-sequence block counts sit in the lanes
-    // (kVlMaxSeqs / 64 per lane); each level costs one ballot per chunk.
+    // (kVlMaxSeqs / 64 per lane).
     int nbk[kVlMaxSeqs / 64];
 #pragma unroll
     for (int c = 0; c < kVlMaxSeqs / 64; ++c) {
@@ -268,8 +279,7 @@ __device__ __forceinline__ bool pf_unit(const PrefillParams& p, int64_t x, int l
       int mine = 0;
 #pragma unroll
       for (int c = 0; c < kVlMaxSeqs / 64; ++c) mine += nbk[c];
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) mine += __shfl_xor(mine, o, 64);
+      mine = pf_wave_sum(mine);
       // No more than the grid and the workspace hold: a cu_q whose ranges overlap
       // ([0, 512, 0, 512] of 512 rows) has more rows than T.  The units past them
       // stay unserved, as past the end of the unsplit kernel's grid.
@@ -280,24 +290,40 @@ __device__ __forceinline__ bool pf_unit(const PrefillParams& p, int64_t x, int l
       x -= part * total;
     }
     unit = x;
-    int64_t rem = x;
-    int fb = -1, ft = 0, fh = 0;
-    for (int t = nq - 1; t >= 0 && fb < 0; --t) {  // wave-uniform
+    // The largest block t with more units from it on than x, by bisection (a walk
+    // down from the last block costs up to 0.6 us a step, and packed heads have many:
+    // fp16, 8/1 heads of 128, one prompt of 512 rows at 1024, split, 60.3 -> 22.3 us;
+    // of 1024 at 2048 121.9 -> 35.0; of 2048, unsplit, 68.5 -> 44.6).
+    int ft = 0, hi = nq;
+    int64_t past = 0;  // units of the blocks past it
+    while (hi - ft > 1) {  // wave-uniform
+      const int mid = (ft + hi) >> 1;
+      int s = 0;
 #pragma unroll
-      for (int c = 0; c < kVlMaxSeqs / 64; ++c) {
-        const uint64_t m = __builtin_amdgcn_ballot_w64(nbk[c] > t);
-        const int64_t cnt = (int64_t)__builtin_popcountll(m) * p.HG;
-        if (fb < 0) {
-          if (rem < cnt) {
-            const int k = (int)(rem / p.HG);
-            const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-            const uint64_t sel = __builtin_amdgcn_ballot_w64(((m >> lane) & 1u) != 0 && rank == k);
-            fb = c * 64 + __builtin_ctzll(sel);
-            ft = t;
-            fh = (int)(rem - (int64_t)k * p.HG);
-          } else {
-            rem -= cnt;
-          }
+      for (int c = 0; c < kVlMaxSeqs / 64; ++c) s += max(nbk[c] - mid, 0);
+      const int64_t from = (int64_t)pf_wave_sum(s) * p.HG;
+      if (x < from) {
+        ft = mid;
+      } else {
+        hi = mid;
+        past = from;
+      }
+    }
+    int64_t rem = x - past;
+    int fb = -1, fh = 0;
+#pragma unroll
+    for (int c = 0; c < kVlMaxSeqs / 64; ++c) {
+      const uint64_t m = __builtin_amdgcn_ballot_w64(nbk[c] > ft);
+      const int64_t cnt = (int64_t)__builtin_popcountll(m) * p.HG;
+      if (fb < 0) {
+        if (rem < cnt) {
+          const int k = (int)(rem / p.HG);
+          const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+          const uint64_t sel = __builtin_amdgcn_ballot_w64(((m >> lane) & 1u) != 0 && rank == k);
+          fb = c * 64 + __builtin_ctzll(sel);
+          fh = (int)(rem - (int64_t)k * p.HG);
+        } else {
+          rem -= cnt;
         }
       }
     }

@@ -74,3 +74,26 @@ def test_packed_heads_turn(pa, dev, HKV, rows, ctx):
     q, *rest = args
     got = pa.paged_attention_prefill_varlen(q.reshape(B * rows, HKV * G, D), *rest, cu, rows, 0.2)
     close(to_host(got).reshape(want.shape), want)
+
+
+@pytest.mark.parametrize("B,rows", [(1, 700), (3, 260), (66, 40), (130, 17)])
+def test_packed_varlen_many_blocks(pa, dev, B, rows):
+    """A variable-length batch of many packed blocks (up to 175 to a sequence) over
+    one to three chunks of 64 sequences, empty and one-row ones between: every
+    row once, as the prefill of its sequence alone."""
+    HKV, G, D = 1, 16, 32
+    lens = [[rows, rows - 1 - i % 7, 0, 1, 5][0 if i in (0, B - 1) else i % 5] for i in range(B)]
+    ctx = [n + 3 * (i % 9) for i, n in enumerate(lens)]
+    inp = oracle.paged_inputs(B, 1, HKV, D, 16, ctx, seed=B, kv_dtype="f16")
+    q = oracle.quantize(np.random.default_rng(B).standard_normal((sum(lens), G * HKV, D), dtype=np.float32), "f16")
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    print("packed varlen blocks", B, rows, flush=True)
+    got = to_host(pa.paged_attention_prefill_varlen(
+        to_dev(q, "f16", dev), to_dev(inp["k"], "f16", dev), to_dev(inp["v"], "f16", dev),
+        torch.from_numpy(inp["bt"]).to(dev), torch.from_numpy(inp["ctx"]).to(dev), torch.from_numpy(cu).to(dev),
+        rows, 0.2))
+    for b, n in enumerate(lens):
+        if n:
+            want = oracle.prefill(q[None, cu[b]:cu[b + 1]], inp["k"], inp["v"], inp["bt"][b:b + 1], inp["ctx"][b:b + 1],
+                                  0.2, "f16")[0]
+            close(got[cu[b]:cu[b + 1]], want)
