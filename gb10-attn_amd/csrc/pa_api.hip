@@ -422,8 +422,16 @@ int make_plan(const DecodeParams& p, int gc, int kv_bytes, int64_t num_splits, P
 // ALU, and cut contexts took 0.72 to 0.96 of the speed of whole ones over ragged
 // contexts to 8192 (64/8 heads of 128, FP8, 78 rows and two chunks of 512: 584 and
 // 811 us; fp16, 59 rows: 649 and 727), 0.88 to 1.24 over equal ones.
-int plan_varlen_decode(const DecodeParams& p, int gc, int kv_bytes, Plan* plan) {
+// Nor in a batch of T rows that leaves no sequence a single one (B of up to max_q
+// rows each; more rows than that are padding, and tell nothing): the merge alone
+// cost 2 to 3 us (12 heads of 64, one prompt of 2048 rows 33 -> 35).
+int plan_varlen_decode(const DecodeParams& p, int gc, int kv_bytes, int64_t T, int64_t max_q, Plan* plan) {
   int cus = 0, rc;
+  const int64_t B = p.B;
+  if (max_q > 1 && T <= B * max_q && T - B > (B - 1) * (max_q - 1)) {
+    *plan = {false, 1, 0, true, 0};
+    return PA_OK;
+  }
   if ((rc = make_plan(p, gc, kv_bytes, 0, plan)) || plan->direct) return rc;
   if ((rc = device_cu_count(&cus))) return rc;
   const double rows = (double)p.MB * p.BS * p.D / 64.0, units = (double)p.B * p.HKV * ((p.G + gc - 1) / gc);
@@ -870,7 +878,7 @@ int run_varlen(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k_cach
     Plan plan;
     plan.direct = true;
     if (ws.given) {
-      if ((rc = plan_varlen_decode(d.p, d.gc, dtype_bytes(d.kv_dtype), &plan))) return rc;
+      if ((rc = plan_varlen_decode(d.p, d.gc, dtype_bytes(d.kv_dtype), T, a.p.Sq, &plan))) return rc;
       decode_bytes = workspace_bytes_for(d.p.B, d.p.H, d.p.D, plan);
       PrefillParams pp = prefill_params(a, cu, T, scale * k_scale);  // every check before the first launch
       if ((rc = bind_split(pp, true, ws, decode_bytes))) return rc;
@@ -1111,7 +1119,7 @@ size_t paged_attention_prefill_workspace_size(const pa_tensor_t* q, const pa_ten
   d.B = pp.B; d.Sq = 1; d.H = pp.H; d.HKV = (int)HKV; d.G = pp.G; d.D = pp.D; d.BS = pp.BS; d.MB = pp.MB;
   d.k_sh = k_cache->stride[2];
   Plan plan;
-  if (plan_varlen_decode(d, decode_heads_per_wg(d.G), dtype_bytes(k_cache->dtype), &plan)) return (size_t)-1;
+  if (plan_varlen_decode(d, decode_heads_per_wg(d.G), dtype_bytes(k_cache->dtype), pp.q_total, pp.S, &plan)) return (size_t)-1;
   return bytes + workspace_bytes_for(d.B, d.H, d.D, plan);
 }
 

@@ -140,3 +140,23 @@ def test_varlen_split_rule(pa, dev, npf, mb, split):
     for b in range(len(lens)):
         close(got[cu[b]:cu[b + 1]], oracle.prefill(q[None, cu[b]:cu[b + 1]], inp["k"], inp["v"], inp["bt"][b:b + 1],
                                                    inp["ctx"][b:b + 1], 0.1, "f16")[0])
+
+
+@pytest.mark.parametrize("lens,cut", [([70], False), ([70, 69], False), ([70, 1], True), ([70, 1, 0], True)])
+def test_varlen_decode_rows_possible(pa, dev, lens, cut):
+    """The decode rows' split is planned only where the batch's row count leaves a
+    sequence with one row; every sequence against the oracle."""
+    HKV, G, D = 2, 2, 64
+    ctx = [3000 - 7 * i if n else 5 for i, n in enumerate(lens)]
+    inp = oracle.paged_inputs(len(lens), 1, HKV, D, 16, ctx, seed=4, kv_dtype="f16")
+    q = oracle.quantize(np.random.default_rng(4).standard_normal((sum(lens), G * HKV, D), dtype=np.float32), "f16")
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    print("decode rows possible", lens, flush=True)
+    got = to_host(pa.paged_attention_prefill_varlen(
+        to_dev(q, "f16", dev), to_dev(inp["k"], "f16", dev), to_dev(inp["v"], "f16", dev),
+        torch.from_numpy(inp["bt"]).to(dev), torch.from_numpy(inp["ctx"]).to(dev), torch.from_numpy(cu).to(dev), 70, 0.1))
+    assert ("pa::reduce_kernel" in pa.last_launch()) == cut, pa.last_launch()
+    for b, n in enumerate(lens):
+        if n:
+            close(got[cu[b]:cu[b + 1]], oracle.prefill(q[None, cu[b]:cu[b + 1]], inp["k"], inp["v"], inp["bt"][b:b + 1],
+                                                       inp["ctx"][b:b + 1], 0.1, "f16")[0])
