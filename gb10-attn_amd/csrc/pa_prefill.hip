@@ -21,11 +21,7 @@ static hipError_t launch_pp(const PrefillParams& p, hipStream_t stream) {
   static std::atomic<int64_t> cache[64];
   const auto kernel = prefill_pp_kernel<KV, D>;
   PrefillParams q = p;
-  q.q_tiles = (int32_t)(((int64_t)p.S * p.gp + kPpRows - 1) / kPpRows);
-  const int64_t units = (int64_t)q.B * q.HG * q.q_tiles;
-  int64_t cus = 0, per_cu = 0;
-  residency(kernel, cache, &cus, &per_cu, kPpThreads);
-  q.wg_cus = units > cus && units <= cus * per_cu ? (int32_t)cus : 0;  // one resident wave
+  const int64_t units = pf_grid(kernel, cache, kPpRows, q, kPpThreads);
   note_launch("pa::prefill_pp_kernel<%s, %d>", KV::kName, D);
   hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(kPpThreads), 0, stream, q);
   return hipGetLastError();

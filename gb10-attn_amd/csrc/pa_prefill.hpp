@@ -1263,31 +1263,20 @@ void prefill_pp_kernel(const PrefillParams p) {
   const int n = lane & 31;
   const int hh = lane >> 5;
 
-  // Work-group -> unit (b, h, query block), as the four-wave kernel.
-  const int nq = p.q_tiles;
-  const int64_t nbh = (int64_t)p.B * p.HG;
-  int64_t x = blockIdx.x;
-  if (p.wg_cus > 0) {
-    const int64_t C = p.wg_cus, g = x / C, jj = x - g * C;
-    if ((g & 1) && (g + 1) * C <= nbh * nq) x = g * C + (C % 8 == 0 ? C - 8 - (jj & ~(int64_t)7) + (jj & 7) : C - 1 - jj);
-  }
-  const int qt = nq - 1 - (int)(x / nbh);
-  const int64_t bh = x % nbh;
-  const int b = (int)(bh / p.HG);
-  const int hg = pf_turn(p, b, (int)(bh % p.HG));
+  // Work-group -> unit (b, h, query block), as the four-wave kernel; also compacted:
+  // a work-group without rows held a CU to exit, and with packed heads the few with
+  // rows came singly between them (fp16, 64/8 heads of 128, 16 decode rows and one
+  // prompt of 2048 at 4096: unpacked 248 us, packed 297, compacted 235).
+  int part, qt, hg, b;
+  int64_t unit;
+  if (!pf_unit<QB, false>(p, blockIdx.x, lane, part, unit, qt, hg, b)) return;
   const int h0 = hg * p.gp;  // first query head of the unit
   const int kvh = h0 / p.G;
 
-  int S = p.S;
-  int64_t tok0 = (int64_t)b * p.S;
-  if (p.cu_q) {
-    const int qa = p.cu_q[b], qb = p.cu_q[b + 1];
-    const bool ok = qa >= 0 && qb >= qa && (int64_t)qb <= p.q_total;
-    S = ok ? qb - qa : 0;
-    tok0 = ok ? qa : 0;
-    if (p.skip_single && S == 1) return;
-  }
-  const int Sr = min(S, p.S) * p.gp;  // packed rows served
+  int S, served;
+  int64_t tok0;
+  if (!pf_rows(p, b, S, tok0, served)) return;
+  const int Sr = served * p.gp;  // packed rows served
   const int qs0 = qt * QB;
   if (qs0 >= Sr) return;
   const int qw0 = qs0 + wave * QW;
@@ -1826,14 +1815,14 @@ static void residency(F kernel, std::atomic<int64_t> (&cache)[64], int64_t* cus,
   *per_cu = k;
 }
 
-// Grid of a 4-wave kernel of QB-row blocks: its work-groups, and the fields of
+// Grid of a prefill kernel of QB-row blocks: its work-groups, and the fields of
 // q that number them.
 template <typename F>
-static int64_t pf_grid(F kernel, std::atomic<int64_t> (&cache)[64], int QB, PrefillParams& q) {
+static int64_t pf_grid(F kernel, std::atomic<int64_t> (&cache)[64], int QB, PrefillParams& q, int threads = kPfThreads) {
   q.q_tiles = (int32_t)(((int64_t)q.S * q.gp + QB - 1) / QB);
   int64_t units = (int64_t)q.B * q.HG * q.q_tiles;
   int64_t cus = 0, per_cu = 0;
-  residency(kernel, cache, &cus, &per_cu);
+  residency(kernel, cache, &cus, &per_cu, threads);
   q.wg_cus = units > cus && units <= cus * per_cu ? (int32_t)cus : 0;  // one resident wave
   // Variable-length batches of up to kVlMaxSeqs sequences: a compacted grid
   // of at most the units with rows (sum over sequences of ceil(rows / QB) <
