@@ -1104,10 +1104,10 @@ def c2_split_records(pa, pools, steps):
     """Config 2 through an explicit split: the reference's own count
     (choose_num_splits on its 48-SM GB10: 64) and the fastest of a few
     explicit counts, each timed as the API call the reference makes
-    (paged_attention_v3 with num_splits: partition + reduce, or from 8
-    partitions on the library's own plan, one launch here).  The reference's count is
-    also timed as two launches (pa_v3_partition, then pa_v3_reduce) with the
-    partition kernel and the reduce timed apart."""
+    (paged_attention_v3 with num_splits: partition + reduce, or the library's
+    own plan, one launch here, from the count on where that is faster).  The
+    reference's count is also timed as two launches (pa_v3_partition, then
+    pa_v3_reduce) with the partition kernel and the reduce timed apart."""
     recs = []
     for ns in (64, 2, 4, 8, 16):
         w = DecodeWorkload(pa, B=64, H=12, HKV=12, D=64, BS=16, ctx=[2048] * 64, dtype=torch.float16,

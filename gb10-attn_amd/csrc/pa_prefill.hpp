@@ -384,12 +384,15 @@ __device__ __forceinline__ bool pf_rows(const PrefillParams& p, int b, int& S, i
 //
 // kX (fp32-precision mode, prefill32_kernel): q and the weights are carried as
 // two fp16 pieces (three bf16 pieces over a bf16 cache) whose sum is the fp32
-// value to 2^-24 (bf16: exactly), and every product of a piece with a K or V
-// element is exact in the matrix cores' fp32 accumulation, so both products
-// keep fp32 precision at two (three) 16-bit products each.  fp16 pieces need
-// the range: each q row is scaled by a power of two that puts its largest
-// element in [2^14, 2^15), and the weights by 2^7 (they are at most 2^8 by
-// the lazy maximum, which is kept an integer so that these shifts are exact).
+// value to 2^-24 of it or the pieces' smallest step (bf16: exactly), and every
+// product of a piece with a K or V element is exact in the matrix cores' fp32
+// accumulation, so both products keep fp32 precision at two (three) 16-bit
+// products each.  fp16 pieces need the range: each q row is scaled by a power of
+// two that puts its largest element in [2^14, 2^15), and the weights by 2^7 (they
+// are at most 2^8 by the lazy maximum, which is kept an integer so that these
+// shifts are exact).  The smallest step, half of fp16's 2^-24, is then 2^-32 of a
+// weight of 1 and 2^-39 of a row's largest q: below those the rounding is
+// absolute, under the 2^-24 that fp32 sums of the largest terms carry.
 // Bound by the matrix and vector work of the pieces (the 16-bit-weight kernel's
 // chain of tiles with four products for its three and ~180 more vector
 // instructions per 64 keys).  B = 4, S = 512, context 2048, 12 heads of 64,

@@ -111,14 +111,21 @@ int paged_attention_v2(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t
  * kernels/paged_attn_v3.h:13-16 (kernels/paged_attn_v3.cu:192-261).
  * num_splits > 0: sequence b is cut into num_splits partitions
  *   [s*chunk, min((s+1)*chunk, ctx_b)), chunk = ceil(ctx_b / num_splits),
- *   exactly as kernels/paged_attn_v3.cu:65-68.
+ *   as kernels/paged_attn_v3.cu:65-68, except as below.
  * num_splits <= 0: the library plans fixed-size partitions from MB*BS, the
  *   batch size and the device's CU count (see pa_plan_partitions); when the
  *   batch alone fills the GPU no split and no reduce launch happen.
- * A call with 16 or more explicit partitions (MHA: 8, at rows of 1 KB 4) computes the same merged result
- * over the partitions the library plans (no more than num_splits): the
- * partials are not part of its result, and pa_v3_partition / pa_v3_reduce run
- * the explicit ones.
+ * The partials are not part of the result, so a call with 16 or more explicit
+ * partitions (one query head per KV head: 8, at rows of 1 KB 4) may compute it
+ * over the partitions the library plans, no more than num_splits: it does where
+ * those were measured to be faster (short partitions that fill the GPU, groups
+ * of eight over 16-bit caches, few partitions for the GPU).  The weights keep
+ * the precision of the explicit partitions.  pa_v3_partition / pa_v3_reduce
+ * always run the explicit ones.
+ * Groups of eight query heads and more over 16-bit caches run on the matrix
+ * cores (every decode entry point) with the weights as two 16-bit pieces: an
+ * infinite V element may give NaN in place of an infinity in the rows that
+ * attend it, except where bf16 weights keep three pieces as above.
  * workspace must be device memory of at least
  *   paged_attention_v3_workspace_size(...) bytes (NULL allowed when that is 0). */
 int paged_attention_v3(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k_cache,
@@ -165,16 +172,21 @@ int64_t choose_num_splits_for(int64_t num_seqs, int64_t num_heads, int64_t max_c
  * tokens and the number of partitions per sequence (1 = no split).  It
  * sees no cache layout: for MHA caches whose head rows are shorter than 128
  * bytes (served two heads per work-group) paged_attention_v3 plans with
- * num_kv_heads / 2 units, and a split whose heads can share a work-group may
- * take more, shorter partitions; paged_attention_v3_workspace_size always
- * matches the call. */
+ * num_kv_heads / 2 units, and a split of MHA heads of 128 elements and more
+ * that can share a work-group may take more, shorter partitions;
+ * paged_attention_v3_workspace_size always matches the call. */
 int pa_plan_partitions(int64_t num_seqs, int64_t num_heads, int64_t num_kv_heads,
                        int64_t head_dim, int64_t max_context, int64_t num_compute_units,
                        int64_t* partition_tokens, int64_t* num_partitions);
 
-/* Causal (chunked) prefill at fp32 precision (over 16-bit and FP8 caches on
- * the matrix cores, fp32 operands carried as sums of 16-bit pieces).  Replaces paged_attention_prefill(),
- * kernels/paged_attn_prefill.h:13-15 (kernels/paged_attn_prefill.cu:122-175).
+/* Causal (chunked) prefill at fp32 precision.  Replaces
+ * paged_attention_prefill(), kernels/paged_attn_prefill.h:13-15
+ * (kernels/paged_attn_prefill.cu:122-175).  Larger calls over 16-bit and FP8
+ * caches run on the matrix cores, fp32 operands carried as sums of 16-bit
+ * pieces (over fp16 and FP8 caches held no finer than 2^-32 of the weight at
+ * the row's reference maximum, q than 2^-39 of its row's largest element: both
+ * under the rounding of the fp32 sums).  GQA groups over fp16 caches are the exception: their weights
+ * stay fp16 pairs of keys in P V (1.3e-4 from 64 bits).
  * Query s of sequence b sits at q_pos = ctx_b - S + s and attends keys
  * [0, q_pos]; q_pos < 0 gives a zero row (kernels/paged_attn_prefill.cu:62-74). */
 int paged_attention_prefill(pa_tensor_t* out, const pa_tensor_t* q, const pa_tensor_t* k_cache,
