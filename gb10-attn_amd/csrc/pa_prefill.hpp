@@ -218,7 +218,7 @@ __device__ inline int swv(int row, int cc) {
 // 16 prompts of 512 rows 94 -> 96 -> 83 us.
 __device__ __forceinline__ int pf_turn(const PrefillParams& p, int b, int i) {
   if (p.gp == 1) return i;
-  i += (int)(((uint32_t)b * (uint32_t)p.HG >> 3) % (uint32_t)p.HG);
+  i += (b & 7) * p.HG >> 3;
   return i >= p.HG ? i - p.HG : i;
 }
 
