@@ -640,8 +640,10 @@ constexpr int64_t kPrefill32Units = 768;
 // weights as fp16 pairs (1.3e-4 from 64 bits; the matrix kernel 1.7e-7), and the
 // calls' results stay what they were to the fp32 tolerance.  (8/2 heads of 128,
 // 75 us against 19 there.)
+// D = 256 is off: 18 sequences of 64 rows, fp16 q and cache, gave wrong rows once
+// and a memory fault in a repetition, and the cause is not found.
 bool prefill32_eligible(const DecodeArgs& a, const pa_tensor_t* q) {
-  return prefill_kv(a.kv_dtype) && !(a.kv_dtype == kF16 && a.gc > 1) && aligned16(q->data);
+  return a.p.D < 256 && prefill_kv(a.kv_dtype) && !(a.kv_dtype == kF16 && a.gc > 1) && aligned16(q->data);
 }
 bool prefill32_pays(const DecodeArgs& a, const PrefillParams& pp) {
   const int64_t units = (int64_t)a.p.B * a.p.Sq * a.p.HKV * a.p.head_chunks;
